@@ -770,14 +770,15 @@ static int create_buffers(sphk_engine* e, size_t capacity) {
     }
     HIP_TRY(dalloc(&e->fscal, 4));
     HIP_TRY(dalloc(&e->uscal, 4));
-    HIP_TRY(dalloc(&e->nstats, 2));
+    HIP_TRY(dalloc(&e->nstats, kStatSlots * kStatStride));
     HIP_TRY(hipMemsetAsync(e->acc, 0, C * sizeof(float4), e->stream));
     HIP_TRY(hipMemsetAsync(e->vel, 0, C * sizeof(float4), e->stream));
     HIP_TRY(hipMemsetAsync(e->rho, 0, C * sizeof(float), e->stream));
     HIP_TRY(hipMemsetAsync(e->prs, 0, C * sizeof(float), e->stream));
     HIP_TRY(hipMemsetAsync(e->fscal, 0, 4 * sizeof(float), e->stream));
     HIP_TRY(hipMemsetAsync(e->uscal, 0, 4 * sizeof(uint32_t), e->stream));
-    HIP_TRY(hipMemsetAsync(e->nstats, 0, 2 * sizeof(unsigned long long), e->stream));
+    HIP_TRY(hipMemsetAsync(e->nstats, 0, kStatSlots * kStatStride * sizeof(unsigned long long),
+                           e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     return SPHK_OK;
 }
@@ -1182,13 +1183,15 @@ int sphk_get_stats(sphk_engine* e, sphk_stats* out) {
     if (int rc = check_engine(e)) return rc;
     if (!out) return set_error(SPHK_E_INVALID, "null output");
     if (int rc = set_device(e)) return rc;
-    unsigned long long ns[2];
+    unsigned long long ns[kStatSlots * kStatStride];
     HIP_TRY(hipMemcpyAsync(ns, e->nstats, sizeof(ns), hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     if (int rc = drain_timing(e)) return rc;
     *out = e->stats;
-    out->max_neighbors = ns[0];
-    out->total_neighbors = ns[1];
+    for (uint32_t k = 0; k < kStatSlots; ++k) {
+        out->max_neighbors = std::max<uint64_t>(out->max_neighbors, ns[k * kStatStride]);
+        out->total_neighbors += ns[k * kStatStride + 1];
+    }
     return SPHK_OK;
 }
 
@@ -1197,7 +1200,8 @@ int sphk_reset_stats(sphk_engine* e) {
     if (int rc = set_device(e)) return rc;
     if (int rc = drain_timing(e)) return rc;
     e->stats = sphk_stats{};
-    HIP_TRY(launch_fill_u32(reinterpret_cast<uint32_t*>(e->nstats), 0u, 4, e->stream));
+    HIP_TRY(launch_fill_u32(reinterpret_cast<uint32_t*>(e->nstats), 0u,
+                            2 * kStatSlots * kStatStride, e->stream));
     return SPHK_OK;
 }
 

@@ -112,7 +112,7 @@ struct sphk_engine {
     float* fscal = nullptr;
     // [0] out-of-grid flag, [1] cfl scratch
     uint32_t* uscal = nullptr;
-    // [0] max neighbours, [1] total neighbours
+    // kStatSlots pairs: [0] max neighbours, [1] total neighbours
     unsigned long long* nstats = nullptr;
 
     // scenes and their grids

@@ -761,8 +761,10 @@ __device__ __forceinline__ void init_sentinel(uint32_t* __restrict__ lmask,
     if (lane == 0) lwj0[kSeg - 1] = c.pad_slot;
 }
 
+// Adds a wavefront's neighbour counts to the statistics slot of its workgroup.
 __device__ __forceinline__ void add_nbr_stats(uint32_t cnt, unsigned long long* stats,
                                               uint32_t lane) {
+    stats += (blockIdx.x % kStatSlots) * kStatStride;
     uint32_t mx = cnt;
     unsigned long long sm = cnt;
     for (int off = 32; off > 0; off >>= 1) {
