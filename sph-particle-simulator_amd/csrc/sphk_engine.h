@@ -127,6 +127,12 @@ struct sphk_engine {
     // restore that leaves the grids as they were re-uploads nothing)
     std::vector<SceneGrid> table_uploaded;
     uint64_t table_uploaded_gen = ~0ull;
+    // bounding-box reduction: scene ranges (and what the device holds of them), part boxes
+    uint32_t* bbox_ranges = nullptr;
+    uint64_t bbox_ranges_cap = 0;
+    std::vector<uint32_t> bbox_uploaded;
+    uint32_t* bbox_out = nullptr;
+    uint64_t bbox_out_cap = 0;
     StepConsts consts{};
     bool sorted_valid = false;  // work arrays hold the cell-sorted image of the current state
     uint64_t buffer_gen = 0;    // bumped when a buffer used by the step is reallocated

@@ -1,0 +1,39 @@
+"""Edges of the launch rules: scene extents, lane-team walks, sort routes, read-backs."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sizes", [[1, 0, 257, 5000, 3], [3] * 1100, [70001]])
+def test_scene_extents_measured_on_the_device(sphk, sizes):
+    # The extents of scenes whose state was replaced are measured on the device in one launch
+    # (parts of a scene folded on the host): scenes of one particle, none, only non-finite
+    # ones, more scenes than workgroups, one scene over many parts.  A particle outside its
+    # measured grid would be reported by the read-back; the step equals the scene alone.
+    rng = np.random.default_rng(7)
+    offs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
+    n = int(offs[-1])
+    centre = np.repeat(rng.uniform(-3, 3, (len(sizes), 3)), sizes, axis=0)
+    pos = (centre + rng.uniform(-0.2, 0.2, (n, 3))).astype(np.float32)
+    if len(sizes) > 4:
+        a, b = int(offs[4]), int(offs[5])
+        pos[a:b] = np.nan
+        pos[int(offs[2])] = np.inf
+    p = sphk.default_params(xmin=-4, xmax=4, ymin=-4, ymax=4, zmin=-4, zmax=4, formulation=1)
+    e = sphk.Engine(n, p)
+    e.upload(pos)
+    e.set_scenes(offs)
+    e.snapshot_save()
+    for _ in range(2):
+        e.snapshot_restore()
+        e.step(1e-4)
+    got = e.positions()
+    for k in [0, 2, 3, 4, len(sizes) - 1]:
+        if k >= len(sizes) or sizes[k] == 0:
+            continue
+        a, b = int(offs[k]), int(offs[k + 1])
+        one = sphk.Engine(b - a, p)
+        one.upload(pos[a:b])
+        one.step(1e-4)
+        np.testing.assert_array_equal(got[a:b], one.positions())
