@@ -121,6 +121,22 @@ __device__ __forceinline__ int axis_edge_flags(float x, float inv, float r2) {
     return flags;
 }
 
+// Whether axis_edge_flags(x, inv, r2) can set a flag at all (r2 = fl(R^2), inv = fl(1 / R)).
+// With u = 2^-24 and t = fl(x inv), c = floor(t): a neighbour b in cell c + 2 has
+// b / R >= c + 2 - 2.1 u |c + 2| and b - x <= R (1 + 3 u), so t >= c + 1 - 5 u (|c| + 3); in
+// cell c - 2, by the same bounds, t <= c + 5 u (|c| + 3).  Tested with 32 u for 5 u.  The
+// bracket searches of the exact flags (six divisions a lane) are then skipped by every chunk
+// without such a lane: 1M step 1.086 -> 1.081 ms, 9.6M 0.8 % faster, and every wavefront of a
+// walk pays them.
+__device__ __forceinline__ bool axis_edge_near(float x, float inv) {
+    const float t = x * inv;
+    const float c = floorf(t);
+    const float margin = (fabsf(c) + 3.0f) * 0x1p-19f;
+    const float f = t - c;
+    // (written so that a NaN counts as near)
+    return !(f > margin && f < 1.0f - margin);
+}
+
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
 constexpr uint32_t kXcds = 8;
@@ -686,7 +702,10 @@ __device__ __forceinline__ bool load_chunk(uint32_t item, const uint32_t* __rest
     const float qnan = __int_as_float(0x7fc00000);
     pi = active ? spm[s] : make_float4(qnan, qnan, qnan, 0.0f);
     int fx = 0, fy = 0, fz = 0;
-    if (active) {
+    const bool near = active && (axis_edge_near(pi.x, c.inv_cell) ||
+                                 axis_edge_near(pi.y, c.inv_cell) ||
+                                 axis_edge_near(pi.z, c.inv_cell));
+    if (near) {
         fx = axis_edge_flags(pi.x, c.inv_cell, c.r2);
         fy = axis_edge_flags(pi.y, c.inv_cell, c.r2);
         fz = axis_edge_flags(pi.z, c.inv_cell, c.r2);
