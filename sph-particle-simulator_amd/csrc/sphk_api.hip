@@ -408,6 +408,8 @@ int ensure_grid(sphk_engine* e) {
             if (*p) HIP_TRY(hipFree(*p));
             *p = nullptr;
         }
+        if (wb.desc) HIP_TRY(hipFree(wb.desc));
+        wb.desc = nullptr;
         const size_t want = std::max<size_t>(chunks, wb.chunk_cap * 5 / 4);
         // kMaxWords words (64 KiB of bits) per chunk while the buffers stay within the budget
         const uint32_t mw =
@@ -415,6 +417,7 @@ int ensure_grid(sphk_engine* e) {
         wb.chunk_cap = 0;
         wb.max_words = 0;
         HIP_TRY(dalloc(&wb.items, want));
+        HIP_TRY(dalloc(&wb.desc, want));
         HIP_TRY(dalloc(&wb.mask, want * mw * 64));
         HIP_TRY(dalloc(&wb.wj0, want * mw));
         HIP_TRY(dalloc(&wb.nwords, want));
@@ -497,7 +500,7 @@ int build_sorted(sphk_engine* e, const StepTail* tail) {
         t.n = n;
     }
     HIP_TRY(launch_chunks(e->cell_start, e->consts, e->d_scenes, e->walk.colcnt, e->scan_scratch,
-                          e->walk.items, e->walk.nitems, tail ? &t : nullptr, st));
+                          e->walk.items, e->walk.desc, e->walk.nitems, tail ? &t : nullptr, st));
     e->sorted_valid = true;
     return SPHK_OK;
 }
@@ -824,7 +827,7 @@ int sphk_destroy(sphk_engine* e) {
                     e->nstats, e->frows, e->sq};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
-    for (void* p : {(void*)e->walk.items, (void*)e->walk.nitems, (void*)e->walk.colcnt,
+    for (void* p : {(void*)e->walk.items, (void*)e->walk.desc, (void*)e->walk.nitems, (void*)e->walk.colcnt,
                     (void*)e->walk.mask, (void*)e->walk.wj0, (void*)e->walk.nwords,
                     (void*)e->walk.pstarts, (void*)e->walk.part_acc, (void*)e->walk.part_cnt,
                     (void*)e->walk.part_force, (void*)e->scan_scratch, (void*)e->d_scenes,

@@ -115,6 +115,10 @@ constexpr uint32_t kStatStride = 16;  // unsigned long longs per slot
 // HBM buffers of the chunked walks (sized for max_chunks())
 struct WalkBuffers {
     uint32_t* items = nullptr;    // first sorted slot of each chunk
+    uint4* desc = nullptr;        // end slot, scene and column (x, y in its grid) of each chunk:
+                                  // the walks start from it instead of looking the scene and the
+                                  // column of the first particle up (a chain of dependent loads
+                                  // and four divisions per wavefront)
     uint32_t* nitems = nullptr;   // [1] number of chunks
     uint32_t* colcnt = nullptr;   // [ncols + 1] per-column chunk counts -> offsets
     uint32_t* mask = nullptr;     // [chunks][max_words][64] neighbour bits
@@ -235,7 +239,7 @@ uint32_t max_chunks(uint32_t n, const StepConsts& c);
 // chunk list of the sorted particles; with `tail`, also the non-finite particles' step
 hipError_t launch_chunks(const uint32_t* cell_start, const StepConsts& c, const SceneGrid* scenes,
                          uint32_t* cnt_scratch, uint32_t* scan_scratch, uint32_t* items,
-                         uint32_t* nitems, const StepTail* tail, hipStream_t st);
+                         uint4* desc, uint32_t* nitems, const StepTail* tail, hipStream_t st);
 hipError_t launch_density_walk(const WalkBuffers& wb, const float4* spm, const uint2* sq,
                                float4* svr,
                                ForceRow* rows, const uint32_t* skey,

@@ -259,7 +259,7 @@ k_sur_forward(WalkBuffers wb, const uint32_t* __restrict__ batch, uint32_t nbatc
     uint32_t s;
     bool active;
     float4 pi;
-    if (!load_chunk(item, wb.items, wb.nitems, skey, cs, spm, c, scenes, clane, ch, s, active,
+    if (!load_chunk(item, wb.items, wb.desc, wb.nitems, skey, spm, c, scenes, clane, ch, s, active,
                     pi))
         return;
     const float4 vi = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(64 * kEdgeWaves) void k_sur_edges_bwd(
     uint32_t s;
     bool active;
     float4 pi;
-    if (!load_chunk(item, wb.items, wb.nitems, skey, cs, spm, c, scenes, clane, ch, s, active,
+    if (!load_chunk(item, wb.items, wb.desc, wb.nitems, skey, spm, c, scenes, clane, ch, s, active,
                     pi))
         return;
     const float4 vi = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 0.f);

@@ -27,7 +27,7 @@
 #include <algorithm>
 #include <climits>
 
-#include "sphk_walk_common.h"
+#include "sphk_walk_pairs.h"
 
 namespace sphk {
 
@@ -50,19 +50,32 @@ __global__ __launch_bounds__(256) void k_chunk_count(const uint32_t* __restrict_
     cnt[col] = (b - a + 63u) / 64u;
 }
 
+// Items and descriptions of one column's chunks, its slots [r.x, r.y), from item `o` on.
+__device__ __forceinline__ void column_items(uint2 r, uint32_t scene, const SceneGrid& g,
+                                             uint32_t col, uint32_t o,
+                                             uint32_t* __restrict__ items,
+                                             uint4* __restrict__ desc) {
+    const uint32_t rx = (col - g.col_base) / (uint32_t)g.ny, ry = (col - g.col_base) % (uint32_t)g.ny;
+    for (uint32_t s = r.x; s < r.y; s += 64u) {
+        items[o] = s;
+        desc[o++] = make_uint4(min(s + 64u, r.y), scene, rx, ry);
+    }
+}
+
 __global__ __launch_bounds__(256) void k_chunk_fill(const uint32_t* __restrict__ cs, StepConsts c,
                                                     const SceneGrid* __restrict__ scenes,
                                                     const uint32_t* __restrict__ offs,
                                                     uint32_t* __restrict__ items,
+                                                    uint4* __restrict__ desc,
                                                     uint32_t* __restrict__ nitems) {
     const uint32_t col = blockIdx.x * blockDim.x + threadIdx.x;
     if (col == 0) nitems[0] = offs[c.ncols];
     if (col >= c.ncols) return;
-    const SceneGrid g = scenes[scene_of_col(scenes, c.nscenes, col)];
+    const uint32_t scene = scene_of_col(scenes, c.nscenes, col);
+    const SceneGrid g = scenes[scene];
     const uint32_t first = g.cell_base + (col - g.col_base) * (uint32_t)g.nz;
-    const uint32_t a = cs[first], b = cs[first + (uint32_t)g.nz];
-    uint32_t o = offs[col];
-    for (uint32_t s = a; s < b; s += 64u) items[o++] = s;
+    column_items(make_uint2(cs[first], cs[first + (uint32_t)g.nz]), scene, g, col, offs[col],
+                 items, desc);
 }
 
 uint32_t max_chunks(uint32_t n, const StepConsts& c) { return (n + 63u) / 64u + c.ncols; }
@@ -78,40 +91,6 @@ uint32_t max_chunks(uint32_t n, const StepConsts& c) { return (n + 63u) / 64u + 
 // runs over the set bits, self included.  Stores the neighbour words of every chunk and the
 // force walk's neighbour rows of every particle.
 // ---------------------------------------------------------------------------
-// The cubic spline (CubicSplineKernel::W_3d, src/kernels.cpp:58-66) as one expression:
-// 6 W(q) / sigma = (2 - q)^3 - 4 (1 - q)^3 for q <= 1
-// and (2 - q)^3 for 1 < q <= 2, i.e. t^3 - 4 s^3 with t = max(2 - q, 0), s = max(1 - q, 0).
-// The walk sums an eighth of it, u^3 + s^2 (-s / 2) with u = t / 2 = max(1 - q / 2, 0): every
-// rounding is that of the t-form scaled by 2^-3 (terms below 2^-126 aside), so the sums are
-// the same bits / 8; u and s lie in [0, 1], where the max is the instructions' clamp bit
-// (seven operations, no select).  The sum is scaled by 8 sigma / 6 at the end.
-__device__ __forceinline__ float w6_shape8(float r, float half_inv_h, float inv_h) {
-    const float u = __builtin_amdgcn_fmed3f(__builtin_fmaf(-half_inv_h, r, 1.0f), 0.0f, 1.0f);
-    const float s = __builtin_amdgcn_fmed3f(__builtin_fmaf(-inv_h, r, 1.0f), 0.0f, 1.0f);
-    return __builtin_fmaf(s * s, -0.5f * s, u * u * u);
-}
-
-// One neighbour's m_j (6 W / 8 sigma).  Pairs the filter let through beyond the radius: with
-// a radius of at least 2h they have q >= 2 (up to the rounding of sqrt, which leaves a shape
-// below 2^-75) and weigh nothing, so d^2 may be formed with fused multiply-adds; with a smaller
-// radius (kCut) the reference's test d^2 <= r^2, on the reference's unfused d^2, drops them.
-// (The neighbour count, which needs the reference's test on every pair, is taken by the force
-// walk: this walk is bound by VALU issue, the force walk by its row gathers.)
-template <bool kCut>
-__device__ __forceinline__ float density_pair(const float4& pi, const float4& q,
-                                              const StepConsts& c, float half_inv_h, float acc) {
-    float d2;
-    if (kCut) {
-        d2 = dist2_exact(pi.x, pi.y, pi.z, q.x, q.y, q.z);
-    } else {
-        const float dx = pi.x - q.x, dy = pi.y - q.y, dz = pi.z - q.z;
-        d2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-    }
-    float w = w6_shape8(__builtin_amdgcn_sqrtf(d2), half_inv_h, c.inv_h);
-    if (kCut) w = d2 <= c.r2 ? w : 0.0f;
-    return __builtin_fmaf(q.w, w, acc);
-}
-
 // A value computed here, before whatever follows.  Pinning each pair's sum keeps it ahead of
 // the next step's refill branch, so the row it used is dead when the row after it is requested
 // and the two share registers; left to the compiler, the sums sink past the branches and the
@@ -217,22 +196,6 @@ __device__ __forceinline__ float density_run(BitWalk<kW>& bw, float4& q0, float4
     return acc;
 }
 
-// Density, the force rows of the particle (B = m/rho and C = B P / 4, so that
-// m_j (P_i + P_j) / (2 rho_j) = 2 ((P_i / 4) B_j + C_j); the 2 rides on dW/dq) and rho in
-// svr.w.
-__device__ __forceinline__ void density_epilogue(float sum, const float4& pi, uint32_t s,
-                                                 const StepConsts& c, float4* __restrict__ svr,
-                                                 ForceRow* __restrict__ rows) {
-    const float rho = c.sigma * (sum * (8.0f / 6.0f));  // 8.0f / 6.0f == 8 * (1.0f / 6.0f)
-    float4 v = svr[s];
-    v.w = rho;
-    svr[s] = v;
-    const float B = pi.w / rho;
-    const float P = c.k_gas * (rho - c.rho0);
-    rows[s].a = make_float4(pi.x, pi.y, pi.z, B);
-    rows[s].b = make_float4(v.x, v.y, v.z, 0.25f * B * P);
-}
-
 // Density pass over one chunk (kSplit false: all parts; true: the part of this wavefront,
 // three wavefronts per chunk, the sums finished by k_density_finish).  Seven wavefronts per
 // SIMD: the 15-word shapes' LDS allows it, and the walk is VALU-bound (a few spills outside
@@ -242,7 +205,8 @@ __device__ __forceinline__ void density_epilogue(float sum, const float4& pi, ui
 // allows (6 with two 12-word buffers, 4 with two 16-word ones).
 template <class Shape, bool kSplit, bool kCut>
 __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(kSplit ? 1 : Shape::density_waves, 8))) void k_density_walk(
-    const uint32_t* __restrict__ items, const uint32_t* __restrict__ nitems,
+    const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
+    const uint32_t* __restrict__ nitems,
     const float4* __restrict__ spm, const uint2* __restrict__ sq, float4* __restrict__ svr,
     ForceRow* __restrict__ rows, const uint32_t* __restrict__ skey,
     const uint32_t* __restrict__ cs, StepConsts c, const SceneGrid* __restrict__ scenes,
@@ -266,7 +230,7 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
     uint32_t s;
     bool active;
     float4 pi;
-    if (!load_chunk(item, items, nitems, skey, cs, spm, c, scenes, lane, ch, s, active, pi)) return;
+    if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
     const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
     init_sentinel<kLds>(lmask, lwj0, lane, c);
     MfmaFilter mf;
@@ -422,108 +386,6 @@ __global__ __launch_bounds__(256) void k_density_finish(
 // (src/sph_engine.cpp:390-443), integrate_leapfrog (:290-310) and
 // apply_boundary_conditions (src/particle.cpp:122-153).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void integrate_clamp(float4& p, float3& v, float3 a, float dt,
-                                                const StepConsts& c, const float* lo,
-                                                const float* hi) {
-#pragma clang fp contract(off)
-    float hx = 0.5f * a.x, hy = 0.5f * a.y, hz = 0.5f * a.z;
-    v.x = v.x + hx * dt;
-    v.y = v.y + hy * dt;
-    v.z = v.z + hz * dt;
-    p.x = p.x + v.x * dt;
-    p.y = p.y + v.y * dt;
-    p.z = p.z + v.z * dt;
-    v.x = v.x + hx * dt;
-    v.y = v.y + hy * dt;
-    v.z = v.z + hz * dt;
-    v.x = v.x * c.damping;
-    v.y = v.y * c.damping;
-    v.z = v.z * c.damping;
-    const float wd = -0.8f;
-    if (p.x < lo[0]) {
-        p.x = lo[0];
-        v.x = v.x * wd;
-    } else if (p.x > hi[0]) {
-        p.x = hi[0];
-        v.x = v.x * wd;
-    }
-    if (p.y < lo[1]) {
-        p.y = lo[1];
-        v.y = v.y * wd;
-    } else if (p.y > hi[1]) {
-        p.y = hi[1];
-        v.y = v.y * wd;
-    }
-    if (p.z < lo[2]) {
-        p.z = lo[2];
-        v.z = v.z * wd;
-    } else if (p.z > hi[2]) {
-        p.z = hi[2];
-        v.z = v.z * wd;
-    }
-}
-
-__device__ __forceinline__ float3 final_accel(float3 fp, float3 fv, float m_i, float rho_i,
-                                              const StepConsts& c) {
-    // explicit fused forms: left to contraction, the choice of which product to fuse can
-    // differ between the kernels that inline this, and so would their bits
-    const float fx = __builtin_fmaf(fp.x, c.grad_scale, fv.x * c.lap_scale);
-    const float fy = __builtin_fmaf(fp.y, c.grad_scale, fv.y * c.lap_scale);
-    const float fz = __builtin_fmaf(fp.z, c.grad_scale, fv.z * c.lap_scale);
-    const float m = c.formulation == 1 ? rho_i : m_i;
-    const float inv_m = 1.0f / m;
-    return make_float3(fx * inv_m, __builtin_fmaf(c.grav, m, fy) * inv_m, fz * inv_m);
-}
-
-// Pressure and viscosity sums of one target over neighbour rows (ForceRow a, b).
-// The self pair (r = 0, v_j = v_i) and the padding slot (B = C = 0) add exactly zero.  Pairs
-// the filter let through beyond the radius: with a radius of at least 2h they have q >= 2 (up
-// to rounding, which leaves a Laplacian factor below 3e-8 of a neighbour's) and add nothing;
-// with a smaller radius (kCut) the reference's test on its own d^2 drops them: d^2 is pushed
-// to 1e30, where both kernel factors clamp to zero.
-struct ForceSums {
-    float3 fp = make_float3(0.f, 0.f, 0.f);
-    float3 fv = make_float3(0.f, 0.f, 0.f);
-    template <bool kCut>
-    // `cnt` counts the pairs that pass the reference's test d^2 <= r^2 on the reference's
-    // unfused d^2 (the particle itself included): the engine's neighbour statistics.
-    __device__ __forceinline__ void add(const float4& pi, const float3& vi, float p_quarter,
-                                        const float4& a, const float4& b, const StepConsts& c,
-                                        uint32_t& cnt) {
-        const float rx = pi.x - a.x, ry = pi.y - a.y, rz = pi.z - a.z;
-        float d2 = dist2_exact(pi.x, pi.y, pi.z, a.x, a.y, a.z);
-        const bool in = d2 <= c.r2;
-        cnt += in ? 1u : 0u;
-        if (kCut) d2 = in ? d2 : 1e30f;
-        const float rinv = __builtin_amdgcn_rsqf(fmaxf(d2, 1e-30f));
-        const float rl = d2 * rinv;
-        // u = (2 - q) / 2 and s = 1 - q, clamped to [0, 1] by the instructions' clamp bit
-        // (seven operations, no select): dwq = (s - u)(s + u) = s^2 - u^2 is q (3q - 4) / 4
-        // for q <= 1 and -(2 - q)^2 / 4 beyond, proportional to dW/dq; lap = u - 2 s is
-        // (3q - 2) / 2 and (2 - q) / 2.  grad_scale and lap_scale carry the constant factors.
-        const float u =
-            __builtin_amdgcn_fmed3f(__builtin_fmaf(-0.5f * c.inv_h, rl, 1.0f), 0.0f, 1.0f);
-        const float s = __builtin_amdgcn_fmed3f(__builtin_fmaf(-c.inv_h, rl, 1.0f), 0.0f, 1.0f);
-        const float dwq = (s - u) * (s + u);
-        const float lap = __builtin_fmaf(-2.0f, s, u);
-        // gradW is zero below |r| = 1e-6 (src/kernels.cpp:96-98)
-        const float dw = rl >= 1e-6f ? dwq : 0.0f;
-        const float coef = __builtin_fmaf(p_quarter, a.w, b.w) * dw * rinv;
-        fp.x -= coef * rx;
-        fp.y -= coef * ry;
-        fp.z -= coef * rz;
-        const float cv = a.w * lap;
-        fv.x += cv * (b.x - vi.x);
-        fv.y += cv * (b.y - vi.y);
-        fv.z += cv * (b.z - vi.z);
-    }
-    // the sums (and the count) formed here, before whatever follows (see pinned)
-    __device__ __forceinline__ void pin(uint32_t& cnt) {
-        asm volatile("" : "+v"(fp.x), "+v"(fp.y), "+v"(fp.z), "+v"(fv.x), "+v"(fv.y),
-                     "+v"(fv.z), "+v"(cnt));
-    }
-};
-
 // The wavefront runs its largest lane count; rows are requested two neighbours ahead, in
 // three rotating register sets (a gather from L2 takes several hundred cycles, one step of
 // pair arithmetic about a hundred).
@@ -658,29 +520,6 @@ __device__ __forceinline__ void fold_parts_reg(float (&t)[6], ForceSums& f, int 
     f = ForceSums();
 }
 
-// Acceleration, leapfrog, clamp and the caller-order writes of one target.
-__device__ __forceinline__ void force_epilogue(const ForceSums& f, float4 pi, float3 vi,
-                                               float rho_i, float P_i, uint32_t s,
-                                               const SceneGrid& g, const StepConsts& c,
-                                               const uint32_t* __restrict__ sid,
-                                               const float* __restrict__ dt_dev, float dt_arg,
-                                               float4* __restrict__ pm, float4* __restrict__ vel,
-                                               float4* __restrict__ acc_out,
-                                               float* __restrict__ rho_out,
-                                               float* __restrict__ prs_out) {
-    const float3 a = final_accel(f.fp, f.fv, pi.w, rho_i, c);
-    const float dt = dt_dev ? *dt_dev : dt_arg;
-    float3 v = vi;
-    float4 p = pi;
-    integrate_clamp(p, v, a, dt, c, g.lo, g.hi);
-    const uint32_t id = sid[s];
-    pm[id] = p;
-    vel[id] = make_float4(v.x, v.y, v.z, 0.0f);
-    acc_out[id] = make_float4(a.x, a.y, a.z, 0.0f);
-    rho_out[id] = rho_i;
-    prs_out[id] = P_i;
-}
-
 // Force pass over one chunk (kSplit false: all parts; true: the part of this wavefront,
 // three wavefronts per chunk, finished by k_force_finish).  Shapes of 24 words and more keep
 // the parts' running total in registers: their LDS, not their registers, limits occupancy,
@@ -688,7 +527,8 @@ __device__ __forceinline__ void force_epilogue(const ForceSums& f, float4 pi, fl
 template <class Shape, bool kSplit, bool kCut>
 __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(Shape::force_waves)))
 void k_force_walk(
-    const uint32_t* __restrict__ items, const uint32_t* __restrict__ nitems,
+    const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
+    const uint32_t* __restrict__ nitems,
     const float4* __restrict__ spm, const uint2* __restrict__ sq,
     const float4* __restrict__ svr, const ForceRow* __restrict__ rows,
     const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sid,
@@ -722,7 +562,7 @@ void k_force_walk(
     uint32_t s;
     bool active;
     float4 pi;
-    if (!load_chunk(item, items, nitems, skey, cs, spm, c, scenes, lane, ch, s, active, pi)) return;
+    if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
     const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
     init_sentinel<kLds>(lmask, lwj0, lane, c);
     if (kLdsTot) {
@@ -1027,6 +867,7 @@ template <bool kTail>
 __global__ __launch_bounds__(256) void k_chunk_list(const uint32_t* __restrict__ cs, StepConsts c,
                                                     const SceneGrid* __restrict__ scenes,
                                                     uint32_t* __restrict__ items,
+                                                    uint4* __restrict__ desc,
                                                     uint32_t* __restrict__ nitems,
                                                     uint32_t fill_blocks, StepTail t) {
     if (blockIdx.x >= fill_blocks) {
@@ -1079,15 +920,14 @@ __global__ __launch_bounds__(256) void k_chunk_list(const uint32_t* __restrict__
     if (blockIdx.x == 0 && threadIdx.x == 0) nitems[0] = total;
     const uint32_t col = blockIdx.x * 256u + threadIdx.x;
     if (col >= ncols) return;
-    const uint2 r = one ? column_slots<true>(cs, scenes, c, g0, col)
-                        : column_slots<false>(cs, scenes, c, g0, col);
-    uint32_t o = off[col];
-    for (uint32_t s = r.x; s < r.y; s += 64u) items[o++] = s;
+    const uint32_t scene = one ? 0u : scene_of_col(scenes, c.nscenes, col);
+    const SceneGrid g = one ? g0 : scenes[scene];
+    column_items(column_slots<true>(cs, scenes, c, g, col), scene, g, col, off[col], items, desc);
 }
 
 hipError_t launch_chunks(const uint32_t* cell_start, const StepConsts& c, const SceneGrid* scenes,
                          uint32_t* cnt_scratch, uint32_t* scan_scratch, uint32_t* items,
-                         uint32_t* nitems, const StepTail* tail, hipStream_t st) {
+                         uint4* desc, uint32_t* nitems, const StepTail* tail, hipStream_t st) {
     // the non-finite bin holds at most n particles; its start is read on the device
     const uint32_t tail_blocks =
         tail ? std::max<uint32_t>(1u, std::min<uint32_t>((tail->n + 255u) / 256u, 64u)) : 0u;
@@ -1095,10 +935,10 @@ hipError_t launch_chunks(const uint32_t* cell_start, const StepConsts& c, const 
         const uint32_t fill_blocks = std::max<uint32_t>(1u, (c.ncols + 255u) / 256u);
         if (tail)
             hipLaunchKernelGGL(k_chunk_list<true>, dim3(fill_blocks + tail_blocks), dim3(256), 0,
-                               st, cell_start, c, scenes, items, nitems, fill_blocks, *tail);
+                               st, cell_start, c, scenes, items, desc, nitems, fill_blocks, *tail);
         else
             hipLaunchKernelGGL(k_chunk_list<false>, dim3(fill_blocks), dim3(256), 0, st,
-                               cell_start, c, scenes, items, nitems, fill_blocks, StepTail{});
+                               cell_start, c, scenes, items, desc, nitems, fill_blocks, StepTail{});
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_chunk_count, dim3((c.ncols + 1 + 255) / 256), dim3(256), 0, st,
@@ -1106,7 +946,7 @@ hipError_t launch_chunks(const uint32_t* cell_start, const StepConsts& c, const 
     hipError_t e = scan_exclusive(cnt_scratch, c.ncols + 1, scan_scratch, st);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_chunk_fill, dim3((c.ncols + 255) / 256 + 1), dim3(256), 0, st, cell_start,
-                       c, scenes, cnt_scratch, items, nitems);
+                       c, scenes, cnt_scratch, items, desc, nitems);
     if (tail)
         hipLaunchKernelGGL(k_nonfinite_step, dim3(tail_blocks), dim3(256), 0, st, *tail,
                            cell_start, c, scenes);
@@ -1119,7 +959,8 @@ hipError_t launch_chunks(const uint32_t* cell_start, const StepConsts& c, const 
 // ---------------------------------------------------------------------------
 template <class Shape>
 __global__ __launch_bounds__(Shape::threads) void k_nbr_lists(
-    const uint32_t* __restrict__ items, const uint32_t* __restrict__ nitems,
+    const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
+    const uint32_t* __restrict__ nitems,
     const float4* __restrict__ spm, const uint2* __restrict__ sq,
     const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sid,
     const uint32_t* __restrict__ cs, StepConsts c, const SceneGrid* __restrict__ scenes,
@@ -1139,7 +980,7 @@ __global__ __launch_bounds__(Shape::threads) void k_nbr_lists(
     float4 pi;
     const uint32_t wid = xcd_unit(uni(nitems[0]), Shape::waves, wave);
     if (wid == ~0u) return;
-    if (!load_chunk(wid, items, nitems, skey, cs, spm, c, scenes,
+    if (!load_chunk(wid, items, desc, nitems, skey, spm, c, scenes,
                     lane, ch, s, active, pi))
         return;
     const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
@@ -1242,7 +1083,7 @@ hipError_t launch_density_walk(const WalkBuffers& wb, const float4* spm, const u
 #define SPHK_DENSITY_LAUNCH(CUT)                                                            \
     SPHK_DISPATCH_SHAPE(shape, hipLaunchKernelGGL((k_density_walk<S, kS, CUT>),               \
                                                   dim3(grid_for<S>(chunks, kS)),             \
-                                                  dim3(S::threads), 0, st, wb.items,         \
+                                                  dim3(S::threads), 0, st, wb.items, wb.desc, \
                                                   wb.nitems, spm, sq, svr, rows, skey,       \
                                                   cell_start, c, scenes, wb.mask, wb.wj0,    \
                                                   wb.nwords, wb.pstarts, ps))
@@ -1273,7 +1114,7 @@ hipError_t launch_force_walk(const WalkBuffers& wb, const float4* spm, const uin
 #define SPHK_FORCE_LAUNCH(CUT)                                                              \
     SPHK_DISPATCH_SHAPE(shape, hipLaunchKernelGGL((k_force_walk<S, kS, CUT>),                 \
                                                   dim3(grid_for<S>(chunks, kS)),             \
-                                                  dim3(S::threads), 0, st, wb.items,         \
+                                                  dim3(S::threads), 0, st, wb.items, wb.desc, \
                                                   wb.nitems, spm, sq, svr, rows, skey, sid,  \
                                                   cell_start, c, scenes, wb.mask, wb.wj0,    \
                                                   wb.nwords, wb.pstarts, ps, dt_dev, dt, pm, \
@@ -1303,7 +1144,7 @@ hipError_t launch_nbr_lists(const WalkBuffers& wb, const float4* spm, const uint
     // ping-pong shape with the single-buffer shape of the same LDS size)
     const int base = shape == 5 ? 0 : shape == 6 ? 1 : shape == 7 ? 4 : shape == 8 ? 1 : shape;
     SPHK_DISPATCH_SHAPE(base, hipLaunchKernelGGL(k_nbr_lists<S>, dim3(grid_for<S>(chunks)),
-                                                  dim3(S::threads), 0, st, wb.items, wb.nitems,
+                                                  dim3(S::threads), 0, st, wb.items, wb.desc, wb.nitems,
                                                   spm, sq, skey, sid, cell_start, c, scenes,
                                                   pass, count_by_id, offsets_by_id, idx));
     return hipGetLastError();

@@ -676,31 +676,30 @@ __device__ __forceinline__ int phase1_table(const WordTable& t, int& i,
 // Builds the wave-uniform chunk description; returns false for an out-of-range item.
 // Lanes past the chunk get NaN coordinates, so every test fails for them.
 __device__ __forceinline__ bool load_chunk(uint32_t item, const uint32_t* __restrict__ items,
+                                           const uint4* __restrict__ desc,
                                            const uint32_t* __restrict__ nitems,
                                            const uint32_t* __restrict__ skey,
-                                           const uint32_t* __restrict__ cs,
                                            const float4* __restrict__ spm, const StepConsts& c,
                                            const SceneGrid* __restrict__ scenes, uint32_t lane,
                                            Chunk& ch, uint32_t& s, bool& active, float4& pi) {
     if (item >= uni(nitems[0])) return false;
     ch.s0 = uni(items[item]);
-    const uint32_t L0 = uni(skey[ch.s0]);
-    ch.scene = uni(scene_of_cell(scenes, c.nscenes, L0));
+    const uint4 d = desc[item];
+    s = ch.s0 + lane;
+    const float4 row = spm[min(s, c.pad_slot)];  // requested before the chain of lookups below
+    ch.s_end = uni(d.x);
+    ch.scene = uni(d.y);
+    ch.rx = unii((int)d.z);
+    ch.ry = unii((int)d.w);
     ch.cell_base = uni(scenes[ch.scene].cell_base);
     ch.ny = uni((uint32_t)scenes[ch.scene].ny);
     ch.nz = uni((uint32_t)scenes[ch.scene].nz);
-    const uint32_t local = L0 - ch.cell_base;
-    const uint32_t col = local / ch.nz;
-    const uint32_t col_end = uni(cs[ch.cell_base + (col + 1u) * ch.nz]);
-    ch.s_end = min(ch.s0 + 64u, col_end);
-    ch.rx = (int)(col / ch.ny);
-    ch.ry = (int)(col % ch.ny);
-    const int zmin = (int)(local % ch.nz);
-    const int zmax = (int)((uni(skey[ch.s_end - 1u]) - ch.cell_base) % ch.nz);
-    s = ch.s0 + lane;
+    const uint32_t first = ch.cell_base + ((uint32_t)ch.rx * ch.ny + (uint32_t)ch.ry) * ch.nz;
+    const int zmin = (int)(uni(skey[ch.s0]) - first);
+    const int zmax = (int)(uni(skey[ch.s_end - 1u]) - first);
     active = s < ch.s_end;
     const float qnan = __int_as_float(0x7fc00000);
-    pi = active ? spm[s] : make_float4(qnan, qnan, qnan, 0.0f);
+    pi = active ? row : make_float4(qnan, qnan, qnan, 0.0f);
     int fx = 0, fy = 0, fz = 0;
     const bool near = active && (axis_edge_near(pi.x, c.inv_cell) ||
                                  axis_edge_near(pi.y, c.inv_cell) ||
