@@ -32,7 +32,8 @@ constexpr int kSurH = 128;           // message hidden, message output and node 
 constexpr int kSurNF = 9;            // edge features
 constexpr int kSurNodeIn = 132;      // 128 + rho + v(3)
 constexpr int kSurRow = 144;         // row stride of S, X, Z (multiple of 16)
-constexpr int kSurOutRow = 32;       // row stride of the output-gradient rows (3 used)
+constexpr int kSurOutRow = 4;        // row stride of the output-gradient rows (3 used)
+constexpr uint32_t kSurSlabRows = 512;  // rows of one weight-gradient partial
 constexpr uint32_t kSurNoSlot = 0xffffffffu;
 
 // flat parameter offsets
@@ -72,24 +73,6 @@ struct SurScales {
     float rho0, rho_scale, msg_scale, acc_scale;
 };
 
-// Epilogues of the row GEMM C = A * Bt^T.
-enum SurEpi : int {
-    kEpiM = 0,    // X[:, :128] = bf16(C + cnt[row] * b2)
-    kEpiZ = 1,    // Z[:, :128] = bf16(ReLU(C + bn1))
-    kEpiOut = 2,  // OUT[row][0..2] = C + bn2           (FP32, 4 floats per row)
-    kEpiDZ = 3,   // DZ = Z > 0 ? bf16(C) : 0             (row stride 128)
-    kEpiDM = 4,   // DM = bf16(C)                         (row stride 128)
-    kEpiDS = 5,   // DS = bf16(c * C)                     (row stride 128)
-};
-
-struct SurEpiArgs {
-    void* out;          // destination
-    const float* bias;  // FP32 bias (bf16-rounded values)
-    const float* cnt;   // c * n_i per row (kEpiM)
-    const __bf16* z;    // Z rows (kEpiDZ)
-    float scale;        // kEpiDS
-};
-
 // Packs FP32 parameters into the bf16 operand images and the FP32 rounded copies.
 hipError_t launch_sur_pack(const float* params, __bf16* pk, float* pf, hipStream_t st);
 
@@ -127,18 +110,34 @@ hipError_t launch_sur_forward(bool integrate, const WalkBuffers& wb, const uint3
                               const SurScales& sc, const SurRows& rows, const SurStep& step,
                               hipStream_t st);
 
-// Row GEMM: C[R x N] = A[R x K] * Bt[N x K]^T (bf16, FP32 accumulate), R multiple of 32,
-// K multiple of 16, N <= 128 multiple of 32.
-hipError_t launch_sur_gemm(int epi, const __bf16* A, int lda, const __bf16* Bt, int ldb, int K,
-                           int N, uint32_t R, const SurEpiArgs& ep, hipStream_t st);
+// Gradient rows of a batch (bf16): output (stride kSurOutRow), z, m and S (stride 128).
+struct SurGradRows {
+    __bf16 *DOUT, *DZ, *DM, *DS;
+};
 
-// Weight gradient partials: part[slab][m][n] = sum over the slab's rows r of
-// P[r][m] * Q[r][n], m < M, n < N (tiles of 32).  rows_per_slab multiple of 16.
-hipError_t launch_sur_wgrad(const __bf16* P, int ldp, int M, const __bf16* Q, int ldq, int N,
-                            uint32_t R, uint32_t rows_per_slab, uint32_t slabs, float* part,
-                            hipStream_t st);
+// Gradient partials: weight gradients per slab of kSurSlabRows rows, [128 or 3][kSurRow] each
+// (bias column after the weight's), and of the message layer per batch chunk, [128][16].
+struct SurParts {
+    float *Wn1, *W2, *Wn2, *W1;
+};
+inline uint32_t sur_slabs(uint32_t R) { return (R + kSurSlabRows - 1) / kSurSlabRows; }
+// Loss partials (one pair per 128 rows).
+inline uint32_t sur_loss_parts(uint32_t R) { return (R + 127u) / 128u; }
 
-// Edge backward over a batch: partials part[2 b + half][128][16] of d(W1|b1): columns 0..8
+// Loss rows and the backward pass through the node MLP and the hoisted message layer for R
+// rows (a multiple of 64): DOUT = 2 (OUT - target) for rows with a slot (zero otherwise) and
+// the gradients behind it; loss_part gets the partial sums of squared errors and numbers of
+// rows with a slot, interleaved.  The 1/(3 rows) of the mean is applied by launch_sur_reduce.
+hipError_t launch_sur_node_bwd(const float4* out, const uint32_t* rowslot, const uint32_t* sid,
+                               const float4* target, uint32_t R, const __bf16* Z,
+                               const __bf16* pk, float msg_scale, const SurGradRows& g,
+                               float* loss_part, hipStream_t st);
+
+// Weight-gradient partials of (Wn1|bn1) = DZ^T X, (W2|b2) = DM^T S, (Wn2|bn2) = DOUT^T Z.
+hipError_t launch_sur_wgrad(const SurGradRows& g, const __bf16* S, const __bf16* X,
+                            const __bf16* Z, uint32_t R, const SurParts& parts, hipStream_t st);
+
+// Edge backward over a batch: partials part[b][128][16] of d(W1|b1): columns 0..8
 // are W1's, column 9 is b1.
 hipError_t launch_sur_edges_bwd(const WalkBuffers& wb, const uint32_t* batch, uint32_t nbatch,
                                 const float4* spm, const float4* svr, const uint32_t* skey,
@@ -146,19 +145,9 @@ hipError_t launch_sur_edges_bwd(const WalkBuffers& wb, const uint32_t* batch, ui
                                 const SceneGrid* scenes, const __bf16* pk, const SurScales& sc,
                                 const __bf16* DS, float* part, hipStream_t st);
 
-// Sums `slabs` partial matrices [M_all][ld] into grad: rows m < M, columns n < ncols go to
-// grad[dst + m * ncols + n]; column bias_col (if >= 0) goes to grad[bias_dst + m].
-// Every value is multiplied by `scale`.
-hipError_t launch_sur_reduce(const float* part, uint32_t slabs, int M_all, int ld, int M,
-                             int ncols, int bias_col, uint32_t dst, uint32_t bias_dst,
-                             float scale, float* grad, hipStream_t st);
-
-// Loss rows: DOUT = 2 (OUT - target) for rows with a slot (zero otherwise); per block the
-// partial sum of squared errors and the number of rows with a slot, interleaved.  The
-// 1/(3B) of the mean is applied when the weight gradients are reduced.
-hipError_t launch_sur_loss(const float* out, const uint32_t* rowslot, const uint32_t* sid,
-                           const float4* target, uint32_t R, __bf16* dout, float* loss_part,
-                           uint32_t* nparts, hipStream_t st);
+// Sums the partials of all parameters into grad, scaled by 1 / (3 rows with a slot).
+hipError_t launch_sur_reduce(const SurParts& parts, uint32_t R, uint32_t nbatch,
+                             const float* loss_part, float* grad, hipStream_t st);
 
 // Targets (normalised): t[id] = (v4 - d^k v0) / (T a_s).
 hipError_t launch_sur_targets(const float4* v0, const float4* v4, uint32_t n, float dk,

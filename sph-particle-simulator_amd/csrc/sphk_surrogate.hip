@@ -135,6 +135,25 @@ __device__ __forceinline__ void layer1_a(bf16x8 fe, __bf16 e8, bool edge, uint32
     a1 = hi ? fe : other;
 }
 
+typedef short short2v __attribute__((ext_vector_type(2)));
+
+// All eight values with their sign flipped.
+__device__ __forceinline__ bf16x8 negated(bf16x8 x) {
+    uint4 w = __builtin_bit_cast(uint4, x);
+    w.x ^= 0x80008000u;
+    w.y ^= 0x80008000u;
+    w.z ^= 0x80008000u;
+    w.w ^= 0x80008000u;
+    return __builtin_bit_cast(bf16x8, w);
+}
+
+// 16-bit masks of a pair: all ones where the value's sign bit is set (a in the low half).
+__device__ __forceinline__ uint32_t neg_masks(float a, float b) {
+    const uint32_t hi =
+        __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(short2v, hi) >> (short)15);
+}
+
 constexpr int kEdgeWaves = 2;   // one chunk per workgroup: 32 targets per wavefront
 constexpr int kStage = 136;     // LDS row stride (bf16) of staged 128-wide rows
 constexpr int kStageX = 152;    // LDS row stride (bf16) of staged node-input rows
@@ -448,83 +467,262 @@ k_sur_forward(WalkBuffers wb, const uint32_t* __restrict__ batch, uint32_t nbatc
 }
 
 // ---------------------------------------------------------------------------
-// row GEMM: one wavefront per 32 rows, all N columns (tiles of 32)
+// Loss and the backward pass through the node MLP and the hoisted message layer, 32 batch rows
+// per wavefront:
+//   d = OUT - target (zero without a slot), DOUT = 2 d, DZ = (Wn2^T DOUT) [Z > 0],
+//   DM = Wn1^T DZ, DS = c W2^T DM.
+// One launch instead of a loss kernel and three row GEMMs: the rows stay in one LDS tile per
+// wavefront, which feeds the next product's A operand and the 16-byte row stores, and Z is the
+// only activation read.  Bound by memory: 0.3 KB read and 0.8 KB written a row.
+// 65,536 rows: loss and products 61 -> 32 us.
+// Per workgroup: the partial sum of squared errors and the number of rows with a slot.
 // ---------------------------------------------------------------------------
-template <int kEpi, int kNT>
-__global__ __launch_bounds__(256) void k_sur_gemm(const __bf16* __restrict__ A, int lda,
-                                                  const __bf16* __restrict__ Bt, int ldb, int K,
-                                                  uint32_t R, SurEpiArgs ep) {
+constexpr uint32_t kNodeWaves = 4;
+
+__global__ __launch_bounds__(64 * kNodeWaves) void k_sur_node_bwd(
+    const float4* __restrict__ out, const uint32_t* __restrict__ rowslot,
+    const uint32_t* __restrict__ sid, const float4* __restrict__ target, uint32_t R,
+    const __bf16* __restrict__ Z, const __bf16* __restrict__ pk, float msg_scale, SurGradRows g,
+    float* __restrict__ loss_part) {
+    __shared__ alignas(16) __bf16 stage_all[kNodeWaves][32 * kStage];
+    __shared__ float red[kNodeWaves], redc[kNodeWaves];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t row0 = (blockIdx.x * 4u + wave) * 32u;
-    if (row0 >= R) return;
     const uint32_t h = lane >> 5, col = lane & 31u;
-    f32x16 acc[kNT];
+    const uint32_t row0 = (blockIdx.x * kNodeWaves + wave) * 32u;
+    __bf16* E = stage_all[wave];
+    float l = 0.0f, cnt = 0.0f;
+    if (row0 < R) {  // R is a multiple of 32
+        const uint32_t row = row0 + col;
+        // 16-byte pieces of 128-wide rows: lane l takes pieces l, l + 64, ... of the 32 x 16
 #pragma unroll
-    for (int t = 0; t < kNT; ++t) acc[t] = zero16();
-    const __bf16* ap = A + (size_t)(row0 + col) * lda + 8u * h;
-    const __bf16* bp = Bt + (size_t)col * ldb + 8u * h;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const bf16x8 a = load8(ap + k0);
-#pragma unroll
-        for (int t = 0; t < kNT; ++t) acc[t] = mfma16(a, load8(bp + (size_t)t * 32 * ldb + k0), acc[t]);
-    }
-#pragma unroll
-    for (int t = 0; t < kNT; ++t) {
-        const uint32_t n = 32u * t + col;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const size_t row = row0 + acc_row(v, h);
-            const float x = acc[t][v];
-            if constexpr (kEpi == kEpiM) {
-                static_cast<__bf16*>(ep.out)[row * kSurRow + n] =
-                    (__bf16)(x + ep.cnt[row] * ep.bias[n]);
-            } else if constexpr (kEpi == kEpiZ) {
-                static_cast<__bf16*>(ep.out)[row * kSurRow + n] = (__bf16)fmaxf(x + ep.bias[n], 0.0f);
-            } else if constexpr (kEpi == kEpiOut) {
-                if (n < 3u) static_cast<float*>(ep.out)[row * 4 + n] = x + ep.bias[n];
-            } else if constexpr (kEpi == kEpiDZ) {
-                const bool on = (float)ep.z[row * kSurRow + n] > 0.0f;
-                static_cast<__bf16*>(ep.out)[row * 128 + n] = (__bf16)(on ? x : 0.0f);
-            } else if constexpr (kEpi == kEpiDM) {
-                static_cast<__bf16*>(ep.out)[row * 128 + n] = (__bf16)x;
-            } else {
-                static_cast<__bf16*>(ep.out)[row * 128 + n] = (__bf16)(ep.scale * x);
-            }
+        for (uint32_t k = 0; k < 8u; ++k) {
+            const uint32_t r = 4u * k + (lane >> 4), piece = lane & 15u;
+            *reinterpret_cast<uint4*>(E + r * kStage + 8u * piece) =
+                *reinterpret_cast<const uint4*>(Z + (size_t)(row0 + r) * kSurRow + 8u * piece);
         }
+        bf16x8 a = zero8();
+        if (h == 0u) {
+            const uint32_t slot = rowslot[row];
+            float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f;
+            if (slot != kSurNoSlot) {
+                cnt = 1.0f;
+                const float4 t = target[sid[slot]];
+                const float4 o = out[row];
+                d0 = o.x - t.x;
+                d1 = o.y - t.y;
+                d2 = o.z - t.z;
+                l = (d0 * d0 + d1 * d1) + d2 * d2;
+            }
+            a[0] = (__bf16)(2.0f * d0);
+            a[1] = (__bf16)(2.0f * d1);
+            a[2] = (__bf16)(2.0f * d2);
+            const uint4 w = __builtin_bit_cast(uint4, a);
+            *reinterpret_cast<uint2*>(g.DOUT + (size_t)row * kSurOutRow) = make_uint2(w.x, w.y);
+        }
+        wave_sync();
+        f32x16 acc[4];
+        // rows of the tile to global memory, 16 bytes a lane
+        auto store_rows = [&](__bf16* dst) {
+            wave_sync();
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) {
+                const uint32_t r = 4u * k + (lane >> 4), piece = lane & 15u;
+                *reinterpret_cast<uint4*>(dst + (size_t)(row0 + r) * 128u + 8u * piece) =
+                    *reinterpret_cast<const uint4*>(E + r * kStage + 8u * piece);
+            }
+        };
+        // DZ: the three output gradients are one K step (k = 0..2)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            acc[t] = mfma16(a, load8(pk + kPkWn2T + (32u * t + col) * 32u + 8u * h), zero16());
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                __bf16* e = E + acc_row(v, h) * kStage + 32u * t + col;
+                *e = (__bf16)((float)*e > 0.0f ? acc[t][v] : 0.0f);
+            }
+        store_rows(g.DZ);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = zero16();
+        tile_gemm(acc, E, kStage, pk + kPkWn1T, 128, 8, 4, lane);
+        wave_sync();
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                E[acc_row(v, h) * kStage + 32u * t + col] = (__bf16)acc[t][v];
+        store_rows(g.DM);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = zero16();
+        tile_gemm(acc, E, kStage, pk + kPkW2T, 128, 8, 4, lane);
+        wave_sync();
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                E[acc_row(v, h) * kStage + 32u * t + col] = (__bf16)(msg_scale * acc[t][v]);
+        store_rows(g.DS);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        l += __shfl_xor(l, off);
+        cnt += __shfl_xor(cnt, off);
+    }
+    if (lane == 0) {
+        red[wave] = l;
+        redc[wave] = cnt;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        loss_part[2 * blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+        loss_part[2 * blockIdx.x + 1] = (redc[0] + redc[1]) + (redc[2] + redc[3]);
     }
 }
 
 // ---------------------------------------------------------------------------
-// weight-gradient partials: one wavefront per (32 x 32 tile, row slab)
+// weight-gradient partials P^T Q of a slab of kSurSlabRows rows (K = rows), one workgroup per
+// slab and product.  An operand needs 8 consecutive rows of one column; which columns form a
+// 32-wide tile is free, so a lane loads the 2 (P) or 4 (Q) neighbouring columns of 8 rows with
+// wide, coalesced loads and its column t belongs to tile t: a byte permute per operand dword
+// does the transpose, no LDS.  The 16 columns of Q beyond 128 (the bias columns and the last
+// node inputs) are a fifth tile.  The next K step's rows are requested before this one's
+// products.  Bound by the read of the rows (4.6 KB and 5 KB a K step of 16): 65,536 rows,
+// three products 218 -> 25 us, against one 32 x 32 tile per wavefront with 2-byte loads.
+// kMT 2: P has 128 columns; two wavefronts split them, two pairs split the rows.
+// kMT 1: P is the output gradient (3 of 4 columns); the four wavefronts split the rows.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_sur_wgrad(const __bf16* __restrict__ P, int ldp, int M,
-                                                  const __bf16* __restrict__ Q, int ldq, int N,
-                                                  uint32_t R, uint32_t rps,
-                                                  float* __restrict__ part) {
-    const int ntn = (N + 31) / 32;
-    const int tm = blockIdx.x / ntn, tn = blockIdx.x % ntn;
-    const uint32_t slab = blockIdx.y;
-    const uint32_t lane = threadIdx.x, h = lane >> 5, col = lane & 31u;
-    const int m = 32 * tm + (int)col, n = 32 * tn + (int)col;
-    const uint32_t r_begin = slab * rps;
-    const uint32_t r_end = min(R, r_begin + rps);
-    f32x16 acc = zero16();
-    for (uint32_t r0 = r_begin; r0 < r_end; r0 += 16u) {
-        bf16x8 a, b;
+struct WgradStep {
+    uint32_t p[8];
+    uint2 q[8];
+    uint32_t x[8];
+};
+
+template <int kMT>
+__device__ __forceinline__ void wgrad_load(WgradStep& w, const __bf16* __restrict__ P,
+                                           const __bf16* __restrict__ Q, uint32_t r,
+                                           uint32_t lane) {
+    const uint32_t h = lane >> 5, col = lane & 31u;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t r = r0 + 8u * h + i;
-            const bool in = r < r_end;
-            a[i] = (in && m < M) ? P[(size_t)r * ldp + m] : (__bf16)0.0f;
-            b[i] = (in && n < N) ? Q[(size_t)r * ldq + n] : (__bf16)0.0f;
+    for (uint32_t i = 0; i < 8u; ++i) {
+        const size_t row = r + 8u * h + i;
+        if (kMT == 2)
+            w.p[i] = *reinterpret_cast<const uint32_t*>(P + row * 128u + 2u * col);
+        else
+            w.p[i] = bits16(P[row * kSurOutRow + min(col, 3u)]);  // column 3 is zero
+        w.q[i] = *reinterpret_cast<const uint2*>(Q + row * kSurRow + 4u * col);
+        w.x[i] = bits16(Q[row * kSurRow + 128u + min(col, 15u)]);
+    }
+}
+
+// Operand of one column from 8 rows' dwords: its low (kHi false) or high halves.
+template <bool kHi>
+__device__ __forceinline__ bf16x8 column8(const uint32_t (&d)[8]) {
+    uint32_t w[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        w[k] = __builtin_amdgcn_perm(d[2 * k + 1], d[2 * k], kHi ? 0x07060302u : 0x05040100u);
+    return __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+}
+
+template <int kMT>
+__device__ __forceinline__ void wgrad_mfma(const WgradStep& w, f32x16 (&acc)[kMT][5]) {
+    bf16x8 a[kMT];
+    a[0] = column8<false>(w.p);
+    if (kMT == 2) a[kMT - 1] = column8<true>(w.p);
+    uint32_t lo[8], hi[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        lo[i] = w.q[i].x;
+        hi[i] = w.q[i].y;
+    }
+    const bf16x8 b[5] = {column8<false>(lo), column8<true>(lo), column8<false>(hi),
+                         column8<true>(hi), column8<false>(w.x)};
+#pragma unroll
+    for (int m = 0; m < kMT; ++m)
+#pragma unroll
+        for (int n = 0; n < 5; ++n) acc[m][n] = mfma16(a[m], b[n], acc[m][n]);
+}
+
+template <int kMT>
+__device__ __forceinline__ void wgrad_slab(const __bf16* __restrict__ P,
+                                           const __bf16* __restrict__ Q, uint32_t R,
+                                           uint32_t slab, float* __restrict__ part,
+                                           float* __restrict__ fold) {
+    constexpr uint32_t kParts = kMT == 2 ? 2u : 4u;  // row parts of the slab
+    constexpr uint32_t kRows = kSurSlabRows / kParts;
+    static_assert(kRows % 32u == 0u, "K steps are taken in pairs");
+    const uint32_t wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t h = lane >> 5, col = lane & 31u;
+    const uint32_t mhalf = kMT == 2 ? wave & 1u : 0u;
+    const uint32_t rp = kMT == 2 ? wave >> 1 : wave;
+    const uint32_t r_begin = slab * kSurSlabRows + rp * kRows;
+    const uint32_t r_end = min(R, r_begin + kRows);  // R is a multiple of 64
+    f32x16 acc[kMT][5];
+#pragma unroll
+    for (int m = 0; m < kMT; ++m)
+#pragma unroll
+        for (int n = 0; n < 5; ++n) acc[m][n] = zero16();
+    if (r_begin < r_end) {
+        const __bf16* Pw = P + 64u * mhalf;
+        WgradStep w0, w1;
+        wgrad_load<kMT>(w0, Pw, Q, r_begin, lane);
+        for (uint32_t r = r_begin; r < r_end; r += 32u) {
+            wgrad_load<kMT>(w1, Pw, Q, r + 16u, lane);
+            wgrad_mfma<kMT>(w0, acc);
+            wgrad_load<kMT>(w0, Pw, Q, r + 32u < r_end ? r + 32u : r, lane);
+            wgrad_mfma<kMT>(w1, acc);
         }
-        acc = mfma16(a, b, acc);
+    }
+    // row parts in order: parts 1.. go through LDS to part 0's wavefront
+    constexpr uint32_t kVals = kMT * 5u * 16u;
+    if (rp > 0u) {
+        float* f = fold + (size_t)((rp - 1u) * (kMT == 2 ? 2u : 1u) + mhalf) * kVals * 64u;
+#pragma unroll
+        for (int m = 0; m < kMT; ++m)
+#pragma unroll
+            for (int n = 0; n < 5; ++n)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    f[((m * 5 + n) * 16 + v) * 64 + lane] = acc[m][n][v];
+    }
+    __syncthreads();
+    if (rp > 0u) return;
+#pragma unroll
+    for (uint32_t q = 0; q + 1u < kParts; ++q) {
+        const float* f = fold + (size_t)(q * (kMT == 2 ? 2u : 1u) + mhalf) * kVals * 64u;
+#pragma unroll
+        for (int m = 0; m < kMT; ++m)
+#pragma unroll
+            for (int n = 0; n < 5; ++n)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[m][n][v] += f[((m * 5 + n) * 16 + v) * 64 + lane];
     }
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int mm = 32 * tm + (int)acc_row(v, h);
-        if (mm < M && n < N) part[((size_t)slab * M + mm) * N + n] = acc[v];
-    }
+    for (int m = 0; m < kMT; ++m)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const uint32_t i = acc_row(v, h);
+            const uint32_t row = kMT == 2 ? 64u * mhalf + 2u * i + m : i;
+            if (kMT == 1 && row >= 3u) continue;
+            float* o = part + (size_t)row * kSurRow;
+            *reinterpret_cast<float4*>(o + 4u * col) =
+                make_float4(acc[m][0][v], acc[m][1][v], acc[m][2][v], acc[m][3][v]);
+            if (col < 16u) o[128u + col] = acc[m][4][v];
+        }
+}
+
+__global__ __launch_bounds__(256) void k_sur_wgrad(SurGradRows g, const __bf16* __restrict__ S,
+                                                   const __bf16* __restrict__ X,
+                                                   const __bf16* __restrict__ Z, uint32_t R,
+                                                   SurParts parts) {
+    __shared__ float fold[2 * 160 * 64];
+    const uint32_t slab = blockIdx.x;
+    if (blockIdx.y == 0)
+        wgrad_slab<2>(g.DZ, X, R, slab, parts.Wn1 + (size_t)slab * 128u * kSurRow, fold);
+    else if (blockIdx.y == 1)
+        wgrad_slab<2>(g.DM, S, R, slab, parts.W2 + (size_t)slab * 128u * kSurRow, fold);
+    else
+        wgrad_slab<1>(g.DOUT, Z, R, slab, parts.Wn2 + (size_t)slab * 3u * kSurRow, fold);
 }
 
 // ---------------------------------------------------------------------------
@@ -532,15 +730,28 @@ __global__ __launch_bounds__(64) void k_sur_wgrad(const __bf16* __restrict__ P, 
 // gradient is formed in the accumulator layout of the recomputed layer-1 product and fed
 // back as an A operand (K = edges); the edge features reach the B operand through LDS.  One
 // workgroup per batch chunk, 32 targets per wavefront.
+//
+// Bound by VALU issue and the latency of its LDS and MFMA chain (two wavefronts per SIMD).
+//  - The layer-1 product is taken with negated weights, so u > 0 is the sign bit of the
+//    result: per pair of values one byte permute (the two high halves), one packed 16-bit shift
+//    (two masks) and one AND with the bf16 gradient pair, instead of two compares, two
+//    selects and a conversion.
+//  - The features are written to LDS as ten rows of 64 edges, in the order the B operand takes
+//    them (the accumulator's row order), so an operand is one 16-byte read instead of eight
+//    2-byte ones and their packing.
+// 1,024 chunks: 600 -> 272 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64 * kEdgeWaves) void k_sur_edges_bwd(
+constexpr uint32_t kEdgeRow = 72;  // LDS row stride (bf16) of one feature over 64 edges
+
+__global__ __launch_bounds__(64 * kEdgeWaves) __attribute__((amdgpu_waves_per_eu(2))) void
+k_sur_edges_bwd(
     WalkBuffers wb, const uint32_t* __restrict__ batch, uint32_t nbatch,
     const float4* __restrict__ spm, const float4* __restrict__ svr,
     const uint32_t* __restrict__ skey, const uint32_t* __restrict__ cs, StepConsts c,
     const SceneGrid* __restrict__ scenes, const __bf16* __restrict__ pk, SurScales sc,
     const __bf16* __restrict__ DS, float* __restrict__ part) {
     __shared__ WalkLds lds_all[kEdgeWaves];
-    __shared__ __bf16 le_all[kEdgeWaves][64 * 16];
+    __shared__ alignas(16) __bf16 le_all[kEdgeWaves][10 * kEdgeRow];
     const uint32_t half = uni(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t col = lane & 31u, h = lane >> 5;
@@ -560,14 +771,27 @@ __global__ __launch_bounds__(64 * kEdgeWaves) void k_sur_edges_bwd(
     const float4 vi = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 0.f);
     Layer1B B;
     load_layer1(pk, lane, B);
-    float ds[4][16];
+#pragma unroll
+    for (int hb = 0; hb < 4; ++hb) {
+        B.blk0[hb] = negated(B.blk0[hb]);
+        B.blk1[hb] = negated(B.blk1[hb]);
+    }
+    // dS of this lane's hidden units for the 16 accumulator rows, as bf16 pairs (rows v, v + 1)
+    uint32_t ds[4][8];
 #pragma unroll
     for (int hb = 0; hb < 4; ++hb)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const size_t row = 64u * (size_t)b + 32u * half + acc_row(v, h);
-            ds[hb][v] = (float)DS[row * 128 + 32u * hb + col];
+        for (int k = 0; k < 8; ++k) {
+            const size_t row = 64u * (size_t)b + 32u * half;
+            const __bf16* d = DS + 32u * hb + col;
+            ds[hb][k] = bits16(d[(row + acc_row(2 * k, h)) * 128u]) |
+                        bits16(d[(row + acc_row(2 * k + 1, h)) * 128u]) << 16;
         }
+    // where this lane's edge goes in a feature row: operand (block, g), lane half, element
+    const uint32_t epos =
+        (lane & 32u) + (col & 16u) + ((col >> 2) & 1u) * 8u + ((col >> 3) & 1u) * 4u + (col & 3u);
+    // this lane's feature row (columns from 10 on are garbage that is never stored)
+    const __bf16* erow = le + min(col, 9u) * kEdgeRow + 8u * h;
     f32x16 accw[4];
 #pragma unroll
     for (int hb = 0; hb < 4; ++hb) accw[hb] = zero16();
@@ -576,70 +800,109 @@ __global__ __launch_bounds__(64 * kEdgeWaves) void k_sur_edges_bwd(
                    bf16x8 fe;
                    __bf16 e8;
                    edge_features(edge, pi, vi, pj, vj, d2, sc, fe, e8);
-                   // E row of this lane's edge: [features 0..8, 1, 0 ...]
-                   bf16x8 ext = zero8();
-                   ext[0] = e8;
-                   ext[1] = (__bf16)(edge ? 1.0f : 0.0f);
-                   *reinterpret_cast<bf16x8*>(le + lane * 16) = fe;
-                   *reinterpret_cast<bf16x8*>(le + lane * 16 + 8) = ext;
+                   // features 0..8 and 1 of this lane's edge
+#pragma unroll
+                   for (int k = 0; k < 8; ++k) le[k * kEdgeRow + epos] = fe[k];
+                   le[8 * kEdgeRow + epos] = e8;
+                   le[9 * kEdgeRow + epos] = (__bf16)(edge ? 1.0f : 0.0f);
                    wave_sync();
                    bf16x8 a[2];
                    layer1_a(fe, e8, edge, lane, a[0], a[1]);
 #pragma unroll
                    for (int blk = 0; blk < 2; ++blk) {
-                       bf16x8 e[2];
-#pragma unroll
-                       for (int g = 0; g < 2; ++g)
-#pragma unroll
-                           for (int i = 0; i < 8; ++i) {
-                               const uint32_t er = 32u * blk + 16u * g + acc_row(i, h);
-                               e[g][i] = col < 10u ? le[er * 16 + col] : (__bf16)0.0f;
-                           }
+                       const bf16x8 e0 = load8(erow + 32 * blk);
+                       const bf16x8 e1 = load8(erow + 32 * blk + 16);
 #pragma unroll
                        for (int hb = 0; hb < 4; ++hb) {
+                           // -u of 16 edges
                            const f32x16 d =
                                mfma16(a[blk], blk == 0 ? B.blk0[hb] : B.blk1[hb], zero16());
-                           bf16x8 g0, g1;
+                           uint32_t g[8];
 #pragma unroll
-                           for (int i = 0; i < 8; ++i) {
-                               g0[i] = (__bf16)(d[i] > 0.0f ? ds[hb][i] : 0.0f);
-                               g1[i] = (__bf16)(d[8 + i] > 0.0f ? ds[hb][8 + i] : 0.0f);
-                           }
-                           accw[hb] = mfma16(g0, e[0], accw[hb]);
-                           accw[hb] = mfma16(g1, e[1], accw[hb]);
+                           for (int k = 0; k < 8; ++k) g[k] = ds[hb][k] & neg_masks(d[2 * k], d[2 * k + 1]);
+                           accw[hb] = mfma16(
+                               __builtin_bit_cast(bf16x8, make_uint4(g[0], g[1], g[2], g[3])), e0,
+                               accw[hb]);
+                           accw[hb] = mfma16(
+                               __builtin_bit_cast(bf16x8, make_uint4(g[4], g[5], g[6], g[7])), e1,
+                               accw[hb]);
                        }
                    }
                    wave_sync();
                });
-    if (col < 16u) {
-        const size_t pbase = (2u * (size_t)b + half) * 128u;
+    // the chunk's partial: half 0 plus half 1 (through LDS, the list is free)
+    float* fold = reinterpret_cast<float*>(&lds_all[1]);  // [64 values][64 lanes]
+    if (half == 1u) {
 #pragma unroll
         for (int hb = 0; hb < 4; ++hb)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const uint32_t m = 32u * hb + acc_row(v, h);
-                part[(pbase + m) * 16u + col] = accw[hb][v];
-            }
+            for (int v = 0; v < 16; ++v) fold[(hb * 16 + v) * 64 + lane] = accw[hb][v];
     }
+    __syncthreads();
+    if (half == 1u || col >= 16u) return;
+#pragma unroll
+    for (int hb = 0; hb < 4; ++hb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const uint32_t m = 32u * hb + acc_row(v, h);
+            part[((size_t)b * 128u + m) * 16u + col] =
+                accw[hb][v] + fold[(hb * 16 + v) * 64 + lane];
+        }
 }
 
 // ---------------------------------------------------------------------------
 // small element-wise kernels
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_sur_reduce(const float* __restrict__ part,
-                                                    uint32_t slabs, int M_all, int ld, int M,
-                                                    int ncols, int bias_col, uint32_t dst,
-                                                    uint32_t bias_dst, float scale,
-                                                    float* __restrict__ grad) {
-    const int per_row = ncols + (bias_col >= 0 ? 1 : 0);
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= M * per_row) return;
-    const int m = i / per_row, k = i % per_row;
-    const int n = k < ncols ? k : bias_col;
+// Gradient of every parameter from the partials of all four products, one launch: a workgroup
+// sums 16 columns of one partial row, 16 threads per column, each a sixteenth of the slabs in
+// order, then folds the sixteen in order.  Scaled by 1 / (3 rows), rows counted in the loss
+// partials (0 when no row has a slot).  Bound by the read of the partials: a chain of 8 slabs
+// (weights) or 64 (edges) per thread instead of one thread per parameter over all of them:
+// 1,024 chunks, four reductions 532 -> 13 us.
+struct SurReduceTask {
+    const float* part;
+    uint32_t slabs, rows, ld;  // partials [slabs][rows][ld]
+    uint32_t ncols;            // columns of the weight; column ncols is the bias
+    uint32_t dst, bias_dst;
+    uint32_t first;            // first workgroup of the task
+};
+struct SurReduceTasks {
+    SurReduceTask t[4];
+};
+
+__global__ __launch_bounds__(256) void k_sur_reduce(SurReduceTasks tasks,
+                                                    const float* __restrict__ loss_part,
+                                                    uint32_t nparts, float* __restrict__ grad) {
+    __shared__ float sums[16][17];
+    __shared__ uint32_t lrows[4];
+    int ti = 0;
+    while (ti < 3 && blockIdx.x >= tasks.t[ti + 1].first) ++ti;
+    const SurReduceTask& t = tasks.t[ti];
+    const uint32_t cblocks = (t.ncols + 16u) / 16u;  // of ncols + 1 columns
+    const uint32_t wg = blockIdx.x - t.first;
+    const uint32_t m = wg / cblocks, n = (wg % cblocks) * 16u + (threadIdx.x & 15u);
+    const uint32_t grp = threadIdx.x >> 4;
+    const uint32_t per = (t.slabs + 15u) / 16u;
+    const uint32_t sl0 = min(grp * per, t.slabs), sl1 = min(sl0 + per, t.slabs);
+    const float* p = t.part + (size_t)m * t.ld + n;  // ld is a multiple of 16
+    const size_t stride = (size_t)t.rows * t.ld;
     float sum = 0.0f;
-    for (uint32_t sl = 0; sl < slabs; ++sl) sum += part[((size_t)sl * M_all + m) * ld + n];
-    if (k < ncols) grad[dst + (uint32_t)(m * ncols + n)] = scale * sum;
-    else grad[bias_dst + (uint32_t)m] = scale * sum;
+#pragma unroll 8
+    for (uint32_t sl = sl0; sl < sl1; ++sl) sum += p[sl * stride];
+    sums[grp][threadIdx.x & 15u] = sum;
+    uint32_t cnt = 0;
+    for (uint32_t b = threadIdx.x; b < nparts; b += 256u) cnt += (uint32_t)loss_part[2u * b + 1u];
+    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
+    if ((threadIdx.x & 63u) == 0u) lrows[threadIdx.x >> 6] = cnt;
+    __syncthreads();
+    if (grp != 0u || n > t.ncols) return;
+    const uint32_t rows = (lrows[0] + lrows[1]) + (lrows[2] + lrows[3]);
+    const float scale = rows ? (float)(1.0 / (3.0 * (double)rows)) : 0.0f;
+    float tot = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) tot += sums[k][threadIdx.x];
+    if (n < t.ncols) grad[t.dst + m * t.ncols + n] = scale * tot;
+    else grad[t.bias_dst + m] = scale * tot;
 }
 
 __device__ __forceinline__ float block_sum_256(float x, float* red) {
@@ -647,47 +910,6 @@ __device__ __forceinline__ float block_sum_256(float x, float* red) {
     if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = x;
     __syncthreads();
     return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-__global__ __launch_bounds__(256) void k_sur_loss(const float* __restrict__ out,
-                                                  const uint32_t* __restrict__ rowslot,
-                                                  const uint32_t* __restrict__ sid,
-                                                  const float4* __restrict__ target, uint32_t R,
-                                                  float scale, __bf16* __restrict__ dout,
-                                                  float* __restrict__ loss_part) {
-    __shared__ float red[4];
-    __shared__ float redc[4];
-    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
-    float l = 0.0f, cnt = 0.0f;
-    if (r < R) {
-        const uint32_t slot = rowslot[r];
-        float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f;
-        if (slot != kSurNoSlot) {
-            cnt = 1.0f;
-            const float4 t = target[sid[slot]];
-            d0 = out[4 * (size_t)r] - t.x;
-            d1 = out[4 * (size_t)r + 1] - t.y;
-            d2 = out[4 * (size_t)r + 2] - t.z;
-            l = (d0 * d0 + d1 * d1) + d2 * d2;
-        }
-        const __bf16 g0 = (__bf16)(scale * d0), g1 = (__bf16)(scale * d1),
-                     g2 = (__bf16)(scale * d2);
-        uint4 v = make_uint4((uint32_t)__builtin_bit_cast(uint16_t, g0) |
-                                 ((uint32_t)__builtin_bit_cast(uint16_t, g1) << 16),
-                             (uint32_t)__builtin_bit_cast(uint16_t, g2), 0u, 0u);
-        uint4* o = reinterpret_cast<uint4*>(dout + (size_t)r * kSurOutRow);
-        o[0] = v;
-        const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-        o[1] = z;
-        o[2] = z;
-        o[3] = z;
-    }
-    const float tot = block_sum_256(l, red);
-    const float tc = block_sum_256(cnt, redc);
-    if (threadIdx.x == 0) {
-        loss_part[2 * blockIdx.x] = tot;
-        loss_part[2 * blockIdx.x + 1] = tc;
-    }
 }
 
 __global__ __launch_bounds__(256) void k_sur_targets(const float4* __restrict__ v0,
@@ -841,31 +1063,18 @@ hipError_t launch_sur_forward(bool integrate, const WalkBuffers& wb, const uint3
     return hipGetLastError();
 }
 
-hipError_t launch_sur_gemm(int epi, const __bf16* A, int lda, const __bf16* Bt, int ldb, int K,
-                           int N, uint32_t R, const SurEpiArgs& ep, hipStream_t st) {
-    if (R == 0) return hipSuccess;
-    const dim3 grid((R / 32u + 3u) / 4u), block(256);
-#define SUR_GEMM(E, NT) \
-    hipLaunchKernelGGL((k_sur_gemm<E, NT>), grid, block, 0, st, A, lda, Bt, ldb, K, R, ep)
-    switch (epi) {
-        case kEpiM: SUR_GEMM(kEpiM, 4); break;
-        case kEpiZ: SUR_GEMM(kEpiZ, 4); break;
-        case kEpiOut: SUR_GEMM(kEpiOut, 1); break;
-        case kEpiDZ: SUR_GEMM(kEpiDZ, 4); break;
-        case kEpiDM: SUR_GEMM(kEpiDM, 4); break;
-        default: SUR_GEMM(kEpiDS, 4); break;
-    }
-#undef SUR_GEMM
-    (void)N;
+hipError_t launch_sur_node_bwd(const float4* out, const uint32_t* rowslot, const uint32_t* sid,
+                               const float4* target, uint32_t R, const __bf16* Z,
+                               const __bf16* pk, float msg_scale, const SurGradRows& g,
+                               float* loss_part, hipStream_t st) {
+    hipLaunchKernelGGL(k_sur_node_bwd, dim3(sur_loss_parts(R)), dim3(64 * kNodeWaves), 0, st, out,
+                       rowslot, sid, target, R, Z, pk, msg_scale, g, loss_part);
     return hipGetLastError();
 }
 
-hipError_t launch_sur_wgrad(const __bf16* P, int ldp, int M, const __bf16* Q, int ldq, int N,
-                            uint32_t R, uint32_t rows_per_slab, uint32_t slabs, float* part,
-                            hipStream_t st) {
-    const int tiles = ((M + 31) / 32) * ((N + 31) / 32);
-    hipLaunchKernelGGL(k_sur_wgrad, dim3(tiles, slabs), dim3(64), 0, st, P, ldp, M, Q, ldq, N, R,
-                       rows_per_slab, part);
+hipError_t launch_sur_wgrad(const SurGradRows& g, const __bf16* S, const __bf16* X,
+                            const __bf16* Z, uint32_t R, const SurParts& parts, hipStream_t st) {
+    hipLaunchKernelGGL(k_sur_wgrad, dim3(sur_slabs(R), 3), dim3(256), 0, st, g, S, X, Z, R, parts);
     return hipGetLastError();
 }
 
@@ -880,23 +1089,21 @@ hipError_t launch_sur_edges_bwd(const WalkBuffers& wb, const uint32_t* batch, ui
     return hipGetLastError();
 }
 
-hipError_t launch_sur_reduce(const float* part, uint32_t slabs, int M_all, int ld, int M,
-                             int ncols, int bias_col, uint32_t dst, uint32_t bias_dst,
-                             float scale, float* grad, hipStream_t st) {
-    const int total = M * (ncols + (bias_col >= 0 ? 1 : 0));
-    hipLaunchKernelGGL(k_sur_reduce, dim3((total + 255) / 256), dim3(256), 0, st, part, slabs,
-                       M_all, ld, M, ncols, bias_col, dst, bias_dst, scale, grad);
-    return hipGetLastError();
-}
-
-hipError_t launch_sur_loss(const float* out, const uint32_t* rowslot, const uint32_t* sid,
-                           const float4* target, uint32_t R, __bf16* dout, float* loss_part,
-                           uint32_t* nparts, hipStream_t st) {
-    const uint32_t blocks = (R + 255u) / 256u;
-    *nparts = blocks;
-    if (blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_sur_loss, dim3(blocks), dim3(256), 0, st, out, rowslot, sid, target, R,
-                       2.0f, dout, loss_part);
+hipError_t launch_sur_reduce(const SurParts& parts, uint32_t R, uint32_t nbatch,
+                             const float* loss_part, float* grad, hipStream_t st) {
+    const uint32_t slabs = sur_slabs(R);
+    SurReduceTasks k;
+    k.t[0] = {parts.Wn1, slabs, 128, kSurRow, kSurNodeIn, kOffWn1, kOffBn1, 0};
+    k.t[1] = {parts.W2, slabs, 128, kSurRow, 128, kOffW2, kOffB2, 0};
+    k.t[2] = {parts.Wn2, slabs, 3, kSurRow, 128, kOffWn2, kOffBn2, 0};
+    k.t[3] = {parts.W1, nbatch, 128, 16, kSurNF, kOffW1, kOffB1, 0};
+    uint32_t wgs = 0;
+    for (auto& t : k.t) {
+        t.first = wgs;
+        wgs += t.rows * ((t.ncols + 16u) / 16u);
+    }
+    hipLaunchKernelGGL(k_sur_reduce, dim3(wgs), dim3(256), 0, st, k, loss_part, sur_loss_parts(R),
+                       grad);
     return hipGetLastError();
 }
 

@@ -60,8 +60,6 @@ void surrogate_free(SurrogateState* s) {
 
 namespace {
 
-constexpr uint32_t kRowsPerSlab = 1024;
-
 uint64_t splitmix64(uint64_t x) {
     uint64_t z = x + 0x9E3779B97F4A7C15ull;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -266,12 +264,25 @@ int loss_grad_batch(sphk_engine* e, SurrogateState* s, uint32_t nb, float* loss)
     HIP_TRY(launch_sur_forward(false, e->walk, s->d_batch, nb, 0, e->spm, e->svr, e->skey,
                                e->sid, e->cell_start, (uint32_t)e->n, e->consts, e->d_scenes,
                                s->pk, s->pf, sc, rows_of(s), SurStep{}, st));
-    // loss and its row gradients
-    const uint32_t blocks = (R + 255u) / 256u;
-    if (int rc = ensure_red(s, 2ull * blocks)) return rc;
-    uint32_t nparts = 0;
-    HIP_TRY(launch_sur_loss(s->OUT, s->rowslot, e->sid, s->target, R, s->DOUT, s->red, &nparts,
-                            st));
+    // loss, its row gradients and the node layers' backward pass, partials of the parameter
+    // gradients, and their sum in a fixed order
+    const uint32_t nparts = sur_loss_parts(R);
+    if (int rc = ensure_red(s, 2ull * nparts)) return rc;
+    const uint64_t slab = (uint64_t)sur_slabs(R) * kSurRow;
+    if (int rc = grow_buf(&s->part, s->part_cap, slab * (128 + 128 + 3) + (uint64_t)nb * 128 * 16))
+        return rc;
+    SurParts parts;
+    parts.Wn1 = s->part;
+    parts.W2 = parts.Wn1 + slab * 128;
+    parts.Wn2 = parts.W2 + slab * 128;
+    parts.W1 = parts.Wn2 + slab * 3;
+    const SurGradRows g = {s->DOUT, s->DZ, s->DM, s->DS};
+    HIP_TRY(launch_sur_node_bwd(reinterpret_cast<const float4*>(s->OUT), s->rowslot, e->sid,
+                                s->target, R, s->Z, s->pk, s->cfg.msg_scale, g, s->red, st));
+    HIP_TRY(launch_sur_wgrad(g, s->S, s->X, s->Z, R, parts, st));
+    HIP_TRY(launch_sur_edges_bwd(e->walk, s->d_batch, nb, e->spm, e->svr, e->skey, e->cell_start,
+                                 e->consts, e->d_scenes, s->pk, sc, s->DS, parts.W1, st));
+    HIP_TRY(launch_sur_reduce(parts, R, nb, s->red, s->grad, st));
     HIP_TRY(hipMemcpyAsync(s->h_red.data(), s->red, 2ull * nparts * sizeof(float),
                            hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
@@ -280,46 +291,7 @@ int loss_grad_batch(sphk_engine* e, SurrogateState* s, uint32_t nb, float* loss)
         sq += s->h_red[2 * b];
         rows += s->h_red[2 * b + 1];
     }
-    if (rows <= 0.0) {
-        HIP_TRY(hipMemsetAsync(s->grad, 0, kSurParams * sizeof(float), st));
-        *loss = 0.0f;
-        return SPHK_OK;
-    }
-    *loss = (float)(sq / (3.0 * rows));
-    const float gscale = (float)(1.0 / (3.0 * rows));
-    // backward through the node MLP and the hoisted message layer
-    SurEpiArgs ep{};
-    ep.out = s->DZ;
-    ep.z = s->Z;
-    HIP_TRY(launch_sur_gemm(kEpiDZ, s->DOUT, kSurOutRow, s->pk + kPkWn2T, 32, 32, 128, R, ep, st));
-    ep = SurEpiArgs{};
-    ep.out = s->DM;
-    HIP_TRY(launch_sur_gemm(kEpiDM, s->DZ, 128, s->pk + kPkWn1T, 128, 128, 128, R, ep, st));
-    ep = SurEpiArgs{};
-    ep.out = s->DS;
-    ep.scale = s->cfg.msg_scale;
-    HIP_TRY(launch_sur_gemm(kEpiDS, s->DM, 128, s->pk + kPkW2T, 128, 128, 128, R, ep, st));
-    // weight gradients (partials per slab of rows, then a fixed-order reduction)
-    const uint32_t slabs = (R + kRowsPerSlab - 1) / kRowsPerSlab;
-    const uint64_t need =
-        std::max<uint64_t>((uint64_t)slabs * 128 * kSurRow, 2ull * nb * 128 * 16);
-    if (int rc = grow_buf(&s->part, s->part_cap, need)) return rc;
-    HIP_TRY(launch_sur_wgrad(s->DOUT, kSurOutRow, 3, s->Z, kSurRow, 129, R, kRowsPerSlab, slabs,
-                             s->part, st));
-    HIP_TRY(launch_sur_reduce(s->part, slabs, 3, 129, 3, 128, 128, kOffWn2, kOffBn2, gscale,
-                              s->grad, st));
-    HIP_TRY(launch_sur_wgrad(s->DZ, 128, 128, s->X, kSurRow, kSurNodeIn + 1, R, kRowsPerSlab,
-                             slabs, s->part, st));
-    HIP_TRY(launch_sur_reduce(s->part, slabs, 128, kSurNodeIn + 1, 128, kSurNodeIn, kSurNodeIn,
-                              kOffWn1, kOffBn1, gscale, s->grad, st));
-    HIP_TRY(launch_sur_wgrad(s->DM, 128, 128, s->S, kSurRow, 129, R, kRowsPerSlab, slabs, s->part,
-                             st));
-    HIP_TRY(launch_sur_reduce(s->part, slabs, 128, 129, 128, 128, 128, kOffW2, kOffB2, gscale,
-                              s->grad, st));
-    HIP_TRY(launch_sur_edges_bwd(e->walk, s->d_batch, nb, e->spm, e->svr, e->skey, e->cell_start,
-                                 e->consts, e->d_scenes, s->pk, sc, s->DS, s->part, st));
-    HIP_TRY(launch_sur_reduce(s->part, 2u * nb, 128, 16, 128, kSurNF, kSurNF, kOffW1, kOffB1,
-                              gscale, s->grad, st));
+    *loss = rows > 0.0 ? (float)(sq / (3.0 * rows)) : 0.0f;
     return SPHK_OK;
 }
 

@@ -280,3 +280,30 @@ def test_trained_network_beats_the_method_without_it(sphk, scenes):
     print(f"judged run: true error {err_run:.3f} kg/m^3, bound {rep.error_bound:.3f}")
     assert rep.judges == 2 and rep.macro_steps == 6
     assert err_run <= rep.error_bound
+
+
+@pytest.mark.parametrize("batch_chunks", [1, 2, 7, 8, 9, 17])
+def test_gradient_of_ragged_batches(sphk, oracle, scenes, batch_chunks):
+    # The weight gradients are summed over slabs of 512 batch rows (eight chunks), each walked
+    # by four wavefronts in row parts: less than one part, one slab, one chunk beyond a slab.
+    # Tolerances of test_gradient_matches_oracle (bf16 operands, FP32 sums).
+    s = _moving_block(scenes, seed=6)
+    e = _engine(sphk, s)
+    e.surrogate_init(seed=4)
+    params = _active_params(e, seed=3)
+    target = np.random.default_rng(5).normal(0, 10, (s.n, 3)).astype(F32)
+    loss, grad, mask = e.surrogate_loss_grad(target, batch_seed=7, batch_chunks=batch_chunks)
+    assert 0 < mask.sum() <= batch_chunks * 64
+    rho = e.surrogate_densities()
+    offs, idx = e.neighbors()
+    cfg = _cfg(oracle, e)
+    lo, go = oracle.sur_loss_grad(cfg, params, e.positions(), e.velocities(), rho, offs, idx,
+                                  mask, target / cfg.acc_scale)
+    assert loss == pytest.approx(lo, rel=1e-4)
+    for name, a, b in BLOCKS:
+        x, y = grad[a:b].astype(np.float64), go[a:b]
+        rel = np.linalg.norm(x - y) / np.linalg.norm(y)
+        assert rel < 5e-3, (name, rel)
+    again = e.surrogate_loss_grad(target, batch_seed=7, batch_chunks=batch_chunks)
+    assert again[0] == loss
+    np.testing.assert_array_equal(again[1], grad)
