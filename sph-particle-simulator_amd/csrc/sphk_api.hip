@@ -182,6 +182,48 @@ int grid_for_ext(const SceneHost& sc, float radius, Grid* g) {
     return SPHK_OK;
 }
 
+// Folds the boxes of a workgroup's 256 threads into out[0, 7): min x, y, z, max x, y, z as
+// order-preserving uints, any.
+__device__ __forceinline__ void block_box(const float (&lo)[3], const float (&hi)[3], bool found,
+                                          uint32_t* __restrict__ out) {
+    auto ord = [](float f) {
+        unsigned b = __float_as_uint(f);
+        return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+    };
+    unsigned olo[3], ohi[3];
+    for (int d = 0; d < 3; ++d) {
+        olo[d] = ord(lo[d]);
+        ohi[d] = ord(hi[d]);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        for (int d = 0; d < 3; ++d) {
+            const unsigned a = __shfl_xor(olo[d], off), b = __shfl_xor(ohi[d], off);
+            olo[d] = a < olo[d] ? a : olo[d];
+            ohi[d] = b > ohi[d] ? b : ohi[d];
+        }
+    }
+    __shared__ unsigned red[4][7];
+    const unsigned wave = threadIdx.x >> 6;
+    const bool any = __ballot(found) != 0ull;
+    if ((threadIdx.x & 63u) == 0u) {
+        for (int d = 0; d < 3; ++d) {
+            red[wave][d] = olo[d];
+            red[wave][3 + d] = ohi[d];
+        }
+        red[wave][6] = any ? 1u : 0u;
+    }
+    __syncthreads();
+    if (threadIdx.x < 7u) {
+        const unsigned d = threadIdx.x;
+        unsigned v = red[0][d];
+        for (unsigned w = 1; w < 4u; ++w) {
+            const unsigned x = red[w][d];
+            v = d < 3u ? (x < v ? x : v) : d < 6u ? (x > v ? x : v) : (v | x);
+        }
+        out[d] = v;
+    }
+}
+
 // Bounding boxes of the scenes' finite positions, every scene in one launch: workgroup b of the
 // grid reduces part b % parts of scene b / parts and writes its box to out[7 b .. 7 b + 6] (min
 // x, y, z, max x, y, z as order-preserving uints, any); the host folds a scene's parts.  Bound
@@ -219,41 +261,76 @@ __global__ __launch_bounds__(256) void k_bbox(const float4* __restrict__ pm,
             }
         }
     }
-    auto ord = [](float f) {
-        unsigned b = __float_as_uint(f);
-        return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-    };
-    unsigned olo[3], ohi[3];
-    for (int d = 0; d < 3; ++d) {
-        olo[d] = ord(lo[d]);
-        ohi[d] = ord(hi[d]);
-    }
-    for (int off = 32; off > 0; off >>= 1) {
+    block_box(lo, hi, found, out + 7 * (size_t)blockIdx.x);
+}
+
+// Uploaded position rows (three floats each, `n` of them): per workgroup the box of the finite
+// ones and, in word 7, the first row whose cell index lies beyond +-2^30 (~0 if none), the
+// same test as floor_cell.  Bound by the read of the rows.
+__global__ __launch_bounds__(256) void k_upload_check(const float* __restrict__ rows, uint32_t n,
+                                                      float inv, uint32_t* __restrict__ out) {
+    float lo[3] = {INFINITY, INFINITY, INFINITY};
+    float hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    bool found = false;
+    uint32_t bad = ~0u;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+        const float p[3] = {rows[3 * (size_t)i], rows[3 * (size_t)i + 1], rows[3 * (size_t)i + 2]};
+        if (!__builtin_isfinite(p[0]) || !__builtin_isfinite(p[1]) || !__builtin_isfinite(p[2]))
+            continue;
+        found = true;
         for (int d = 0; d < 3; ++d) {
-            const unsigned a = __shfl_xor(olo[d], off), b = __shfl_xor(ohi[d], off);
-            olo[d] = a < olo[d] ? a : olo[d];
-            ohi[d] = b > ohi[d] ? b : ohi[d];
+            lo[d] = fminf(lo[d], p[d]);
+            hi[d] = fmaxf(hi[d], p[d]);
+            const float f = floorf(p[d] * inv);
+            if (!(f >= -1073741824.0f && f < 1073741824.0f)) bad = min(bad, i);
         }
     }
-    __shared__ unsigned red[4][7];
-    const unsigned wave = threadIdx.x >> 6;
-    const bool any = __ballot(found) != 0ull;
-    if ((threadIdx.x & 63u) == 0u) {
-        for (int d = 0; d < 3; ++d) {
-            red[wave][d] = olo[d];
-            red[wave][3 + d] = ohi[d];
-        }
-        red[wave][6] = any ? 1u : 0u;
+    __shared__ uint32_t first[4];
+    for (int off = 32; off > 0; off >>= 1) bad = min(bad, (uint32_t)__shfl_xor((int)bad, off));
+    if ((threadIdx.x & 63u) == 0u) first[threadIdx.x >> 6] = bad;
+    block_box(lo, hi, found, out + 8 * (size_t)blockIdx.x);
+    if (threadIdx.x == 0)
+        out[8 * (size_t)blockIdx.x + 7] = min(min(first[0], first[1]), min(first[2], first[3]));
+}
+
+// Home rows of uploaded particles: (x, y, z, m) and (vx, vy, vz, 0) from rows of three floats.
+__global__ __launch_bounds__(256) void k_upload_rows(const float* __restrict__ pos,
+                                                     const float* __restrict__ vel,
+                                                     const float* __restrict__ mass, float m,
+                                                     uint32_t n, float4* __restrict__ pm,
+                                                     float4* __restrict__ v) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const size_t k = 3 * (size_t)i;
+    pm[i] = make_float4(pos[k], pos[k + 1], pos[k + 2], mass ? mass[i] : m);
+    v[i] = vel ? make_float4(vel[k], vel[k + 1], vel[k + 2], 0.0f)
+               : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+// Floats [begin, begin + count) of a packed image of `src`: kComps floats of every row of kStride,
+// from float kOff on; begin a multiple of 4.  Written straight to host memory (dst: pinned), 16
+// bytes a lane; the grid flag of the state goes along.  Bound by the link to the host.
+template <uint32_t kComps, uint32_t kStride, uint32_t kOff>
+__global__ __launch_bounds__(256) void k_download_pack(const float* __restrict__ src,
+                                                       uint32_t begin, uint32_t count,
+                                                       float* __restrict__ dst,
+                                                       const uint32_t* __restrict__ flag,
+                                                       uint32_t* __restrict__ flag_out) {
+    const uint32_t k0 = 4u * (blockIdx.x * 256u + threadIdx.x);
+    if (k0 == 0u) *flag_out = *flag;
+    if (k0 >= count) return;
+    float v[4];
+#pragma unroll
+    for (uint32_t c = 0; c < 4u; ++c) {
+        // (lanes past the end repeat the last float)
+        const uint32_t k = begin + min(k0 + c, count - 1u);
+        const uint32_t row = k / kComps;
+        v[c] = src[(size_t)row * kStride + kOff + (k - row * kComps)];
     }
-    __syncthreads();
-    if (threadIdx.x < 7u) {
-        const unsigned d = threadIdx.x;
-        unsigned v = red[0][d];
-        for (unsigned w = 1; w < 4u; ++w) {
-            const unsigned x = red[w][d];
-            v = d < 3u ? (x < v ? x : v) : d < 6u ? (x > v ? x : v) : (v | x);
-        }
-        out[7 * (size_t)blockIdx.x + d] = v;
+    if (k0 + 4u <= count) {
+        *reinterpret_cast<float4*>(dst + k0) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+        for (uint32_t c = 0; k0 + c < count; ++c) dst[k0 + c] = v[c];
     }
 }
 
@@ -536,6 +613,54 @@ int drain_timing(sphk_engine* e) {
     }
     e->pending.clear();
     return SPHK_OK;
+}
+
+// Downloads floats [0, count) of a packed image of `src` (see k_download_pack) to pageable host
+// memory: the device writes a piece into one half of a pinned buffer while the host copies the
+// piece before it out of the other half.  A state with a raised grid flag is refused before
+// `out` is touched.  Copying 16-byte rows into a fresh host buffer and packing them there took
+// ~480 us for the positions of 177,000 particles, this ~150 (with the upload below, a frame
+// of upload, step and three downloads 2.42 -> 0.80 ms).
+constexpr size_t kStageFloats = 3u << 15;  // one half: 384 KiB
+
+template <uint32_t kComps, uint32_t kStride, uint32_t kOff>
+int download_packed(sphk_engine* e, const void* src, size_t count, float* out) {
+    if (!e->stage) {
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&e->stage),
+                              (2 * kStageFloats + 16) * sizeof(float), hipHostMallocDefault));
+    }
+    for (hipEvent_t& ev : e->stage_ev)
+        if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    uint32_t* flag = reinterpret_cast<uint32_t*>(e->stage + 2 * kStageFloats);
+    const size_t pieces = (count + kStageFloats - 1) / kStageFloats;
+    auto launch = [&](size_t p) -> int {
+        const uint32_t len = (uint32_t)std::min(kStageFloats, count - p * kStageFloats);
+        hipLaunchKernelGGL((k_download_pack<kComps, kStride, kOff>), dim3((len + 1023u) / 1024u),
+                           dim3(256), 0, e->stream, static_cast<const float*>(src),
+                           (uint32_t)(p * kStageFloats), len, e->stage + (p & 1) * kStageFloats, e->uscal,
+                           flag);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipEventRecord(e->stage_ev[p & 1], e->stream));
+        return SPHK_OK;
+    };
+    int rc = pieces ? launch(0) : check_grid_flag(e);
+    for (size_t p = 0; p < pieces && rc == SPHK_OK; ++p) {
+        if (p + 1 < pieces) rc = launch(p + 1);
+        if (rc) break;
+        HIP_TRY(hipEventSynchronize(e->stage_ev[p & 1]));
+        if (p == 0 && *flag) break;
+        const size_t b = p * kStageFloats;
+        memcpy(out + b, e->stage + (p & 1) * kStageFloats,
+               std::min(kStageFloats, count - b) * sizeof(float));
+    }
+    if (rc == SPHK_OK && pieces && *flag) rc = check_grid_flag(e);
+    return rc;
+}
+
+// A download into too small a buffer: a raised grid flag is the graver error.
+int refused_download(sphk_engine* e, size_t need) {
+    if (int rc = check_grid_flag(e)) return rc;
+    return set_error(SPHK_E_INVALID, "need %zu floats", need);
 }
 
 int check_engine(const sphk_engine* e) {
@@ -833,6 +958,9 @@ int sphk_destroy(sphk_engine* e) {
                     (void*)e->walk.part_force, (void*)e->scan_scratch, (void*)e->d_scenes,
                     (void*)e->lookback, (void*)e->bbox_ranges, (void*)e->bbox_out})
         if (p) (void)hipFree(p);
+    if (e->stage) (void)hipHostFree(e->stage);
+    for (hipEvent_t ev : e->stage_ev)
+        if (ev) (void)hipEventDestroy(ev);
     if (e->sur) surrogate_free(e->sur);
     if (e->graph_exec) (void)hipGraphExecDestroy(e->graph_exec);
     for (auto* v : {&e->pending, &e->free_sets})
@@ -876,29 +1004,59 @@ int sphk_upload(sphk_engine* e, size_t offset, size_t n, const float* pos, const
     if (offset > e->n) return set_error(SPHK_E_INVALID, "offset %zu beyond count %zu", offset, e->n);
     if (n && !pos) return set_error(SPHK_E_INVALID, "null positions");
     if (int rc = set_device(e)) return rc;
-    size_t fit = std::min(n, e->cap - offset);
-    std::vector<float4> hp(fit), hv(fit);
-    const float inv = 1.0f / e->params.neighbor_search_radius;
-    for (size_t i = 0; i < fit; ++i) {
-        float x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
-        float m = mass ? mass[i] : e->params.particle_mass;
-        hp[i] = make_float4(x, y, z, m);
-        hv[i] = vel ? make_float4(vel[3 * i], vel[3 * i + 1], vel[3 * i + 2], 0.0f)
-                    : make_float4(0.f, 0.f, 0.f, 0.f);
-        if (std::isfinite(x) && std::isfinite(y) && std::isfinite(z)) {
-            int64_t cc;
-            if (floor_cell(x, inv, &cc) || floor_cell(y, inv, &cc) || floor_cell(z, inv, &cc))
-                return set_error(SPHK_E_DOMAIN,
-                                 "particle %zu at (%g, %g, %g) needs a cell index beyond +-2^30",
-                                 offset + i, (double)x, (double)y, (double)z);
-        }
-    }
+    // The rows go up as they are, into the sorted arrays (work memory of a build, one row
+    // more than the capacity, the last untouched), and are checked and spread to the home
+    // arrays there: 177,000 particles ~150 us; the same loops and 16-byte rows on the host took
+    // most of a millisecond.
+    const size_t fit = std::min(n, e->cap - offset);
+    float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+    bool any = false;
     if (fit) {
-        HIP_TRY(hipMemcpyAsync(e->pm + offset, hp.data(), fit * sizeof(float4),
-                               hipMemcpyHostToDevice, e->stream));
-        HIP_TRY(hipMemcpyAsync(e->vel + offset, hv.data(), fit * sizeof(float4),
-                               hipMemcpyHostToDevice, e->stream));
+        const float inv = 1.0f / e->params.neighbor_search_radius;
+        float* const dpos = reinterpret_cast<float*>(e->spm);
+        float* const dvel = reinterpret_cast<float*>(e->svr);
+        float* const dmass = reinterpret_cast<float*>(e->frows);
+        const uint32_t blocks = (uint32_t)std::min<size_t>((fit + 255) / 256, 256);
+        uint64_t unused = 0;  // no captured step reads this buffer
+        if (int rc = grow(&e->bbox_out, e->bbox_out_cap, 8 * (uint64_t)blocks, unused)) return rc;
+        e->sorted_valid = false;
+        HIP_TRY(hipMemcpyAsync(dpos, pos, 3 * fit * sizeof(float), hipMemcpyHostToDevice,
+                               e->stream));
+        hipLaunchKernelGGL(k_upload_check, dim3(blocks), dim3(256), 0, e->stream, dpos,
+                           (uint32_t)fit, inv, e->bbox_out);
+        HIP_TRY(hipGetLastError());
+        if (vel)
+            HIP_TRY(hipMemcpyAsync(dvel, vel, 3 * fit * sizeof(float), hipMemcpyHostToDevice,
+                                   e->stream));
+        if (mass)
+            HIP_TRY(hipMemcpyAsync(dmass, mass, fit * sizeof(float), hipMemcpyHostToDevice,
+                                   e->stream));
+        std::vector<uint32_t> box(8 * blocks);
+        HIP_TRY(hipMemcpyAsync(box.data(), e->bbox_out, box.size() * 4, hipMemcpyDeviceToHost,
+                               e->stream));
         HIP_TRY(hipStreamSynchronize(e->stream));
+        uint32_t bad = ~0u;
+        for (uint32_t b = 0; b < blocks; ++b) {
+            const uint32_t* o = box.data() + 8 * b;
+            bad = std::min(bad, o[7]);
+            if (!o[6]) continue;
+            for (int d = 0; d < 3; ++d) {
+                const float l = unord(o[d]), h = unord(o[3 + d]);
+                lo[d] = any ? std::min(lo[d], l) : l;
+                hi[d] = any ? std::max(hi[d], h) : h;
+            }
+            any = true;
+        }
+        if (bad != ~0u)
+            return set_error(SPHK_E_DOMAIN,
+                             "particle %zu at (%g, %g, %g) needs a cell index beyond +-2^30",
+                             offset + bad, (double)pos[3 * (size_t)bad],
+                             (double)pos[3 * (size_t)bad + 1], (double)pos[3 * (size_t)bad + 2]);
+        hipLaunchKernelGGL(k_upload_rows, dim3((uint32_t)((fit + 255) / 256)), dim3(256), 0,
+                           e->stream, dpos, vel ? dvel : nullptr, mass ? dmass : nullptr,
+                           e->params.particle_mass, (uint32_t)fit, e->pm + offset,
+                           e->vel + offset);
+        HIP_TRY(hipGetLastError());
     }
     e->n = offset + fit;
     if (!e->scenes_explicit) {
@@ -906,20 +1064,6 @@ int sphk_upload(sphk_engine* e, size_t offset, size_t n, const float* pos, const
         e->scenes.resize(1);
         SceneHost& sc = e->scenes[0];
         if (offset == 0) sc.ext_any = false;
-        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-        bool any = false;
-        for (size_t i = 0; i < fit; ++i) {
-            const float4& q = hp[i];
-            if (std::isfinite(q.x) && std::isfinite(q.y) && std::isfinite(q.z)) {
-                lo[0] = std::min(lo[0], q.x);
-                lo[1] = std::min(lo[1], q.y);
-                lo[2] = std::min(lo[2], q.z);
-                hi[0] = std::max(hi[0], q.x);
-                hi[1] = std::max(hi[1], q.y);
-                hi[2] = std::max(hi[2], q.z);
-                any = true;
-            }
-        }
         if (any) ext_add_box(sc, lo, hi);
         if (offset == 0) e->ext_unknown = false;
     } else {
@@ -1058,45 +1202,26 @@ int sphk_download(sphk_engine* e, int which, float* out, size_t count) {
     if (int rc = check_engine(e)) return rc;
     if (!out && count) return set_error(SPHK_E_INVALID, "null output");
     if (int rc = set_device(e)) return rc;
-    if (int rc = check_grid_flag(e)) return rc;
     const size_t n = e->n;
     switch (which) {
         case SPHK_POSITIONS:
         case SPHK_VELOCITIES:
         case SPHK_ACCELERATIONS: {
-            if (count < n * 3) return set_error(SPHK_E_INVALID, "need %zu floats", n * 3);
+            if (count < n * 3) return refused_download(e, n * 3);
             const float4* src = which == SPHK_POSITIONS ? e->pm
                                 : which == SPHK_VELOCITIES ? e->vel
                                                            : e->acc;
-            std::vector<float4> tmp(n);
-            if (n) HIP_TRY(hipMemcpyAsync(tmp.data(), src, n * sizeof(float4), hipMemcpyDeviceToHost,
-                                          e->stream));
-            HIP_TRY(hipStreamSynchronize(e->stream));
-            for (size_t i = 0; i < n; ++i) {
-                out[3 * i] = tmp[i].x;
-                out[3 * i + 1] = tmp[i].y;
-                out[3 * i + 2] = tmp[i].z;
-            }
-            return SPHK_OK;
+            return download_packed<3, 4, 0>(e, src, n * 3, out);
         }
-        case SPHK_MASSES: {
-            if (count < n) return set_error(SPHK_E_INVALID, "need %zu floats", n);
-            std::vector<float4> tmp(n);
-            if (n) HIP_TRY(hipMemcpyAsync(tmp.data(), e->pm, n * sizeof(float4), hipMemcpyDeviceToHost,
-                                          e->stream));
-            HIP_TRY(hipStreamSynchronize(e->stream));
-            for (size_t i = 0; i < n; ++i) out[i] = tmp[i].w;
-            return SPHK_OK;
-        }
+        case SPHK_MASSES:
+            if (count < n) return refused_download(e, n);
+            return download_packed<1, 4, 3>(e, e->pm, n, out);
         case SPHK_DENSITIES:
-        case SPHK_PRESSURES: {
-            size_t m = std::min(count, e->cap);
-            HIP_TRY(hipMemcpyAsync(out, which == SPHK_DENSITIES ? e->rho : e->prs, m * sizeof(float),
-                                   hipMemcpyDeviceToHost, e->stream));
-            HIP_TRY(hipStreamSynchronize(e->stream));
-            return SPHK_OK;
-        }
+        case SPHK_PRESSURES:
+            return download_packed<1, 1, 0>(e, which == SPHK_DENSITIES ? e->rho : e->prs,
+                                            std::min(count, e->cap), out);
         default:
+            if (int rc = check_grid_flag(e)) return rc;
             return set_error(SPHK_E_INVALID, "unknown download selector %d", which);
     }
 }

@@ -133,6 +133,9 @@ struct sphk_engine {
     std::vector<uint32_t> bbox_uploaded;
     uint32_t* bbox_out = nullptr;
     uint64_t bbox_out_cap = 0;
+    // downloads: pinned memory of two pieces and the grid flag, an event per piece
+    float* stage = nullptr;
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
     StepConsts consts{};
     bool sorted_valid = false;  // work arrays hold the cell-sorted image of the current state
     uint64_t buffer_gen = 0;    // bumped when a buffer used by the step is reallocated

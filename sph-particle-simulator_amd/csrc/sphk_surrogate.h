@@ -149,6 +149,15 @@ hipError_t launch_sur_edges_bwd(const WalkBuffers& wb, const uint32_t* batch, ui
 hipError_t launch_sur_reduce(const SurParts& parts, uint32_t R, uint32_t nbatch,
                              const float* loss_part, float* grad, hipStream_t st);
 
+// dst[i] = (scale * rows[3 i .. 3 i + 2], 0).
+hipError_t launch_sur_scale_rows(const float* rows, uint32_t n, float scale, float4* dst,
+                                 hipStream_t st);
+
+// mask[id] = 1 for the particles of R batch rows, 0 for the other of the n (mask: room for a
+// multiple of 4 bytes).
+hipError_t launch_sur_mask(const uint32_t* rowslot, uint32_t R, const uint32_t* sid, uint32_t n,
+                           uint8_t* mask, hipStream_t st);
+
 // Targets (normalised): t[id] = (v4 - d^k v0) / (T a_s).
 hipError_t launch_sur_targets(const float4* v0, const float4* v4, uint32_t n, float dk,
                               float inv_Tas, float4* target, hipStream_t st);

@@ -924,6 +924,24 @@ __global__ __launch_bounds__(256) void k_sur_targets(const float4* __restrict__ 
                             (b.z - dk * a.z) * inv_Tas, 0.0f);
 }
 
+__global__ __launch_bounds__(256) void k_sur_scale_rows(const float* __restrict__ rows,
+                                                        uint32_t n, float scale,
+                                                        float4* __restrict__ dst) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const float* r = rows + 3 * (size_t)i;
+    dst[i] = make_float4(r[0] * scale, r[1] * scale, r[2] * scale, 0.0f);
+}
+
+__global__ __launch_bounds__(256) void k_sur_mask(const uint32_t* __restrict__ rowslot,
+                                                  uint32_t R, const uint32_t* __restrict__ sid,
+                                                  uint8_t* __restrict__ mask) {
+    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
+    if (r >= R) return;
+    const uint32_t slot = rowslot[r];
+    if (slot != kSurNoSlot) mask[sid[slot]] = 1;
+}
+
 // Particles with a non-finite coordinate (dense index G) have no neighbours: free fall over
 // the macro-step, as in the plain step.
 __global__ __launch_bounds__(256) void k_sur_nonfinite(const float4* __restrict__ spm,
@@ -1104,6 +1122,22 @@ hipError_t launch_sur_reduce(const SurParts& parts, uint32_t R, uint32_t nbatch,
     }
     hipLaunchKernelGGL(k_sur_reduce, dim3(wgs), dim3(256), 0, st, k, loss_part, sur_loss_parts(R),
                        grad);
+    return hipGetLastError();
+}
+
+hipError_t launch_sur_scale_rows(const float* rows, uint32_t n, float scale, float4* dst,
+                                 hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_sur_scale_rows, dim3((n + 255) / 256), dim3(256), 0, st, rows, n, scale,
+                       dst);
+    return hipGetLastError();
+}
+
+hipError_t launch_sur_mask(const uint32_t* rowslot, uint32_t R, const uint32_t* sid, uint32_t n,
+                           uint8_t* mask, hipStream_t st) {
+    hipError_t e = launch_fill_u32(reinterpret_cast<uint32_t*>(mask), 0u, (n + 3u) / 4u, st);
+    if (e != hipSuccess || R == 0) return e;
+    hipLaunchKernelGGL(k_sur_mask, dim3((R + 255) / 256), dim3(256), 0, st, rowslot, R, sid, mask);
     return hipGetLastError();
 }
 

@@ -559,28 +559,26 @@ int sphk_surrogate_loss_grad(sphk_engine* e, const float* target, size_t count,
         return set_error(SPHK_E_INVALID, "need %u gradient floats", kSurParams);
     if (e->n == 0) return set_error(SPHK_E_INVALID, "no particles");
     if (int rc = ensure_particles(s, e->n)) return rc;
-    std::vector<float4> h(e->n);
-    const float inv = 1.0f / s->cfg.acc_scale;
-    for (size_t i = 0; i < e->n; ++i)
-        h[i] = make_float4(target[3 * i] * inv, target[3 * i + 1] * inv, target[3 * i + 2] * inv,
-                           0.0f);
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    HIP_TRY(hipMemcpy(s->target, h.data(), e->n * sizeof(float4), hipMemcpyHostToDevice));
+    // the rows go up as they are, into a work array of the build below, and are scaled there
+    const uint32_t n = (uint32_t)e->n;
+    float* const rows = reinterpret_cast<float*>(e->spm);
+    e->sorted_valid = false;
+    HIP_TRY(hipMemcpyAsync(rows, target, 3 * e->n * sizeof(float), hipMemcpyHostToDevice,
+                           e->stream));
+    HIP_TRY(launch_sur_scale_rows(rows, n, 1.0f / s->cfg.acc_scale, s->target, e->stream));
     if (int rc = prepare_density(e)) return rc;
     uint32_t nb = 0;
     if (int rc = choose_batch(e, s, batch_seed, batch_chunks, &nb)) return rc;
+    // the batch's particles are marked on the device and come back with the gradient
+    uint8_t* const mask = reinterpret_cast<uint8_t*>(s->rho_a);
     if (int rc = loss_grad_batch(e, s, nb, loss)) return rc;
+    if (in_batch) HIP_TRY(launch_sur_mask(s->rowslot, 64u * nb, e->sid, n, mask, e->stream));
+    if (grad)
+        HIP_TRY(hipMemcpyAsync(grad, s->grad, kSurParams * sizeof(float), hipMemcpyDeviceToHost,
+                               e->stream));
+    if (in_batch)
+        HIP_TRY(hipMemcpyAsync(in_batch, mask, e->n, hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
-    if (grad) HIP_TRY(hipMemcpy(grad, s->grad, kSurParams * sizeof(float), hipMemcpyDeviceToHost));
-    if (in_batch) {
-        memset(in_batch, 0, e->n);
-        const uint64_t R = 64ull * nb;
-        std::vector<uint32_t> slots(R), sid(e->n);
-        if (R) HIP_TRY(hipMemcpy(slots.data(), s->rowslot, R * 4, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(sid.data(), e->sid, e->n * 4, hipMemcpyDeviceToHost));
-        for (uint64_t r = 0; r < R; ++r)
-            if (slots[r] != kSurNoSlot) in_batch[sid[slots[r]]] = 1;
-    }
     return SPHK_OK;
 }
 

@@ -37,3 +37,34 @@ def test_scene_extents_measured_on_the_device(sphk, sizes):
         one.upload(pos[a:b])
         one.step(1e-4)
         np.testing.assert_array_equal(got[a:b], one.positions())
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 32767, 32768, 32769, 70000])
+def test_uploads_and_downloads_return_the_rows(sphk, n):
+    # Rows go up and come back through work arrays and two pinned halves of 32,768 rows: every
+    # read-back returns the uploaded bits, non-finite ones included, also after a second
+    # upload behind the first, and a refused upload leaves the state as it was.
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    vel = rng.normal(0, 1, (n, 3)).astype(np.float32)
+    mass = rng.uniform(1, 2, n).astype(np.float32)
+    pos[n // 2, 1] = np.nan
+    pos[n - 1, 2] = -np.inf
+    e = sphk.Engine(n + 300, sphk.default_params())
+    e.upload(pos, vel, mass)
+    far = pos[:1].repeat(300, 0)
+    far[:] = 0.25
+    far[7] = far[11] = 1e9
+    with pytest.raises(sphk.SphkError, match=f"particle {n + 7} "):
+        e.upload(far, offset=n)
+    assert e.size() == n
+    np.testing.assert_array_equal(e.positions(), pos)
+    np.testing.assert_array_equal(e.velocities(), vel)
+    np.testing.assert_array_equal(e.masses(), mass)
+    e.upload(pos[:300], offset=n)  # no velocities, default mass
+    m = min(n, 300)
+    np.testing.assert_array_equal(e.positions(), np.concatenate([pos, pos[:m]]))
+    np.testing.assert_array_equal(e.velocities()[n:], np.zeros((m, 3), np.float32))
+    np.testing.assert_array_equal(e.masses()[n:],
+                                  np.full(m, sphk.default_params().particle_mass, np.float32))
+    assert e.densities().shape == (n + 300,)
