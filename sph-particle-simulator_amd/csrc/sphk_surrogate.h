@@ -69,7 +69,7 @@ constexpr uint32_t kFTotal = kFBn2 + 4;
 
 // Feature and output scales (see the network above).
 struct SurScales {
-    float inv_r, inv_v, inv_h, w_norm;
+    float inv_r, inv_v, inv_h;
     float rho0, rho_scale, msg_scale, acc_scale;
 };
 

@@ -41,23 +41,33 @@ __device__ __forceinline__ uint32_t acc_row(int v, uint32_t h) {
     return (uint32_t)((v >> 2) * 8 + (v & 3)) + 4u * h;
 }
 
-// Cubic-spline shape in the operation order of the oracle (no contraction).
-__device__ __forceinline__ float w_shape_ieee(float q) {
+// W(|r|) / W(0) of the cubic spline.  kOrdered: in the operation order of the oracle (no
+// contraction).  Otherwise by clamped cubes, 2 (u^3 - s^3 / 2) with u = max(1 - q / 2, 0) and
+// s = max(1 - q, 0) (the density walk's form: 8 operations, no select, against 13; each bracket of
+// the piecewise form is this polynomial, to FP32 rounding).
+template <bool kOrdered>
+__device__ __forceinline__ float w_feature(float r, float inv_h) {
 #pragma clang fp contract(off)
-    const float q2 = q * q;
-    const float win = (2.0f / 3.0f - q2) + 0.5f * q2 * q;
-    const float t = 2.0f - q;
-    const float wout = (1.0f / 6.0f) * t * t * t;
-    return q <= 1.0f ? win : (q <= 2.0f ? wout : 0.0f);
+    if (kOrdered) {
+        const float q = r * inv_h;
+        const float q2 = q * q;
+        const float win = (2.0f / 3.0f - q2) + 0.5f * q2 * q;
+        const float t = 2.0f - q;
+        const float wout = (1.0f / 6.0f) * t * t * t;
+        return 1.5f * (q <= 1.0f ? win : (q <= 2.0f ? wout : 0.0f));
+    }
+    const float u = __builtin_amdgcn_fmed3f(__builtin_fmaf(-0.5f * inv_h, r, 1.0f), 0.0f, 1.0f);
+    const float s = __builtin_amdgcn_fmed3f(__builtin_fmaf(-inv_h, r, 1.0f), 0.0f, 1.0f);
+    return 2.0f * __builtin_fmaf(s * s, -0.5f * s, u * u * u);
 }
 
 // Edge features of one pair in FP32 (any values for a non-edge: the caller zeroes them).
+template <bool kOrdered>
 __device__ __forceinline__ void edge_values(float4 pi, float4 vi, float4 pj, float4 vj,
                                             float d2, const SurScales& sc, float (&f)[9]) {
 #pragma clang fp contract(off)
     const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
     const float rl = __builtin_amdgcn_sqrtf(d2);
-    const float w = w_shape_ieee(rl * sc.inv_h);
     f[0] = rx * sc.inv_r;
     f[1] = ry * sc.inv_r;
     f[2] = rz * sc.inv_r;
@@ -65,7 +75,7 @@ __device__ __forceinline__ void edge_values(float4 pi, float4 vi, float4 pj, flo
     f[4] = (vi.y - vj.y) * sc.inv_v;
     f[5] = (vi.z - vj.z) * sc.inv_v;
     f[6] = rl * sc.inv_r;
-    f[7] = w * sc.w_norm;
+    f[7] = w_feature<kOrdered>(rl, sc.inv_h);
     f[8] = (vj.w - sc.rho0) * sc.rho_scale;
 }
 
@@ -73,23 +83,21 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // Edge features of one pair rounded to bf16 (round to nearest even, two per conversion),
-// zero when `edge` is false: features 0..7 as one operand vector, feature 8 (neighbour
-// density) apart.
+// zero when `edge` is false: features 0..7, and [1, feature 8] (neighbour density) packed.
+template <bool kOrdered>
 __device__ __forceinline__ void edge_features(bool edge, float4 pi, float4 vi, float4 pj,
                                               float4 vj, float d2, const SurScales& sc,
-                                              bf16x8& e, __bf16& e8) {
+                                              uint32_t (&e)[4], uint32_t& ext) {
     float f[9];
-    edge_values(pi, vi, pj, vj, d2, sc, f);
-    uint4 w;
-    uint32_t* wp = &w.x;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const f32x2 v = {f[2 * k], f[2 * k + 1]};
+    edge_values<kOrdered>(pi, vi, pj, vj, d2, sc, f);
+    auto pack = [&](float a, float b) {
+        const f32x2 v = {a, b};
         const uint32_t bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-        wp[k] = edge ? bits : 0u;
-    }
-    e = __builtin_bit_cast(bf16x8, w);
-    e8 = edge ? (__bf16)f[8] : (__bf16)0.0f;
+        return edge ? bits : 0u;
+    };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) e[k] = pack(f[2 * k], f[2 * k + 1]);
+    ext = pack(1.0f, f[8]);
 }
 
 __device__ __forceinline__ uint32_t bits16(__bf16 x) {
@@ -97,16 +105,13 @@ __device__ __forceinline__ uint32_t bits16(__bf16 x) {
 }
 
 // B operands of message layer 1 for hidden tile hb (n = 32 hb + l % 32).  The K range of an
-// MFMA is 16: one half of the lanes supplies W1 columns 0..7, the other half [b1, W1 column 8]
-// (k = 8, 9 for block 0; k = 0, 1 for block 1), so W1 e + b1 is one product.
-struct Layer1B {
-    bf16x8 blk0[4], blk1[4];
-};
-
+// MFMA is 16: the lower lanes supply W1 columns 0..7, the upper ones [b1, W1 column 8, 0 ...]
+// (k = 8, 9), so W1 e + b1 is one product.  kSwapped: the two halves of K the other way round.
+template <bool kSwapped = false>
 __device__ __forceinline__ void load_layer1(const __bf16* __restrict__ pk, uint32_t lane,
-                                            Layer1B& B) {
+                                            bf16x8 (&B)[4]) {
     const uint32_t col = lane & 31u;
-    const bool hi = lane >= 32u;
+    const bool hi = kSwapped ? lane < 32u : lane >= 32u;
 #pragma unroll
     for (int hb = 0; hb < 4; ++hb) {
         const uint32_t n = 32u * hb + col;
@@ -114,25 +119,30 @@ __device__ __forceinline__ void load_layer1(const __bf16* __restrict__ pk, uint3
         bf16x8 b = zero8();
         b[0] = pk[kPkB1 + n];
         b[1] = pk[kPkW1r + n];
-        B.blk0[hb] = hi ? b : w;
-        B.blk1[hb] = hi ? w : b;
+        B[hb] = hi ? b : w;
     }
 }
 
-// A operands: row r of block b is the edge of lane 32 b + r.  Its owner supplies features
-// 0..7; the partner lane (l ^ 32) supplies [1, feature 8] (zeros for a padding row, which is
-// then exactly zero).
-__device__ __forceinline__ void layer1_a(bf16x8 fe, __bf16 e8, bool edge, uint32_t lane,
-                                         bf16x8& a0, bf16x8& a1) {
-    const unsigned long long bal = __ballot(edge);
-    const bool pv = ((bal >> (lane ^ 32u)) & 1ull) != 0ull;
-    const uint32_t e8p = (uint32_t)__shfl_xor((int)bits16(e8), 32);
-    bf16x8 other = zero8();
-    other[0] = (__bf16)(pv ? 1.0f : 0.0f);
-    other[1] = __builtin_bit_cast(__bf16, (uint16_t)e8p);
-    const bool hi = lane >= 32u;
-    a0 = hi ? other : fe;
-    a1 = hi ? fe : other;
+// A operands: row r of block b is the edge of lane 32 b + r, its features 0..7 in the lower
+// lanes (k = 0..7) and [1, feature 8, 0 ...] in the upper ones (zeros for a padding row, which is
+// then exactly zero).  One v_permlane32_swap per dword trades the upper lanes' features for
+// the lower lanes' tail, which is both operands at once.  kSwapped: block 1 has the halves of
+// K the other way round (from a second swap), for B operands loaded so.
+template <bool kSwapped>
+__device__ __forceinline__ void layer1_a(const uint32_t (&e)[4], uint32_t ext, bf16x8& a0,
+                                         bf16x8& a1) {
+    uint4 x, y;
+    uint32_t* xp = &x.x;
+    uint32_t* yp = &y.x;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t t = k == 0 ? ext : 0u;
+        const auto r = __builtin_amdgcn_permlane32_swap(e[k], t, false, false);
+        xp[k] = r[0];
+        yp[k] = kSwapped ? __builtin_amdgcn_permlane32_swap(t, e[k], false, false)[1] : r[1];
+    }
+    a0 = __builtin_bit_cast(bf16x8, x);
+    a1 = __builtin_bit_cast(bf16x8, y);
 }
 
 typedef short short2v __attribute__((ext_vector_type(2)));
@@ -254,6 +264,13 @@ __global__ __launch_bounds__(256) void k_sur_pack(const float* __restrict__ p,
 // kIntegrate: the macro-step is applied and written to the caller-order state.  Otherwise
 // the S, X, Z and OUT rows are written for the backward pass (batch: rows 64 b + lane;
 // no batch: rows = sorted slots).
+// Bound by VALU issue (two wavefronts per SIMD, 204 operations beside the 8 products of a step
+// of 64 edges, 128 of them the sums of |u|).  The inference walk takes what is cheapest: long
+// windows, the operands of both blocks from one swap, the shape by clamped cubes, and the
+// sums of a product under the next product.  The rows for the backward pass keep the order of
+// edges, products and sums they have always had: a sum rounded another way flips some of the
+// bf16 roundings behind it (gradients then move by up to 1e-3 of their largest).
+// Macro-step of 295,000 particles 759 -> 664 us.
 // ---------------------------------------------------------------------------
 template <bool kIntegrate>
 __global__ __launch_bounds__(64 * kEdgeWaves) __attribute__((amdgpu_waves_per_eu(2))) void
@@ -282,58 +299,69 @@ k_sur_forward(WalkBuffers wb, const uint32_t* __restrict__ batch, uint32_t nbatc
                     pi))
         return;
     const float4 vi = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    Layer1B B;
+    constexpr bool kOrdered = !kIntegrate;
+    bf16x8 B[4], B1[4];
     load_layer1(pk, lane, B);
+    if constexpr (kOrdered) load_layer1<true>(pk, lane, B1);
     f32x16 acc[4];
 #pragma unroll
     for (int hb = 0; hb < 4; ++hb) acc[hb] = zero16();
-    float se[9];
+    // sum_j (e_ij, 1) of this lane's edges, of the values the layer-1 product sees (sum u is
+    // subtracted from sum |u| for hidden units that are mostly inactive).  On the VALU: an MFMA
+    // against a unit matrix was 2 % faster here, but its accumulation rounds less exactly
+    // (gradients 4e-4 off instead of 3e-7).
+    float se[10];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) se[k] = 0.0f;
-    float ne = 0.0f;
-    walk_pairs(item, ch, s, active, pi, clane, wb, spm, svr, cs, c, L, lane,
+    for (int k = 0; k < 10; ++k) se[k] = 0.0f;
+    walk_pairs<kIntegrate>(item, ch, s, active, pi, clane, wb, spm, svr, cs, c, L, lane,
                [&](bool edge, float4 pj, float4 vj, float d2) {
-                   bf16x8 fe;
-                   __bf16 e8;
-                   edge_features(edge, pi, vi, pj, vj, d2, sc, fe, e8);
-                   // the sums must see the values the MFMA sees (sum u is subtracted from
-                   // sum |u| for hidden units that are mostly inactive)
+                   uint32_t fe[4], ext;
+                   edge_features<kOrdered>(edge, pi, vi, pj, vj, d2, sc, fe, ext);
+                   bf16x8 a[2];
+                   layer1_a<kOrdered>(fe, ext, a[0], a[1]);
 #pragma unroll
-                   for (int k = 0; k < 8; ++k) se[k] += (float)fe[k];
-                   se[8] += (float)e8;
-                   ne += edge ? 1.0f : 0.0f;
-                   bf16x8 a0, a1;
-                   layer1_a(fe, e8, edge, lane, a0, a1);
+                   for (int k = 0; k < 5; ++k) {
+                       const uint32_t w = k < 4 ? fe[k] : ext;
+                       se[2 * k] += __uint_as_float(w << 16);
+                       se[2 * k + 1] += __uint_as_float(w & 0xffff0000u);
+                   }
+                   if constexpr (kOrdered) {
 #pragma unroll
-                   for (int hb = 0; hb < 4; ++hb) {
-                       const f32x16 d0 = mfma16(a0, B.blk0[hb], zero16());
-                       const f32x16 d1 = mfma16(a1, B.blk1[hb], zero16());
+                       for (int hb = 0; hb < 4; ++hb) {
+                           const f32x16 d0 = mfma16(a[0], B[hb], zero16());
+                           const f32x16 d1 = mfma16(a[1], B1[hb], zero16());
 #pragma unroll
-                       for (int v = 0; v < 16; ++v) acc[hb][v] += fabsf(d0[v]) + fabsf(d1[v]);
+                           for (int v = 0; v < 16; ++v) acc[hb][v] += fabsf(d0[v]) + fabsf(d1[v]);
+                       }
+                   } else {
+                       f32x16 d[2];
+                       d[0] = mfma16(a[0], B[0], zero16());
+#pragma unroll
+                       for (int k = 0; k < 8; ++k) {
+                           const int n = k + 1;
+                           if (n < 8) d[n & 1] = mfma16(a[n & 1], B[n >> 1], zero16());
+                           __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                           for (int v = 0; v < 16; ++v) acc[k >> 1][v] += fabsf(d[k & 1][v]);
+                           __builtin_amdgcn_sched_barrier(0);
+                       }
                    }
                });
-    // both lanes of a target hold half of its sums
-#pragma unroll
-    for (int k = 0; k < 9; ++k) se[k] += __shfl_xor(se[k], 32);
-    ne += __shfl_xor(ne, 32);
-    float* lcnt = lcnt_all[half];
-    if (h == 0u) lcnt[col] = ne;
     // sum u + sum |u| = [sum e, n] W1aug^T + acc, on MFMA with the accumulators as C.  The
     // sums enter as three bf16 parts (x = x0 + x1 + x2 to about 2^-27 relative): sum u is
     // cancelled against sum |u| for hidden units that are mostly inactive.
+    // both lanes of a target hold half of its sums: 0..7, n, 8
+#pragma unroll
+    for (int k = 0; k < 10; ++k) se[k] += __shfl_xor(se[k], 32);
+    const float ne = se[8];
+    float* lcnt = lcnt_all[half];
+    if (h == 0u) lcnt[col] = ne;
     {
         // lanes 0..31 supply k = 0..7 (feature sums 0..7), lanes 32..63 k = 8, 9 (the edge
         // count, which meets b1, and feature sum 8, which meets W1 column 8)
         float x[8];
-        if (h == 0u) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) x[k] = se[k];
-        } else {
-            x[0] = ne;
-            x[1] = se[8];
-#pragma unroll
-            for (int k = 2; k < 8; ++k) x[k] = 0.0f;
-        }
+        for (int k = 0; k < 8; ++k) x[k] = h == 0u ? se[k] : k < 2 ? se[8 + k] : 0.0f;
 #pragma unroll
         for (int part = 0; part < 3; ++part) {
             bf16x8 a;
@@ -343,7 +371,7 @@ k_sur_forward(WalkBuffers wb, const uint32_t* __restrict__ batch, uint32_t nbatc
                 x[k] = x[k] - (float)a[k];
             }
 #pragma unroll
-            for (int hb = 0; hb < 4; ++hb) acc[hb] = mfma16(a, B.blk0[hb], acc[hb]);
+            for (int hb = 0; hb < 4; ++hb) acc[hb] = mfma16(a, B[hb], acc[hb]);
         }
     }
     wave_sync();  // the list is free from here on
@@ -739,7 +767,7 @@ __global__ __launch_bounds__(256) void k_sur_wgrad(SurGradRows g, const __bf16* 
 //  - The features are written to LDS as ten rows of 64 edges, in the order the B operand takes
 //    them (the accumulator's row order), so an operand is one 16-byte read instead of eight
 //    2-byte ones and their packing.
-// 1,024 chunks: 600 -> 272 us.
+// 1,024 chunks: 600 -> 231 us.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kEdgeRow = 72;  // LDS row stride (bf16) of one feature over 64 edges
 
@@ -751,12 +779,12 @@ k_sur_edges_bwd(
     const SceneGrid* __restrict__ scenes, const __bf16* __restrict__ pk, SurScales sc,
     const __bf16* __restrict__ DS, float* __restrict__ part) {
     __shared__ WalkLds lds_all[kEdgeWaves];
-    __shared__ alignas(16) __bf16 le_all[kEdgeWaves][10 * kEdgeRow];
+    __shared__ alignas(16) uint16_t le_all[kEdgeWaves][10 * kEdgeRow];
     const uint32_t half = uni(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t col = lane & 31u, h = lane >> 5;
     WalkLds& L = lds_all[half];
-    __bf16* le = le_all[half];
+    uint16_t* le = le_all[half];
     const uint32_t b = blockIdx.x;
     if (b >= nbatch) return;
     const uint32_t item = uni(batch[b]);
@@ -769,13 +797,10 @@ k_sur_edges_bwd(
                     pi))
         return;
     const float4 vi = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    Layer1B B;
+    bf16x8 B[4];
     load_layer1(pk, lane, B);
 #pragma unroll
-    for (int hb = 0; hb < 4; ++hb) {
-        B.blk0[hb] = negated(B.blk0[hb]);
-        B.blk1[hb] = negated(B.blk1[hb]);
-    }
+    for (int hb = 0; hb < 4; ++hb) B[hb] = negated(B[hb]);
     // dS of this lane's hidden units for the 16 accumulator rows, as bf16 pairs (rows v, v + 1)
     uint32_t ds[4][8];
 #pragma unroll
@@ -791,23 +816,25 @@ k_sur_edges_bwd(
     const uint32_t epos =
         (lane & 32u) + (col & 16u) + ((col >> 2) & 1u) * 8u + ((col >> 3) & 1u) * 4u + (col & 3u);
     // this lane's feature row (columns from 10 on are garbage that is never stored)
-    const __bf16* erow = le + min(col, 9u) * kEdgeRow + 8u * h;
+    const __bf16* erow = reinterpret_cast<const __bf16*>(le) + min(col, 9u) * kEdgeRow + 8u * h;
     f32x16 accw[4];
 #pragma unroll
     for (int hb = 0; hb < 4; ++hb) accw[hb] = zero16();
-    walk_pairs(item, ch, s, active, pi, clane, wb, spm, svr, cs, c, L, lane,
+    walk_pairs<true>(item, ch, s, active, pi, clane, wb, spm, svr, cs, c, L, lane,
                [&](bool edge, float4 pj, float4 vj, float d2) {
-                   bf16x8 fe;
-                   __bf16 e8;
-                   edge_features(edge, pi, vi, pj, vj, d2, sc, fe, e8);
+                   uint32_t fe[4], ext;
+                   edge_features<false>(edge, pi, vi, pj, vj, d2, sc, fe, ext);
                    // features 0..8 and 1 of this lane's edge
 #pragma unroll
-                   for (int k = 0; k < 8; ++k) le[k * kEdgeRow + epos] = fe[k];
-                   le[8 * kEdgeRow + epos] = e8;
-                   le[9 * kEdgeRow + epos] = (__bf16)(edge ? 1.0f : 0.0f);
+                   for (int k = 0; k < 4; ++k) {
+                       le[2 * k * kEdgeRow + epos] = (uint16_t)fe[k];
+                       le[(2 * k + 1) * kEdgeRow + epos] = (uint16_t)(fe[k] >> 16);
+                   }
+                   le[8 * kEdgeRow + epos] = (uint16_t)(ext >> 16);
+                   le[9 * kEdgeRow + epos] = (uint16_t)ext;
                    wave_sync();
                    bf16x8 a[2];
-                   layer1_a(fe, e8, edge, lane, a[0], a[1]);
+                   layer1_a<false>(fe, ext, a[0], a[1]);
 #pragma unroll
                    for (int blk = 0; blk < 2; ++blk) {
                        const bf16x8 e0 = load8(erow + 32 * blk);
@@ -815,11 +842,11 @@ k_sur_edges_bwd(
 #pragma unroll
                        for (int hb = 0; hb < 4; ++hb) {
                            // -u of 16 edges
-                           const f32x16 d =
-                               mfma16(a[blk], blk == 0 ? B.blk0[hb] : B.blk1[hb], zero16());
+                           const f32x16 d = mfma16(a[blk], B[hb], zero16());
                            uint32_t g[8];
 #pragma unroll
-                           for (int k = 0; k < 8; ++k) g[k] = ds[hb][k] & neg_masks(d[2 * k], d[2 * k + 1]);
+                           for (int k = 0; k < 8; ++k)
+                               g[k] = ds[hb][k] & neg_masks(d[2 * k], d[2 * k + 1]);
                            accw[hb] = mfma16(
                                __builtin_bit_cast(bf16x8, make_uint4(g[0], g[1], g[2], g[3])), e0,
                                accw[hb]);

@@ -929,6 +929,7 @@ struct ListBuilder {
     uint32_t cnt = 0;    // neighbour bits of this lane's column in the window
 };
 
+template <bool kLong>
 __device__ __forceinline__ bool build_list(ListBuilder& lb, bool stored, int total_words,
                                            const WalkBuffers& wb, uint32_t item,
                                            uint32_t clane, Cursor& cu, const Chunk& ch,
@@ -942,9 +943,11 @@ __device__ __forceinline__ bool build_list(ListBuilder& lb, bool stored, int tot
     bool any = false;
     if (stored) {
         const size_t base = (size_t)item * c.max_words;
-        // a window of up to kListCap words cannot overflow a column list
-        const int end = min(total_words, lb.wpos + kListCap);
-        while (lb.wpos < end) {
+        // A window ends before a column list could overflow: after kListCap words, or (kLong)
+        // when a batch more could fill the longest list.
+        const int end = kLong ? total_words : min(total_words, lb.wpos + kListCap);
+        while (lb.wpos < end &&
+               (!kLong || __ballot(lb.n_ne > (uint32_t)(kListCap - kBatch)) == 0ull)) {
             const int nb = min(kBatch, end - lb.wpos);
             uint32_t wv[kBatch];
             uint32_t jv[kBatch];
@@ -1016,8 +1019,12 @@ struct PairWalk {
 
 // Walks every neighbour j != i of the wavefront's 32 targets, two lanes per target, in
 // uniform steps; body(edge, pj, vj, d2) is called once per step (edge = false on lanes with
-// nothing left).  Neighbour data is requested one step ahead (vj only with kVel).
-template <bool kVel = true, class Body>
+// nothing left).  Neighbour data is requested one step ahead (vj only with kVel).  kLong: windows
+// of as many words as the lists hold (about half of a chunk's words hold no neighbour of a
+// given target, so most chunks of 60 to 90 words are one window, and each window costs the
+// wavefront its largest lane's remainder: edge pass backward 269 -> 232 us with the operands' swap, 1,024
+// chunks).  Windows fix the order of a target's edges.
+template <bool kLong, bool kVel = true, class Body>
 __device__ __forceinline__ void walk_pairs(uint32_t item, const Chunk& ch, uint32_t s,
                                            bool active, float4 pi, uint32_t clane,
                                            const WalkBuffers& wb, const float4* spm,
@@ -1032,7 +1039,7 @@ __device__ __forceinline__ void walk_pairs(uint32_t item, const Chunk& ch, uint3
     if (!stored) cursor_begin(cu, ch, cs_, c);
     ListBuilder lb;
     for (;;) {
-        if (!build_list(lb, stored, total_words, wb, item, clane, cu, ch, spm, cs_, c, pi, lane,
+        if (!build_list<kLong>(lb, stored, total_words, wb, item, clane, cu, ch, spm, cs_, c, pi, lane,
                         L))
             break;
         wave_sync();
