@@ -10,9 +10,9 @@
 // Phase 1 (test): the chunk's candidate words (32 consecutive slots of one column) are
 //   visited in the cursor's order (parts, passes, columns: see kPasses), and each lane gets
 //   one bit per candidate from the conservative integer filter: on the matrix cores
-//   (mfma_filter_word, 32 candidates x 64 targets per word) where the chunk's coordinates fit
-//   its exact range, else one candidate at a time for the whole wave (push_quant, candidate
-//   data through the scalar cache).  `wj0[w]` is the sorted slot of the first candidate of
+//   (mfma_filter_word, 32 candidates x 64 targets per word), or one candidate at a time for
+//   the whole wave (push_quant, candidate data through the scalar cache) in the force walk's
+//   re-test and the neighbour-list export.  `wj0[w]` is the sorted slot of the first candidate of
 //   word w.  Segments hold up to kSeg - 1 words and never span two parts.
 // Phase 2 (evaluate): every lane walks only its own set bits and evaluates the kernel for
 //   those pairs (pairs the filter let through beyond the radius weigh exactly zero).
@@ -197,9 +197,9 @@ __device__ __forceinline__ float density_run(BitWalk<kW>& bw, float4& q0, float4
 }
 
 // Density pass over one chunk (kSplit false: all parts; true: the part of this wavefront,
-// three wavefronts per chunk, the sums finished by k_density_finish).  Seven wavefronts per
-// SIMD: the 15-word shapes' LDS allows it, and the walk is VALU-bound (a few spills outside
-// the walk loops; measured faster at 1M than the 6 the default register allocation gives).
+// three wavefronts per chunk, the sums finished by k_density_finish).  As many wavefronts per
+// SIMD as the LDS allows (six with 24-word segments): the walk is VALU-bound (a few spills
+// outside the walk loops).
 // The split shapes serve small scenes, whose wavefronts are few: no occupancy target, so
 // their deeper read-ahead stays in registers.  The ping-pong shapes aim at what their LDS
 // allows (6 with two 12-word buffers, 4 with two 16-word ones).
@@ -232,11 +232,14 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
     float4 pi;
     if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
     const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
-    init_sentinel<kLds>(lmask, lwj0, lane, c);
     MfmaFilter mf;
-    mfma_filter_begin(mf, ch, sq, qi, lane, c.qneg);
+    mfma_filter_begin(mf, ch, sq, qi, active, lane, c.qneg);
     WordTable wt;
-    const bool tab = word_table_build(wt, ch, cs, c, part, lane);
+    static_assert(kLds * 64 >= kTableWords, "the word table is built in the mask buffer");
+    const bool tab = word_table_build(wt, ch, cs, part, lane, lmask);
+    init_sentinel<kLds>(lmask, lwj0, lane, c);
+    uint32_t* const gm = gmask + (size_t)item * c.max_words * 64;
+    uint32_t* const gj = gwj0 + (size_t)item * c.max_words;
     if (lane == 0 && part <= 0) {
         gpart[item] = pack_parts(wt.ps1, wt.ps2);
         gnw[item] = (uint32_t)wt.total;
@@ -266,7 +269,7 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
                 SegLane sl;
                 int seg_part;
                 const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, qi, active, lm_new, lj_new,
-                                                        lane, sl, seg_part, mf)
+                                                        gm, gj, lane, sl, seg_part, mf)
                                    : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active,
                                                                 lm_new, lj_new, lane, sl,
                                                                 seg_part, &mf);
@@ -274,8 +277,7 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
                     more = false;
                 } else {
                     wave_sync();
-                    store_words(item, c.max_words, seg_base, nw, lm_new, lj_new, gmask, gwj0,
-                                lane);
+                    if (!tab) store_words(c.max_words, seg_base, nw, lm_new, lj_new, gm, gj, lane);
                     seg_base += nw;
                     if (tab ? ti >= wt.n : cu.done) more = false;
                     if (walk_part < 0 || seg_part == walk_part) {
@@ -328,8 +330,8 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
             SegLane sl;
             int seg_part;
             const int nw =
-                tab ? phase1_table<kSeg>(wt, ti, sq, c, qi, active, lmask, lwj0, lane, sl, seg_part,
-                                         mf)
+                tab ? phase1_table<kSeg>(wt, ti, sq, c, qi, active, lmask, lwj0, gm, gj, lane, sl,
+                                         seg_part, mf)
                     : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
                                                  sl, seg_part, &mf);
             if (nw == 0) break;
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
                 }
             }
             wave_sync();
-            store_words(item, c.max_words, seg_base, nw, lmask, lwj0, gmask, gwj0, lane);
+            if (!tab) store_words(c.max_words, seg_base, nw, lmask, lwj0, gm, gj, lane);
             BitWalk<kSeg> bw;
             bw.begin(sl.nonempty, lmask, lwj0, lane);
             const uint32_t steps = wave_max(sl.count);

@@ -353,78 +353,74 @@ struct WordTable {
     int total;        // uniform: words of the whole chunk
 };
 
-// Words of a column of nw words in pass s: s, s + kPasses, ...
-__device__ __forceinline__ int pass_words(int nw, int s) {
-    return nw > s ? (nw - s + kPasses - 1) / kPasses : 0;
+// Inclusive prefix sums over lanes 0-31 and, separately, over lanes 32-63 (row shifts within
+// 16 lanes, then lane 15 of each first row added to the second).
+__device__ __forceinline__ uint32_t half_wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, true);
+    return v;
+}
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
 }
 
 // Counts the chunk's words; fills the table for the range of `part` (all parts if < 0) when
-// it holds at most kTableWords words.  Returns whether the table is filled.
+// it holds at most kTableWords words.  Returns whether the table is filled.  Lane k < 25 owns
+// the column at order position k: the ranges of all columns come in one round trip, word
+// counts and places from two prefix sums (the counts of the four passes in one word, a byte
+// each: a filled table has at most 128), and each lane writes its columns' entries to
+// `scratch` (kTableWords words of LDS).  One column after the other, unrolled over columns,
+// parts and passes, this took 18,000 cycles of a wavefront's 190,000 at 184,000 particles
+// (scalar loads in turn, 2,000 instructions from a cold instruction cache).
 __device__ __forceinline__ bool word_table_build(WordTable& t, const Chunk& ch,
-                                                 const uint32_t* __restrict__ cs,
-                                                 const StepConsts& c, int part, uint32_t lane) {
-    int nw[25];
-    int pw[3] = {0, 0, 0};
-    int W[3][kPasses] = {};
-#pragma unroll
-    for (int k = 0; k < 25; ++k) {
-        int dx, dy;
-        nw[k] = 0;
-        if (column_at(ch, 0, k, dx, dy)) {
-            uint32_t a, b;
-            column_range(ch, dx, dy, cs, c, a, b);
-            nw[k] = (int)((b - a + 31u) / 32u);
-        }
-        const int p = part_of_position(k);
-        pw[p] += nw[k];
-#pragma unroll
-        for (int s = 0; s < kPasses; ++s) W[p][s] += pass_words(nw[k], s);
+                                                 const uint32_t* __restrict__ cs, int part,
+                                                 uint32_t lane, uint32_t* __restrict__ scratch) {
+    static_assert(kPasses == 4 && kTableWords <= 255, "pass counts are packed in bytes");
+    const int code = (int)kColumnOrder[0][min(lane, 24u)];
+    const int dx = code / 5 - 2, dy = code % 5 - 2;
+    const bool walked = lane < 25u && dx >= ch.dx0 && dx <= ch.dx1 && dy >= ch.dy0 && dy <= ch.dy1;
+    uint32_t a = 0u, b = 0u;
+    if (walked) {
+        const uint32_t base = ch.cell_base +
+                              ((uint32_t)(ch.rx + dx) * ch.ny + (uint32_t)(ch.ry + dy)) * ch.nz;
+        a = cs[base + (uint32_t)ch.zlo];
+        b = cs[base + (uint32_t)ch.zhi + 1u];
     }
-    t.ps1 = pw[0];
-    t.ps2 = pw[0] + pw[1];
-    t.total = t.ps2 + pw[2];
+    const int p = part_of_position((int)lane);
+    uint32_t nw = (b - a + 31u) / 32u;
+    const uint32_t words = half_wave_scan(nw);  // words up to this column
+    t.ps1 = (int)lane_value(words, 4);
+    t.ps2 = (int)lane_value(words, 8);
+    t.total = (int)lane_value(words, 24);
     t.first = part > 0 ? (part == 1 ? t.ps1 : t.ps2) : 0;
-    t.n = part >= 0 ? pw[part] : t.total;
+    t.n = part < 0 ? t.total : part == 0 ? t.ps1 : part == 1 ? t.ps2 - t.ps1 : t.total - t.ps2;
     t.e0 = t.e1 = 0u;
     if (t.n > kTableWords) return false;
-    const int i0 = t.first + (int)lane, i1 = i0 + 64;  // stored-word indices of this lane's entries
-    int base = 0;
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-        int pre[kPasses];
-        int pb[kPasses];  // stored-word index where pass s of part p starts
-#pragma unroll
-        for (int s = 0; s < kPasses; ++s) {
-            pre[s] = 0;
-            pb[s] = s == 0 ? base : pb[s - 1] + W[p][s - 1];
+    if (part >= 0 && p != part) nw = 0u;
+    // words of this column in passes 0-3 (s, s + 4, ...), a byte each; sums over the part's
+    // columns before it, and the part's passes before each pass
+    const uint32_t own = (nw + 3u) >> 2 | ((nw + 2u) >> 2) << 8 | ((nw + 1u) >> 2) << 16 |
+                         (nw >> 2) << 24;
+    const uint32_t incl = half_wave_scan(own);
+    const uint32_t i0 = lane_value(incl, 4), i1 = lane_value(incl, 8), i2 = lane_value(incl, 24);
+    const uint32_t before = p == 0 ? 0u : p == 1 ? i0 : i1;
+    const uint32_t sum = p == 0 ? i0 : p == 1 ? i1 - i0 : i2 - i1;
+    const uint32_t lo = incl - own - before + sum * 0x01010100u;
+    const uint32_t base = part >= 0 || p == 0 ? 0u : (uint32_t)(p == 1 ? t.ps1 : t.ps2);
+    for (uint32_t w = 0; __ballot(w < nw) != 0ull; ++w) {
+        if (w < nw) {
+            const uint32_t j0 = a + 32u * w;
+            scratch[base + ((lo >> (8u * (w & 3u))) & 255u) + (w >> 2)] =
+                j0 | (min(32u, b - j0) - 1u) << 27;
         }
-        if (part < 0 || part == p) {
-#pragma unroll
-            for (int k = part_begin(p); k < part_end(p); ++k) {
-                if (nw[k] == 0) continue;
-                int dx, dy;
-                column_at(ch, 0, k, dx, dy);
-                uint32_t a, b;
-                column_range(ch, dx, dy, cs, c, a, b);
-#pragma unroll
-                for (int s = 0; s < kPasses; ++s) {
-                    const int m = pass_words(nw[k], s);
-                    const int lo = pb[s] + pre[s];
-                    // entry for stored-word index i: word s + kPasses (i - lo) of the column
-                    if (i0 >= lo && i0 < lo + m) {
-                        const uint32_t j0 = a + 32u * (uint32_t)(s + kPasses * (i0 - lo));
-                        t.e0 = j0 | (min(32u, b - j0) - 1u) << 27;
-                    }
-                    if (i1 >= lo && i1 < lo + m) {
-                        const uint32_t j0 = a + 32u * (uint32_t)(s + kPasses * (i1 - lo));
-                        t.e1 = j0 | (min(32u, b - j0) - 1u) << 27;
-                    }
-                    pre[s] += m;
-                }
-            }
-        }
-        base += pw[p];
     }
+    wave_sync();
+    if ((int)lane < t.n) t.e0 = scratch[lane];
+    if ((int)lane + 64 < t.n) t.e1 = scratch[64u + lane];
+    wave_sync();
     return true;
 }
 
@@ -473,80 +469,113 @@ __device__ __forceinline__ uint32_t push_quant(uint32_t word, uint2 a, uint2 b, 
 // magnitude <= 2048 (exact in f16) and every partial sum an integer below 2^24 (exact in the
 // FP32 accumulator) when all coordinates lie within +-1024 of the origin: the first target's
 // x, y (candidates are at most 2 cells + 1 unit away: |.| <= 769) and, in z, the middle of the
-// candidate cells (|.| <= 128 (zhi - zlo + 1) + 257: at most 5 candidate z cells).  Chunks with
-// more use the VALU test.  The verdicts equal the VALU test's wherever that one does not wrap
-// around, which only adds far candidates; either way only such candidates differ, and they
+// candidate cells (|.| <= 128 (zhi - zlo + 1) + 257: at most 5 candidate z cells).
+// Chunks of more z cells (sparse columns: the faces and the free surface of every scene) take
+// the z origin of each word in the middle of its first and last candidate and clamp both
+// sides' z to +-1023 of it.  Clamping brings no two points apart, so it can turn a far
+// candidate into a passing one, never a neighbour into a failing one.  Testing such chunks on
+// the VALU instead took 3 times the words' time, and with one wavefront per chunk they ended
+// the launch: a density walk of 184,000 particles 149 -> 106 us, of 1M 430 -> 389 us with this,
+// the word table by lanes and the words stored as they are formed.
+// Only chunks of 2^21 z cells and more, whose z differences could wrap around in 32 bits, use
+// the VALU test.  The verdicts equal the VALU test's but for far candidates, and those
 // add exactly zero.
 // ---------------------------------------------------------------------------
 typedef _Float16 sphk_half8 __attribute__((ext_vector_type(8)));
 typedef float sphk_f32x16 __attribute__((ext_vector_type(16)));
 
 struct MfmaFilter {
-    bool on;             // uniform: the chunk fits the exact range
+    bool on;             // uniform: tested on the matrix cores
+    bool wide;           // uniform: more than 5 candidate z cells, a z origin per word
     uint32_t ox, oz;     // origin: packed x | y << 16 (16-bit wrap-around), z
+    sphk_short2 axy;     // this lane's target: x, y from the origin, its z, and
+    uint32_t qz;         //   x^2 + y^2 + qneg
+    int32_t axy2;
+    bool active;         // this lane has a target
     sphk_half8 b1, b2;   // B operands: targets 0-31 and 32-63 (lanes 0-31 hold them)
     uint32_t crow;       // candidate of this lane's A row: 16 ((m >> 2) & 1) + 4 (m >> 3) + (m & 3)
-    uint32_t pref_j;     // uniform: first slot of the word whose row is in `pref` (~0: none)
-    uint2 pref;          // this lane's row of the next word of the current column
 };
 
-__device__ __forceinline__ void mfma_filter_begin(MfmaFilter& mf, const Chunk& ch,
-                                                  const uint2* __restrict__ sq, uint2 qi,
-                                                  uint32_t lane, int32_t qneg) {
-    mf.on = ch.zhi - ch.zlo <= 4;
-    const uint32_t qfx = uni(sq[ch.s0].x), qfz = uni(sq[ch.s0].y);
-    mf.ox = qfx;
-    mf.oz = qfz + (uint32_t)(128 * (ch.zlo + ch.zhi + 1 - 2 * ch.zfirst));
-    const sphk_short2 a = __builtin_bit_cast(sphk_short2, qi.x) - __builtin_bit_cast(sphk_short2, mf.ox);
-    // (lanes without a target compute garbage in their own columns only; unsigned
-    // arithmetic keeps that free of overflow)
-    const uint32_t az = qi.y - mf.oz;
-    const int32_t aa = __builtin_amdgcn_sdot2(a, a, (int32_t)(az * az + (uint32_t)qneg), false);
+// The B operands for z origin mf.oz.
+__device__ __forceinline__ void mfma_filter_targets(MfmaFilter& mf, uint32_t lane) {
+    const int32_t az = min(max((int32_t)(mf.qz - mf.oz), -1023), 1023);
+    const int32_t aa = mf.axy2 + az * az;
     sphk_half8 p;
-    p[0] = (_Float16)(-2 * (int32_t)a.x);
-    p[1] = (_Float16)(-2 * (int32_t)a.y);
-    p[2] = (_Float16)(int32_t)(0u - 2u * az);
+    p[0] = (_Float16)(-2 * (int32_t)mf.axy.x);
+    p[1] = (_Float16)(-2 * (int32_t)mf.axy.y);
+    p[2] = (_Float16)(-2 * az);
     p[3] = (_Float16)1.0f;
     p[4] = (_Float16)2048.0f;
     p[5] = (_Float16)(aa & 2047);
     p[6] = (_Float16)(aa >> 11);
     p[7] = (_Float16)0.0f;
-    sphk_half8 q;
-    const uint4 pu = __builtin_bit_cast(uint4, p);
-    uint4 qu;
-    qu.x = (uint32_t)__shfl_xor((int)pu.x, 32);
-    qu.y = (uint32_t)__shfl_xor((int)pu.y, 32);
-    qu.z = (uint32_t)__shfl_xor((int)pu.z, 32);
-    qu.w = (uint32_t)__shfl_xor((int)pu.w, 32);
-    q = __builtin_bit_cast(sphk_half8, qu);
-    const bool lo = lane < 32u;
-    const sphk_half8 zero = {};
-    mf.b1 = lo ? p : zero;
-    mf.b2 = lo ? q : zero;
-    const uint32_t m = lane & 31u;
-    mf.crow = 16u * ((m >> 2) & 1u) + 4u * (m >> 3) + (m & 3u);
-    mf.pref_j = ~0u;
-    mf.pref = make_uint2(0u, 0u);
+    uint4 pu = __builtin_bit_cast(uint4, p);
+    if (!mf.active) {
+        // b.b + 2048 * 1024 >= 0: no candidate passes
+        pu = make_uint4(0u, 0x3c000000u, 0x00006800u, 0x00006400u);
+    }
+    // v_permlane32_swap(x, 0): x of the lower lanes with zero above, and x of the upper lanes
+    // moved down with zero above
+    uint32_t l[4], h[4];
+    const uint32_t v[4] = {pu.x, pu.y, pu.z, pu.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v[k], 0u, false, false);
+        l[k] = r[0];
+        h[k] = r[1];
+    }
+    mf.b1 = __builtin_bit_cast(sphk_half8, make_uint4(l[0], l[1], l[2], l[3]));
+    mf.b2 = __builtin_bit_cast(sphk_half8, make_uint4(h[0], h[1], h[2], h[3]));
 }
 
-// Verdict word of this lane's target over candidates j0 .. j0 + cnt - 1 (cnt in 1..32),
-// candidate k at bit 31 - k, like the VALU test.  The rows of the next word to be tested
-// (jn .. jn + cntn - 1; jn = ~0: none) are requested before this word's arithmetic.
-__device__ __forceinline__ uint32_t mfma_filter_word(MfmaFilter& mf,
-                                                     const uint2* __restrict__ sq, uint32_t j0,
-                                                     uint32_t cnt, uint32_t jn, uint32_t cntn,
+__device__ __forceinline__ void mfma_filter_begin(MfmaFilter& mf, const Chunk& ch,
+                                                  const uint2* __restrict__ sq, uint2 qi,
+                                                  bool active, uint32_t lane, int32_t qneg) {
+    const int zspan = ch.zhi - ch.zlo;
+    mf.on = zspan < (1 << 21);
+    mf.wide = zspan > 4;
+    // (the first target is lane 0's)
+    mf.ox = uni(qi.x);
+    mf.oz = uni(qi.y) + (uint32_t)(128 * (ch.zlo + ch.zhi + 1 - 2 * ch.zfirst));
+    mf.axy = __builtin_bit_cast(sphk_short2, qi.x) - __builtin_bit_cast(sphk_short2, mf.ox);
+    mf.axy2 = __builtin_amdgcn_sdot2(mf.axy, mf.axy, qneg, false);
+    mf.qz = qi.y;
+    mf.active = active;
+    const uint32_t m = lane & 31u;
+    mf.crow = 16u * ((m >> 2) & 1u) + 4u * (m >> 3) + (m & 3u);
+    if (!mf.wide) mfma_filter_targets(mf, lane);
+}
+
+// This lane's candidate row of the word [j0, j0 + cnt), cnt in 1..32.
+__device__ __forceinline__ uint2 mfma_filter_row(const MfmaFilter& mf,
+                                                 const uint2* __restrict__ sq, uint32_t j0,
+                                                 uint32_t cnt) {
+    return sq[j0 + min(mf.crow, cnt - 1u)];
+}
+
+// Verdict word of this lane's target over the word's `cnt` candidates, candidate k at bit
+// 31 - k, like the VALU test (no bit for lanes without a target).  qb: this lane's row.
+__device__ __forceinline__ uint32_t mfma_filter_word(MfmaFilter& mf, uint2 qb, uint32_t cnt,
                                                      uint32_t lane) {
-    const uint2 qb = mf.pref_j == j0 ? mf.pref : sq[j0 + min(mf.crow, cnt - 1u)];
+    int32_t bz;
+    if (mf.wide) {
+        // rows 0 and 31 (the last candidate) are lane 0's and lane 31's
+        const uint32_t z0 = uni(qb.y), z1 = lane_value(qb.y, 31);
+        mf.oz = z0 + (uint32_t)((int32_t)(z1 - z0) >> 1);
+        mfma_filter_targets(mf, lane);
+        bz = min(max((int32_t)(qb.y - mf.oz), -1023), 1023);
+    } else {
+        bz = (int16_t)(qb.y - mf.oz);
+    }
     const sphk_short2 b = __builtin_bit_cast(sphk_short2, qb.x) - __builtin_bit_cast(sphk_short2, mf.ox);
     // candidate offsets from the origin are below 2^11 per axis (the candidates lie within
     // the chunk's two-cell reach), so bz^2 is a 24-bit product and every A entry converts
     // from 16 bits in one instruction
-    const int16_t bz = (int16_t)(qb.y - mf.oz);
-    const int32_t bb = __builtin_amdgcn_sdot2(b, b, (int32_t)bz * (int32_t)bz, false);
+    const int32_t bb = __builtin_amdgcn_sdot2(b, b, __mul24(bz, bz), false);
     sphk_half8 a;
     a[0] = (_Float16)b.x;
     a[1] = (_Float16)b.y;
-    a[2] = (_Float16)bz;
+    a[2] = (_Float16)(int16_t)bz;
     a[3] = (_Float16)(int16_t)(bb & 2047);
     a[4] = (_Float16)(int16_t)(bb >> 11);
     a[5] = (_Float16)1.0f;
@@ -554,13 +583,6 @@ __device__ __forceinline__ uint32_t mfma_filter_word(MfmaFilter& mf,
     a[7] = (_Float16)0.0f;
     // lanes 32-63 supply K slots 8-15, whose B rows are zero: their A entries (the same
     // candidate's, finite) add exactly 0 and need no masking
-    // next word's rows, requested once this word's are used up (the empty asm pins the A
-    // operand before the request, so this word does not wait for the next one's load)
-    asm volatile("" ::"v"(a));
-    if (jn != ~0u) {
-        mf.pref = sq[jn + min(mf.crow, cntn - 1u)];
-        mf.pref_j = jn;
-    }
     const sphk_f32x16 z16 = {};
     const sphk_f32x16 d1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, mf.b1, z16, 0, 0, 0);
     const sphk_f32x16 d2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, mf.b2, z16, 0, 0, 0);
@@ -577,6 +599,30 @@ __device__ __forceinline__ uint32_t mfma_filter_word(MfmaFilter& mf,
     const auto xy = __builtin_amdgcn_permlane32_swap(x, y, false, false);
     const uint32_t word = xy[0] << 16 | xy[1];
     return word & (~0u << (32u - cnt));
+}
+
+// The same word on the VALU.
+__device__ __forceinline__ uint32_t valu_filter_word(const uint2* __restrict__ sq, uint32_t j0,
+                                                     uint32_t cnt, uint2 qi, bool active,
+                                                     int32_t qneg) {
+    const uint2* __restrict__ pb = sq + j0;  // uniform base: scalar loads
+    uint32_t word = 0;
+    if (cnt == 32u) {
+#pragma unroll
+        for (int k = 0; k < 32; ++k) word = push_quant(word, qi, pb[k], qneg);
+    } else {
+        for (uint32_t k = 0; k < cnt; ++k) word = push_quant(word, qi, pb[k], qneg);
+        word <<= (32u - cnt);
+    }
+    return active ? word : 0u;
+}
+
+// A formed word `w` of a segment: into LDS and the lane's summary.
+__device__ __forceinline__ void put_word(uint32_t word, int w, uint32_t* __restrict__ lmask,
+                                         uint32_t lane, SegLane& sl) {
+    lmask[w * 64 + lane] = word;
+    sl.nonempty |= min(word, 1u) << w;
+    sl.count += (uint32_t)__builtin_popcount(word);
 }
 
 template <int kSeg, bool kMfma = false>
@@ -601,24 +647,13 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
         }
         const uint32_t j0 = uni(cu.j);
         const uint32_t cnt = uni(min(32u, cu.end - j0));
-        uint32_t word = 0;
-        const uint2* __restrict__ pb = sq + j0;  // uniform base: scalar loads
-        if (kMfma && mf->on) {
-            const uint32_t jn = j0 + cu.step;
-            word = mfma_filter_word(*mf, sq, j0, cnt, jn < cu.end ? jn : ~0u,
-                                    jn < cu.end ? min(32u, cu.end - jn) : 0u, lane);
-        } else if (cnt == 32u) {
-#pragma unroll
-            for (int k = 0; k < 32; ++k) word = push_quant(word, qi, pb[k], c.qneg);
-        } else {
-            for (uint32_t k = 0; k < cnt; ++k) word = push_quant(word, qi, pb[k], c.qneg);
-            word <<= (32u - cnt);
-        }
-        word = active ? word : 0u;
-        lmask[w * 64 + lane] = word;
+        uint32_t word;
+        if (kMfma && mf->on)
+            word = mfma_filter_word(*mf, mfma_filter_row(*mf, sq, j0, cnt), cnt, lane);
+        else
+            word = valu_filter_word(sq, j0, cnt, qi, active, c.qneg);
+        put_word(word, w, lmask, lane, sl);
         if (lane == 0) lwj0[w] = j0;
-        sl.nonempty |= (word != 0u ? 1u : 0u) << w;
-        sl.count += (uint32_t)__builtin_popcount(word);
         cu.j = j0 + cu.step;
         ++w;
     }
@@ -626,51 +661,71 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
 }
 
 // Phase 1 over the word table: the next segment of up to kSeg - 1 words from local entry `i`
-// (advanced), never past a part start, tested on the matrix cores (or the VALU test where the
-// chunk is too wide for them).  Same words and order as phase1_segment.
+// (advanced), never past a part start.  Same words and order as phase1_segment.  The words go
+// to LDS and, from the registers that formed them, to the chunk's stored words (gm: its word
+// 0, `max_words` of them; nontemporal: the force walk reads them once, long after, and the rows
+// the walks gather should keep L2).  The candidate rows of kAheadWords words are in flight.
+constexpr int kAheadWords = 4;
 template <int kSeg>
 __device__ __forceinline__ int phase1_table(const WordTable& t, int& i,
                                             const uint2* __restrict__ sq, const StepConsts& c,
                                             uint2 qi, bool active, uint32_t* __restrict__ lmask,
-                                            uint32_t* __restrict__ lwj0, uint32_t lane,
+                                            uint32_t* __restrict__ lwj0,
+                                            uint32_t* __restrict__ gm,
+                                            uint32_t* __restrict__ gj, uint32_t lane,
                                             SegLane& sl, int& part, MfmaFilter& mf) {
     static_assert(kSeg <= 32, "one nonempty bit per word");
-    int w = 0;
     sl.nonempty = 0;
     sl.count = 0;
     const int g0 = t.first + i;
     part = g0 < t.ps1 ? 0 : g0 < t.ps2 ? 1 : 2;
-    while (w < kSeg - 1 && i < t.n) {
-        const int g = t.first + i;
-        if (w > 0 && (g == t.ps1 || g == t.ps2)) break;  // a new part starts the next segment
-        uint32_t j0, cnt;
-        word_table_entry(t, i, j0, cnt);
-        j0 = uni(j0);
-        cnt = uni(cnt);
-        uint32_t word = 0;
-        if (mf.on) {
-            uint32_t jn = ~0u, cntn = 0u;
-            if (i + 1 < t.n) word_table_entry(t, i + 1, jn, cntn);
-            word = mfma_filter_word(mf, sq, j0, cnt, uni(jn), uni(cntn), lane);
-        } else {
-            const uint2* __restrict__ pb = sq + j0;  // uniform base: scalar loads
-            if (cnt == 32u) {
+    const int part_last = part == 0 ? t.ps1 : part == 1 ? t.ps2 : t.total;
+    const int nw = min(min(kSeg - 1, t.n - i), part_last - g0);
+    if (nw <= 0) return 0;
+    const int stored = (int)c.max_words - g0;  // words of the segment the engine stores
+    uint32_t jv = 0;                           // lane w: first slot of word w
+    auto store = [&](uint32_t word, int w) {
+        put_word(word, w, lmask, lane, sl);
+        if (w < stored) __builtin_nontemporal_store(word, &gm[(size_t)(g0 + w) * 64 + lane]);
+    };
+    if (mf.on) {
+        uint2 q[kAheadWords] = {};
+        auto request = [&](int w, uint2& r) {
+            uint32_t j0, cnt;
+            if (w >= nw) return;
+            word_table_entry(t, i + w, j0, cnt);
+            r = mfma_filter_row(mf, sq, j0, cnt);
+        };
 #pragma unroll
-                for (int k = 0; k < 32; ++k) word = push_quant(word, qi, pb[k], c.qneg);
-            } else {
-                for (uint32_t k = 0; k < cnt; ++k) word = push_quant(word, qi, pb[k], c.qneg);
-                word <<= (32u - cnt);
+        for (int k = 0; k < kAheadWords; ++k) request(k, q[k]);
+        for (int w0 = 0; w0 < nw; w0 += kAheadWords) {
+#pragma unroll
+            for (int k = 0; k < kAheadWords; ++k) {
+                const int w = w0 + k;
+                if (w < nw) {
+                    uint32_t j0, cnt;
+                    word_table_entry(t, i + w, j0, cnt);
+                    jv = lane == (uint32_t)w ? j0 : jv;
+                    const uint32_t word = mfma_filter_word(mf, q[k], cnt, lane);
+                    request(w + kAheadWords, q[k]);
+                    store(word, w);
+                }
             }
         }
-        word = active ? word : 0u;
-        lmask[w * 64 + lane] = word;
-        if (lane == 0) lwj0[w] = j0;
-        sl.nonempty |= (word != 0u ? 1u : 0u) << w;
-        sl.count += (uint32_t)__builtin_popcount(word);
-        ++i;
-        ++w;
+    } else {
+        for (int w = 0; w < nw; ++w) {
+            uint32_t j0, cnt;
+            word_table_entry(t, i + w, j0, cnt);
+            jv = lane == (uint32_t)w ? j0 : jv;
+            store(valu_filter_word(sq, uni(j0), uni(cnt), qi, active, c.qneg), w);
+        }
     }
-    return w;
+    if ((int)lane < nw) {
+        lwj0[lane] = jv;
+        if ((int)lane < stored) gj[g0 + (int)lane] = jv;
+    }
+    i += nw;
+    return nw;
 }
 
 // Builds the wave-uniform chunk description; returns false for an out-of-range item.
@@ -796,26 +851,18 @@ __device__ __forceinline__ void add_nbr_stats(uint32_t cnt, unsigned long long* 
     }
 }
 
-// Stores the LDS words [0, nw) of segment `seg_base` of this chunk into HBM (nontemporal: the
-// force walk reads them once, long after, and the rows the walks gather should keep L2).
-__device__ __forceinline__ void store_words(uint32_t item, uint32_t max_words, int seg_base,
-                                            int nw,
+// Stores the LDS words [0, nw) of segment `seg_base` of a chunk into its stored words gm and
+// gj (the cursor's route; phase1_table stores its words as it forms them).
+__device__ __forceinline__ void store_words(uint32_t max_words, int seg_base, int nw,
                                             const uint32_t* __restrict__ lmask,
                                             const uint32_t* __restrict__ lwj0,
-                                            uint32_t* __restrict__ gmask,
-                                            uint32_t* __restrict__ gwj0, uint32_t lane) {
-    const size_t base = (size_t)item * max_words;
-    for (int w = 0; w < nw; ++w) {
-        int gw = seg_base + w;
-        if (gw >= (int)max_words) break;
-        __builtin_nontemporal_store(lmask[w * 64 + lane], &gmask[(base + gw) * 64 + lane]);
-    }
-    for (int w = (int)lane; w < nw; w += 64) {
-        int gw = seg_base + w;
-        if (gw < (int)max_words) gwj0[base + gw] = lwj0[w];
-    }
+                                            uint32_t* __restrict__ gm, uint32_t* __restrict__ gj,
+                                            uint32_t lane) {
+    const int end = min(nw, (int)max_words - seg_base);
+    for (int w = 0; w < end; ++w)
+        __builtin_nontemporal_store(lmask[w * 64 + lane], &gm[(size_t)(seg_base + w) * 64 + lane]);
+    if ((int)lane < end) gj[seg_base + (int)lane] = lwj0[lane];
 }
-
 
 // ---------------------------------------------------------------------------
 // Pair walk: two lanes per target (l and l ^ 32), 32 targets per wavefront.  The non-empty
@@ -1086,8 +1133,9 @@ struct WalkShape {
     // occupancy target of the force walk: 5 wavefronts per SIMD where the LDS allows it
     // (24- and 28-word segments without the LDS running total), else what the registers give
     static constexpr int force_waves = (!kPP && (kSeg == 24 || kSeg == 28)) ? 5 : 1;
-    // occupancy target of the single-wavefront density walk
-    static constexpr int density_waves = !kPP ? 7 : kSeg <= 12 ? 6 : 4;
+    // occupancy target of the single-wavefront density walk: what its LDS allows, 7 at most
+    static constexpr int density_waves =
+        kPP ? (kSeg <= 12 ? 6 : 4) : kSeg <= 16 ? 7 : kSeg <= 24 ? 6 : kSeg <= 28 ? 5 : 4;
 };
 
 }  // namespace

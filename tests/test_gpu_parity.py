@@ -345,6 +345,32 @@ def test_stored_candidate_words_hold_every_pair(sphk, oracle, scenes, scene_kind
     assert 0.0 <= slack < 0.05  # measured 0.011 (lattice) and 0.006 (config 0)
 
 
+@pytest.mark.parametrize("shape", ["seg24_waves4", "seg16_waves4_split", "seg32_waves4_split",
+                                   "pp12_waves4"])
+@pytest.mark.parametrize("per_cell", [0.3, 2.0, 12.0])
+def test_sparse_columns_hold_every_pair(sphk, oracle, scenes, per_cell, shape):
+    # Chunks that span more than five z cells (tall, sparsely filled columns; at 0.3 particles a
+    # cell a word of 32 candidates spans some hundred cells) take the matrix-core filter's z
+    # origin word by word, z clamped on both sides: no neighbour may be lost, none stored
+    # twice.  A dense block in the same columns mixes narrow and wide chunks.
+    rng = np.random.default_rng(int(10 * per_cell))
+    cells = 4 * 4 * 200
+    pos = rng.uniform([0.01, 0.01, -3.0], [0.17, 0.17, 5.0], size=(int(cells * per_cell), 3))
+    pos = np.concatenate([pos, rng.uniform(0.02, 0.10, size=(700, 3))]).astype(np.float32)
+    e = sphk.Engine(len(pos), sphk.default_params(xmin=0, xmax=1, ymin=0, ymax=1, zmin=-4, zmax=6))
+    e.upload(pos)
+    names = sphk.walk_shape_names()
+    e.set_walk_shapes(names.index(shape), names.index("seg32_waves4"))
+    n = len(pos)
+    tgt, cand, overflow = _stored_pairs(e, n)
+    assert overflow == 0
+    codes = tgt * n + cand
+    assert len(np.unique(codes)) == len(codes), "a candidate stored twice"
+    boffs, bidx = oracle.brute_neighbors(pos, np.float32(R2))
+    bt = np.repeat(np.arange(n, dtype=np.int64), np.diff(boffs))
+    assert np.isin(bt * n + bidx.astype(np.int64), codes).all(), "a neighbour was filtered out"
+
+
 def test_far_from_origin_against_brute_force(sphk, oracle):
     # Coordinates near 1000 (cell index ~25,000): the quantized filter keeps its coordinates
     # modulo 2^16 (x, y) and 2^32 (z), so neighbour differences must survive the wrap-around.
