@@ -509,22 +509,6 @@ int ensure_grid(sphk_engine* e) {
         e->shape_density = small ? kShapeSmall : kShapeLargeDensity;
         e->shape_force = small ? kShapeSmall : kShapeLargeForce;
     }
-    // per-part sums of the split walk shapes: three sums per slot, only while selected
-    if ((walk_shape_split(e->shape_density) || walk_shape_split(e->shape_force)) &&
-        wb.part_cap < e->cap) {
-        if (wb.part_acc) HIP_TRY(hipFree(wb.part_acc));
-        wb.part_acc = nullptr;
-        if (wb.part_cnt) HIP_TRY(hipFree(wb.part_cnt));
-        wb.part_cnt = nullptr;
-        if (wb.part_force) HIP_TRY(hipFree(wb.part_force));
-        wb.part_force = nullptr;
-        wb.part_cap = 0;
-        HIP_TRY(dalloc(&wb.part_acc, kParts * e->cap));
-        HIP_TRY(dalloc(&wb.part_cnt, kParts * e->cap));
-        HIP_TRY(dalloc(&wb.part_force, 2 * kParts * e->cap));
-        wb.part_cap = e->cap;
-        ++e->buffer_gen;
-    }
     uint64_t ccap = wb.col_cap;
     if (int rc = grow(&wb.colcnt, ccap, ncols + 1, e->buffer_gen)) return rc;
     wb.col_cap = ccap;
@@ -954,8 +938,7 @@ int sphk_destroy(sphk_engine* e) {
         if (p) (void)hipFree(p);
     for (void* p : {(void*)e->walk.items, (void*)e->walk.desc, (void*)e->walk.nitems, (void*)e->walk.colcnt,
                     (void*)e->walk.mask, (void*)e->walk.wj0, (void*)e->walk.nwords,
-                    (void*)e->walk.pstarts, (void*)e->walk.part_acc, (void*)e->walk.part_cnt,
-                    (void*)e->walk.part_force, (void*)e->scan_scratch, (void*)e->d_scenes,
+                    (void*)e->walk.pstarts, (void*)e->scan_scratch, (void*)e->d_scenes,
                     (void*)e->lookback, (void*)e->bbox_ranges, (void*)e->bbox_out})
         if (p) (void)hipFree(p);
     if (e->stage) (void)hipHostFree(e->stage);
@@ -1597,10 +1580,6 @@ int sphk_set_walk_shapes(sphk_engine* e, int density_shape, int force_shape) {
     e->shape_density = density_shape;
     e->shape_force = force_shape;
     e->shapes_explicit = true;
-    // a split shape needs the per-part sums, sized with the grid buffers
-    if ((walk_shape_split(density_shape) || walk_shape_split(force_shape)) &&
-        e->walk.part_cap < e->cap)
-        e->grid_valid = false;
     return SPHK_OK;
 }
 

@@ -92,11 +92,8 @@ constexpr int kNumWalkShapes = 9;  // launch shapes selectable per walk (see wal
 const char* walk_shape_name(int v);
 // Parts of a chunk's candidate columns (corners, edges, centre with the outer ring).
 constexpr int kParts = 3;
-// Shapes that walk each chunk with three wavefronts, one per part of its candidate columns;
-// they need the per-part sums of WalkBuffers.
-constexpr bool walk_shape_split(int v) { return v == 5 || v == 6; }
 // Shapes an engine uses until the caller sets its own: below kSplitBelow particles the
-// single-wavefront walk leaves most of the GPU idle and the split seg32_waves4 is faster;
+// single-wavefront walk leaves most of the GPU idle and the team seg32_waves4 is faster;
 // above, seg24_waves4 for the density walk and pp16_waves4 for the force walk (the fastest
 // pair on the 1M dam break on MI355X).
 constexpr int kShapeSmall = 6;
@@ -128,20 +125,6 @@ struct WalkBuffers {
     size_t chunk_cap = 0;
     uint32_t max_words = 0;       // stride of mask and wj0 (kMaxWords or kMinWords)
     size_t col_cap = 0;
-    // per-part sums of the split shapes, [3][part_cap] by sorted slot (allocated only
-    // while a split shape is selected)
-    float* part_acc = nullptr;     // density sums
-    uint32_t* part_cnt = nullptr;  // neighbour counts
-    float4* part_force = nullptr;  // [3][part_cap][2]: pressure sum, viscosity sum
-    size_t part_cap = 0;
-};
-
-// Device view of the per-part sums.
-struct PartSums {
-    float* acc;
-    uint32_t* cnt;
-    float4* force;
-    size_t cap;
 };
 
 // Scene lookups by binary search over the scene table (few scenes; uniform per wave where

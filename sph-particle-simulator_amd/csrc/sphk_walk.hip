@@ -196,36 +196,29 @@ __device__ __forceinline__ float density_run(BitWalk<kW>& bw, float4& q0, float4
     return acc;
 }
 
-// Density pass over one chunk (kSplit false: all parts; true: the part of this wavefront,
-// three wavefronts per chunk, the sums finished by k_density_finish).  As many wavefronts per
-// SIMD as the LDS allows (six with 24-word segments): the walk is VALU-bound (a few spills
-// outside the walk loops).
-// The split shapes serve small scenes, whose wavefronts are few: no occupancy target, so
-// their deeper read-ahead stays in registers.  The ping-pong shapes aim at what their LDS
+// Density pass over one chunk by one wavefront.  As many wavefronts per SIMD as the LDS
+// allows (six with 24-word segments): the walk is VALU-bound (a few spills outside the walk
+// loops).  The ping-pong shapes aim at what their LDS
 // allows (6 with two 12-word buffers, 4 with two 16-word ones).
-template <class Shape, bool kSplit, bool kCut>
-__global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(kSplit ? 1 : Shape::density_waves, 8))) void k_density_walk(
+template <class Shape, bool kCut>
+__global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(Shape::density_waves, 8))) void k_density_walk(
     const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
     const uint32_t* __restrict__ nitems,
     const float4* __restrict__ spm, const uint2* __restrict__ sq, float4* __restrict__ svr,
     ForceRow* __restrict__ rows, const uint32_t* __restrict__ skey,
     const uint32_t* __restrict__ cs, StepConsts c, const SceneGrid* __restrict__ scenes,
     uint32_t* __restrict__ gmask, uint32_t* __restrict__ gwj0, uint32_t* __restrict__ gnw,
-    uint32_t* __restrict__ gpart, PartSums ps) {
+    uint32_t* __restrict__ gpart) {
     constexpr int kSeg = Shape::seg;
     constexpr int kLds = Shape::lds_words;
-    static_assert(!(kSplit && Shape::pp), "ping-pong shapes walk a chunk with one wavefront");
     __shared__ uint32_t lmask_all[Shape::waves][kLds * 64];
     __shared__ uint32_t lwj0_all[Shape::waves][kLds];
     const uint32_t wave = uni(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t* lmask = lmask_all[wave];
     uint32_t* lwj0 = lwj0_all[wave];
-    const uint32_t units = kSplit ? uni(nitems[0]) * kParts : uni(nitems[0]);
-    const uint32_t wid = xcd_unit(units, Shape::waves, wave);
-    if (wid == ~0u) return;
-    const uint32_t item = kSplit ? wid / kParts : wid;
-    const int part = kSplit ? (int)(wid % kParts) : -1;
+    const uint32_t item = xcd_unit(uni(nitems[0]), Shape::waves, wave);
+    if (item == ~0u) return;
     Chunk ch;
     uint32_t s;
     bool active;
@@ -236,16 +229,16 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
     mfma_filter_begin(mf, ch, sq, qi, active, lane, c.qneg);
     WordTable wt;
     static_assert(kLds * 64 >= kTableWords, "the word table is built in the mask buffer");
-    const bool tab = word_table_build(wt, ch, cs, part, lane, lmask);
+    const bool tab = word_table_build(wt, ch, cs, -1, lane, lmask);
     init_sentinel<kLds>(lmask, lwj0, lane, c);
     uint32_t* const gm = gmask + (size_t)item * c.max_words * 64;
     uint32_t* const gj = gwj0 + (size_t)item * c.max_words;
-    if (lane == 0 && part <= 0) {
+    if (lane == 0) {
         gpart[item] = pack_parts(wt.ps1, wt.ps2);
         gnw[item] = (uint32_t)wt.total;
     }
     Cursor cu;
-    if (!tab) cursor_begin(cu, ch, cs, c, 0, part);
+    if (!tab) cursor_begin(cu, ch, cs, c);
     // per-part running sum `cur`, parts folded into `total` as (p0 + p1) + p2
     float total = 0.0f, cur = 0.0f;
     int cur_part = 0;
@@ -335,32 +328,20 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
                     : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
                                                  sl, seg_part, &mf);
             if (nw == 0) break;
-            if (!kSplit) {
-                for (; cur_part < seg_part; ++cur_part) {
-                    total = cur_part == 0 ? cur : total + cur;
-                    cur = 0.0f;
-                }
+            for (; cur_part < seg_part; ++cur_part) {
+                total = cur_part == 0 ? cur : total + cur;
+                cur = 0.0f;
             }
             wave_sync();
             if (!tab) store_words(c.max_words, seg_base, nw, lmask, lwj0, gm, gj, lane);
             BitWalk<kSeg> bw;
             bw.begin(sl.nonempty, lmask, lwj0, lane);
             const uint32_t steps = wave_max(sl.count);
-            if constexpr (kSplit)
-                cur = density_bits_deep<kCut, kSeg, kDeepAhead>(bw, steps, lmask, lwj0, lane, spm,
-                                                                pi, c, cur);
-            else
-                cur = density_bits<kCut>(bw, steps, lmask, lwj0, lane, spm, pi, c, cur);
+            cur = density_bits<kCut>(bw, steps, lmask, lwj0, lane, spm, pi, c, cur);
             seg_base += nw;
             wave_sync();
             if (tab ? ti >= wt.n : cu.done) break;
         }
-    }
-    if (kSplit) {
-        if (active) {
-            ps.acc[(size_t)part * ps.cap + s] = cur;
-        }
-        return;
     }
     for (; cur_part < kParts; ++cur_part) {
         total = cur_part == 0 ? cur : total + cur;
@@ -369,15 +350,187 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
     if (active) density_epilogue(total, pi, s, c, svr, rows);
 }
 
-// Finishes split density passes: per finite particle (sorted slots below the non-finite
-// bin), the three part sums in order, then the same epilogue as the single-wavefront pass.
-__global__ __launch_bounds__(256) void k_density_finish(
-    const float4* __restrict__ spm, float4* __restrict__ svr, ForceRow* __restrict__ rows,
-    const uint32_t* __restrict__ cs, StepConsts c, PartSums ps) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= cs[c.G]) return;
-    const float a0 = ps.acc[s], a1 = ps.acc[ps.cap + s], a2 = ps.acc[2 * ps.cap + s];
-    density_epilogue((a0 + a1) + a2, spm[s], s, c, svr, rows);
+// ---------------------------------------------------------------------------
+// Team walks (the "_split" shapes): one workgroup per chunk, for scenes whose chunks are fewer
+// than the GPU's SIMDs hold (10,000 particles: 178 chunks for 1,024 SIMDs), where a step
+// takes as long as its longest chunk.  A lone wavefront issues a dependent instruction every
+// 6 to 8 cycles, so a chunk's time is its instruction count: kTeam wavefronts share the candidate
+// words of the chunk (about 1,000 cycles each), then each part's pairs are walked by one
+// wavefront (a part's sum runs in candidate order) and the first one finishes the
+// particles from LDS.  Against three independent wavefronts per chunk and a finishing launch
+// per walk: a step of 2,145 particles 108 -> 96 us, of 10,000 126 -> 110 us, ten steps of 34,000
+// 1.36 -> 1.24 ms.  Eight wavefronts a team are slower from 10,000 particles on (two
+// workgroups a CU).
+// ---------------------------------------------------------------------------
+constexpr int kTeam = 4;
+
+// LDS rows of the team's words: a part's words in groups of kSeg - 1, each group followed by
+// the sentinel word of its walk.
+__device__ __forceinline__ int team_rows(int words, int group) {
+    return words + (words + group - 1) / group;
+}
+
+// The part's sum over the words of its cursor or its own table: chunks of more than kTableWords
+// words, one wavefront per part.
+template <class Shape, bool kCut>
+__device__ __forceinline__ float density_part_alone(
+    const Chunk& ch, MfmaFilter& mf, int part, const float4* __restrict__ spm,
+    const uint2* __restrict__ sq, const uint32_t* __restrict__ cs, const StepConsts& c, uint2 qi,
+    bool active, const float4& pi, uint32_t* __restrict__ gm, uint32_t* __restrict__ gj,
+    uint32_t* __restrict__ lmask, uint32_t* __restrict__ lwj0, uint32_t* __restrict__ scratch,
+    uint32_t lane) {
+    constexpr int kSeg = Shape::seg;
+    WordTable wt;
+    const bool tab = word_table_build(wt, ch, cs, part, lane, scratch);
+    init_sentinel<kSeg>(lmask, lwj0, lane, c);
+    Cursor cu;
+    if (!tab) cursor_begin(cu, ch, cs, c, 0, part);
+    float cur = 0.0f;
+    int seg_base = wt.first;
+    int ti = 0;
+    for (;;) {
+        SegLane sl;
+        int seg_part;
+        const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, qi, active, lmask, lwj0, gm, gj,
+                                                lane, sl, seg_part, mf)
+                           : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
+                                                        lane, sl, seg_part, &mf);
+        if (nw == 0) break;
+        wave_sync();
+        if (!tab) store_words(c.max_words, seg_base, nw, lmask, lwj0, gm, gj, lane);
+        BitWalk<kSeg> bw;
+        bw.begin(sl.nonempty, lmask, lwj0, lane);
+        cur = density_bits_deep<kCut, kSeg, kDeepAhead>(bw, wave_max(sl.count), lmask, lwj0, lane,
+                                                        spm, pi, c, cur);
+        seg_base += nw;
+        wave_sync();
+        if (tab ? ti >= wt.n : cu.done) break;
+    }
+    return cur;
+}
+
+template <class Shape, bool kCut>
+__global__ __launch_bounds__(64 * kTeam) void k_density_team(
+    const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
+    const uint32_t* __restrict__ nitems, const float4* __restrict__ spm,
+    const uint2* __restrict__ sq, float4* __restrict__ svr, ForceRow* __restrict__ rows,
+    const uint32_t* __restrict__ skey, const uint32_t* __restrict__ cs, StepConsts c,
+    const SceneGrid* __restrict__ scenes, uint32_t* __restrict__ gmask,
+    uint32_t* __restrict__ gwj0, uint32_t* __restrict__ gnw, uint32_t* __restrict__ gpart) {
+    constexpr int kSeg = Shape::seg;
+    constexpr int kGroup = kSeg - 1;
+    constexpr int kRows = kTableWords + kTableWords / kGroup + kParts;
+    static_assert(kTeam >= kParts && kRows >= kParts * kSeg, "one walker and its words per part");
+    __shared__ uint32_t lmask[kRows * 64];
+    __shared__ uint32_t lwj0[kRows];
+    __shared__ uint32_t scratch[kTeam][kTableWords];
+    __shared__ float lsum[kParts][64];
+    const uint32_t wave = uni(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t item = xcd_unit(uni(nitems[0]), 1u, 0u);
+    if (item == ~0u) return;
+    Chunk ch;
+    uint32_t s;
+    bool active;
+    float4 pi;
+    if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
+    const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
+    MfmaFilter mf;
+    mfma_filter_begin(mf, ch, sq, qi, active, lane, c.qneg);
+    WordTable wt;
+    const bool tab = word_table_build(wt, ch, cs, -1, lane, scratch[wave]);
+    uint32_t* const gm = gmask + (size_t)item * c.max_words * 64;
+    uint32_t* const gj = gwj0 + (size_t)item * c.max_words;
+    if (wave == 0 && lane == 0) {
+        gpart[item] = pack_parts(wt.ps1, wt.ps2);
+        gnw[item] = (uint32_t)wt.total;
+    }
+    float cur = 0.0f;
+    if (tab) {
+        const int n0 = wt.ps1, n1 = wt.ps2 - wt.ps1, n2 = wt.total - wt.ps2;
+        const int r1 = team_rows(n0, kGroup), r2 = r1 + team_rows(n1, kGroup);
+        auto row_of = [&](int w) {
+            const int l = w < wt.ps1 ? w : w < wt.ps2 ? w - wt.ps1 : w - wt.ps2;
+            return (w < wt.ps1 ? 0 : w < wt.ps2 ? r1 : r2) + l + l / kGroup;
+        };
+        auto form = [&](int w, auto&& verdicts) {
+            uint32_t j0, cnt;
+            word_table_entry(wt, w, j0, cnt);
+            const uint32_t word = verdicts(j0, cnt);
+            const int r = row_of(w);
+            lmask[r * 64 + lane] = word;
+            if (lane == 0) lwj0[r] = j0;
+            if (w < (int)c.max_words)
+                __builtin_nontemporal_store(word, &gm[(size_t)w * 64 + lane]);
+        };
+        if (mf.on) {
+            uint2 q[kAheadWords] = {};
+            auto request = [&](int w, uint2& r) {
+                if (w >= wt.total) return;
+                uint32_t j0, cnt;
+                word_table_entry(wt, w, j0, cnt);
+                r = mfma_filter_row(mf, sq, j0, cnt);
+            };
+#pragma unroll
+            for (int k = 0; k < kAheadWords; ++k) request((int)wave + k * kTeam, q[k]);
+            for (int w0 = (int)wave; w0 < wt.total; w0 += kAheadWords * kTeam) {
+#pragma unroll
+                for (int k = 0; k < kAheadWords; ++k) {
+                    const int w = w0 + k * kTeam;
+                    if (w < wt.total) {
+                        form(w, [&](uint32_t, uint32_t cnt) {
+                            const uint32_t word = mfma_filter_word(mf, q[k], cnt, lane);
+                            request(w + kAheadWords * kTeam, q[k]);
+                            return word;
+                        });
+                    }
+                }
+            }
+        } else {
+            for (int w = (int)wave; w < wt.total; w += kTeam)
+                form(w, [&](uint32_t j0, uint32_t cnt) {
+                    return valu_filter_word(sq, uni(j0), uni(cnt), qi, active, c.qneg);
+                });
+        }
+        if (wave == kTeam - 1) {
+            constexpr uint32_t kSlot = (1u << 27) - 1u;
+            const int stored = min(wt.total, (int)c.max_words);
+            if ((int)lane < stored) gj[lane] = wt.e0 & kSlot;
+            if ((int)lane + 64 < stored) gj[lane + 64u] = wt.e1 & kSlot;
+        }
+        __syncthreads();
+        if (wave < kParts) {
+            const int n = wave == 0 ? n0 : wave == 1 ? n1 : n2;
+            const int r0 = wave == 0 ? 0 : wave == 1 ? r1 : r2;
+            for (int g = 0; g * kGroup < n; ++g) {
+                const int m = min(kGroup, n - g * kGroup);
+                uint32_t* const lm = lmask + (r0 + g * kSeg) * 64;
+                uint32_t* const lj = lwj0 + r0 + g * kSeg;
+                SegLane sl = {0u, 0u};
+#pragma unroll 4
+                for (int w = 0; w < m; ++w) {
+                    const uint32_t word = lm[w * 64 + lane];
+                    sl.nonempty |= min(word, 1u) << w;
+                    sl.count += (uint32_t)__builtin_popcount(word);
+                }
+                lm[m * 64 + lane] = 0x80000000u;
+                if (lane == 0) lj[m] = c.pad_slot;
+                wave_sync();
+                BitWalk<kSeg> bw;
+                bw.begin(sl.nonempty, lm, lj, lane, 1u << m);
+                cur = density_bits_deep<kCut, kSeg, kDeepAhead>(bw, wave_max(sl.count), lm, lj,
+                                                                lane, spm, pi, c, cur);
+            }
+        }
+    } else if (wave < kParts) {
+        cur = density_part_alone<Shape, kCut>(ch, mf, (int)wave, spm, sq, cs, c, qi, active, pi,
+                                              gm, gj, lmask + wave * kSeg * 64,
+                                              lwj0 + wave * kSeg, scratch[wave], lane);
+    }
+    if (wave < kParts) lsum[wave][lane] = cur;
+    __syncthreads();
+    if (wave == 0 && active)
+        density_epilogue((lsum[0][lane] + lsum[1][lane]) + lsum[2][lane], pi, s, c, svr, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -522,11 +675,37 @@ __device__ __forceinline__ void fold_parts_reg(float (&t)[6], ForceSums& f, int 
     f = ForceSums();
 }
 
-// Force pass over one chunk (kSplit false: all parts; true: the part of this wavefront,
-// three wavefronts per chunk, finished by k_force_finish).  Shapes of 24 words and more keep
+// Loads a segment of `nw` stored words (from stored word `base` on) into LDS, with the lane's
+// summary.  All loads are issued before the first is used (a loop over nw would wait for each
+// load of its remainder in turn); slots past nw re-read word nw - 1 and are dropped.  The words
+// are read once: nontemporal loads keep them from evicting the neighbour rows from L2.
+template <int kSeg>
+__device__ __forceinline__ void load_words(const uint32_t* __restrict__ gmask,
+                                           const uint32_t* __restrict__ gwj0, size_t base, int nw,
+                                           uint32_t* __restrict__ lmask,
+                                           uint32_t* __restrict__ lwj0, uint32_t lane,
+                                           SegLane& sl) {
+    uint32_t wv[kSeg - 1];
+    sl.nonempty = 0;
+    sl.count = 0;
+#pragma unroll
+    for (int w = 0; w < kSeg - 1; ++w)
+        wv[w] = __builtin_nontemporal_load(&gmask[(base + (size_t)min(w, nw - 1)) * 64 + lane]);
+#pragma unroll
+    for (int w = 0; w < kSeg - 1; ++w) {
+        if (w < nw) {
+            lmask[w * 64 + lane] = wv[w];
+            sl.nonempty |= (wv[w] != 0u ? 1u : 0u) << w;
+            sl.count += (uint32_t)__builtin_popcount(wv[w]);
+        }
+    }
+    if ((int)lane < nw) lwj0[lane] = gwj0[base + lane];
+}
+
+// Force pass over one chunk by one wavefront.  Shapes of 24 words and more keep
 // the parts' running total in registers: their LDS, not their registers, limits occupancy,
 // and the 1.5 KB per wavefront it frees lets the 28-word shape run 5 wavefronts per SIMD.
-template <class Shape, bool kSplit, bool kCut>
+template <class Shape, bool kCut>
 __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(Shape::force_waves)))
 void k_force_walk(
     const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
@@ -536,30 +715,26 @@ void k_force_walk(
     const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sid,
     const uint32_t* __restrict__ cs, StepConsts c, const SceneGrid* __restrict__ scenes,
     const uint32_t* __restrict__ gmask, const uint32_t* __restrict__ gwj0,
-    const uint32_t* __restrict__ gnw, const uint32_t* __restrict__ gpart, PartSums ps,
+    const uint32_t* __restrict__ gnw, const uint32_t* __restrict__ gpart,
     const float* __restrict__ dt_dev, float dt_arg,
     float4* __restrict__ pm,
     float4* __restrict__ vel, float4* __restrict__ acc_out, float* __restrict__ rho_out,
     float* __restrict__ prs_out, unsigned long long* __restrict__ stats) {
     constexpr int kSeg = Shape::seg;
     constexpr int kLds = Shape::lds_words;
-    static_assert(!(kSplit && Shape::pp), "ping-pong shapes walk a chunk with one wavefront");
     __shared__ uint32_t lmask_all[Shape::waves][kLds * 64];
     __shared__ uint32_t lwj0_all[Shape::waves][kLds];
     const uint32_t wave = uni(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
-    constexpr bool kRegTot = !kSplit && !Shape::pp && kSeg >= 24;
-    constexpr bool kLdsTot = !kSplit && !kRegTot;
+    constexpr bool kRegTot = !Shape::pp && kSeg >= 24;
+    constexpr bool kLdsTot = !kRegTot;
     __shared__ float ltot_all[kLdsTot ? Shape::waves : 1][kLdsTot ? 6 * 64 : 1];
     float rtot[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     uint32_t* lmask = lmask_all[wave];
     uint32_t* lwj0 = lwj0_all[wave];
     float* ltot = ltot_all[kLdsTot ? wave : 0];
-    const uint32_t units = kSplit ? uni(nitems[0]) * kParts : uni(nitems[0]);
-    const uint32_t wid = xcd_unit(units, Shape::waves, wave);
-    if (wid == ~0u) return;
-    const uint32_t item = kSplit ? wid / kParts : wid;
-    const int part = kSplit ? (int)(wid % kParts) : -1;
+    const uint32_t item = xcd_unit(uni(nitems[0]), Shape::waves, wave);
+    if (item == ~0u) return;
     Chunk ch;
     uint32_t s;
     bool active;
@@ -583,13 +758,9 @@ void k_force_walk(
     const bool stored = total_words <= (int)c.max_words;
     const uint32_t pstarts = stored ? uni(gpart[item]) : 0u;
     Cursor cu;
-    if (!stored) cursor_begin(cu, ch, cs, c, 0, part);
-    // stored words of this wavefront: all, or those of its part
-    int seg_base = 0, words_end = total_words;
-    if (kSplit) {
-        seg_base = part_word_start(pstarts, part);
-        words_end = part_word_end(pstarts, part, total_words);
-    }
+    if (!stored) cursor_begin(cu, ch, cs, c);
+    int seg_base = 0;
+    const int words_end = total_words;
     if constexpr (Shape::pp) {
         // As in the density walk: segments are loaded into the newer buffer; one of the part
         // being walked joins the walk at once, one of the next part waits until every lane
@@ -619,21 +790,8 @@ void k_force_walk(
                         seg_part = part_of_word(seg_base, pstarts);
                         const int pend_end = part_word_end(pstarts, seg_part, total_words);
                         nw = min(kSeg - 1, pend_end - seg_base);
-                        const size_t base = (size_t)item * c.max_words + seg_base;
-                        uint32_t wv[kSeg - 1];
-#pragma unroll
-                        for (int w = 0; w < kSeg - 1; ++w)
-                            wv[w] = __builtin_nontemporal_load(
-                                &gmask[(base + (size_t)min(w, nw - 1)) * 64 + lane]);
-#pragma unroll
-                        for (int w = 0; w < kSeg - 1; ++w) {
-                            if (w < nw) {
-                                lm_new[w * 64 + lane] = wv[w];
-                                sl.nonempty |= (wv[w] != 0u ? 1u : 0u) << w;
-                                sl.count += (uint32_t)__builtin_popcount(wv[w]);
-                            }
-                        }
-                        for (int w = (int)lane; w < nw; w += 64) lj_new[w] = gwj0[base + w];
+                        load_words<kSeg>(gmask, gwj0, (size_t)item * c.max_words + seg_base, nw,
+                                         lm_new, lj_new, lane, sl);
                         seg_base += nw;
                     }
                     if (seg_base >= words_end) more = false;
@@ -693,61 +851,27 @@ void k_force_walk(
                 seg_part = part_of_word(seg_base, pstarts);
                 const int pend = part_word_end(pstarts, seg_part, total_words);
                 nw = min(kSeg - 1, pend - seg_base);
-                const size_t base = (size_t)item * c.max_words + seg_base;
-                sl.nonempty = 0;
-                sl.count = 0;
-                // all of the segment's word loads are issued before the first is used (a loop
-                // over nw would wait for each load of its remainder in turn); slots past nw
-                // re-read word nw - 1 and are dropped.  The words are read once: nontemporal
-                // loads keep them from evicting the neighbour rows from L2
-                uint32_t wv[kSeg - 1];
-    #pragma unroll
-                for (int w = 0; w < kSeg - 1; ++w)
-                    wv[w] = __builtin_nontemporal_load(
-                        &gmask[(base + (size_t)min(w, nw - 1)) * 64 + lane]);
-    #pragma unroll
-                for (int w = 0; w < kSeg - 1; ++w) {
-                    if (w < nw) {
-                        lmask[w * 64 + lane] = wv[w];
-                        sl.nonempty |= (wv[w] != 0u ? 1u : 0u) << w;
-                        sl.count += (uint32_t)__builtin_popcount(wv[w]);
-                    }
-                }
-                for (int w = (int)lane; w < nw; w += 64) lwj0[w] = gwj0[base + w];
+                load_words<kSeg>(gmask, gwj0, (size_t)item * c.max_words + seg_base, nw, lmask,
+                                 lwj0, lane, sl);
             } else {
                 nw = phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
                                           seg_part);
                 if (nw == 0) break;
             }
-            if (!kSplit) {
-                if (kRegTot)
-                    fold_parts_reg(rtot, f, seg_part - cur_part);
-                else
-                    fold_parts(ltot, lane, f, seg_part - cur_part);
-                cur_part = seg_part;
-            }
+            if (kRegTot)
+                fold_parts_reg(rtot, f, seg_part - cur_part);
+            else
+                fold_parts(ltot, lane, f, seg_part - cur_part);
+            cur_part = seg_part;
             wave_sync();
             BitWalk<kSeg> bw;
             bw.begin(sl.nonempty, lmask, lwj0, lane);
-            if constexpr (kSplit)
-                force_bits_deep<kSeg, kCut, kDeepAhead>(bw, wave_max(sl.count), lmask, lwj0, lane,
-                                                        rows, pi, vi, p_quarter, c, f, cnt);
-            else
-                force_bits<kSeg, kCut>(bw, wave_max(sl.count), lmask, lwj0, lane, rows, pi, vi,
-                                       p_quarter, c, f, cnt);
+            force_bits<kSeg, kCut>(bw, wave_max(sl.count), lmask, lwj0, lane, rows, pi, vi,
+                                   p_quarter, c, f, cnt);
             seg_base += nw;
             wave_sync();
             if (!stored && cu.done) break;
         }
-    }
-    if (kSplit) {
-        if (active) {
-            float4* out = ps.force + 2 * ((size_t)part * ps.cap + s);
-            out[0] = make_float4(f.fp.x, f.fp.y, f.fp.z, 0.0f);
-            out[1] = make_float4(f.fv.x, f.fv.y, f.fv.z, 0.0f);
-            ps.cnt[(size_t)part * ps.cap + s] = cnt;
-        }
-        return;
     }
     if (stats) add_nbr_stats(cnt, stats, lane);
     if (kRegTot)
@@ -767,46 +891,103 @@ void k_force_walk(
                    acc_out, rho_out, prs_out);
 }
 
-// Finishes split force passes: per finite particle, the three part sums in order, then the
-// same epilogue as the single-wavefront pass.
-__global__ __launch_bounds__(256) void k_force_finish(
-    const float4* __restrict__ spm, const float4* __restrict__ svr,
+// Force pass over one chunk by a team of two wavefronts (see k_density_team): the first walks
+// part 0, the second parts 1 and 2 (the ring two columns out is nearly always empty); the first
+// folds the parts' sums from LDS and finishes the particles.  Two teams in one workgroup of four
+// wavefronts were slower (ten steps of 34,000 particles 1.24 -> 1.33 ms: coarser workgroups
+// spread the chunks less evenly over the CUs).
+constexpr int kForceTeam = 2;
+
+template <class Shape, bool kCut>
+__global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
+    const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
+    const uint32_t* __restrict__ nitems, const float4* __restrict__ spm,
+    const uint2* __restrict__ sq, const float4* __restrict__ svr,
+    const ForceRow* __restrict__ rows, const uint32_t* __restrict__ skey,
     const uint32_t* __restrict__ sid, const uint32_t* __restrict__ cs, StepConsts c,
-    const SceneGrid* __restrict__ scenes, PartSums ps, const float* __restrict__ dt_dev,
-    float dt_arg, float4* __restrict__ pm, float4* __restrict__ vel,
-    float4* __restrict__ acc_out, float* __restrict__ rho_out, float* __restrict__ prs_out,
+    const SceneGrid* __restrict__ scenes, const uint32_t* __restrict__ gmask,
+    const uint32_t* __restrict__ gwj0, const uint32_t* __restrict__ gnw,
+    const uint32_t* __restrict__ gpart, const float* __restrict__ dt_dev, float dt_arg,
+    float4* __restrict__ pm, float4* __restrict__ vel, float4* __restrict__ acc_out,
+    float* __restrict__ rho_out, float* __restrict__ prs_out,
     unsigned long long* __restrict__ stats) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = s < cs[c.G];
-    if (stats) {
-        const uint32_t cnt =
-            active ? ps.cnt[s] + ps.cnt[ps.cap + s] + ps.cnt[2 * ps.cap + s] : 0u;
-        add_nbr_stats(cnt, stats, threadIdx.x & 63u);
+    constexpr int kSeg = Shape::seg;
+    __shared__ uint32_t lmask_all[kForceTeam][kSeg * 64];
+    __shared__ uint32_t lwj0_all[kForceTeam][kSeg];
+    __shared__ float lsum[kParts][6][64];
+    __shared__ uint32_t lcnt[64];
+    const uint32_t wave = uni(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t* lmask = lmask_all[wave];
+    uint32_t* lwj0 = lwj0_all[wave];
+    const uint32_t item = xcd_unit(uni(nitems[0]), 1u, 0u);
+    if (item == ~0u) return;
+    Chunk ch;
+    uint32_t s;
+    bool active;
+    float4 pi;
+    if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
+    const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
+    init_sentinel<kSeg>(lmask, lwj0, lane, c);
+    const float4 vr = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 1.f);
+    const float3 vi = make_float3(vr.x, vr.y, vr.z);
+    const float rho_i = vr.w;
+    const float P_i = c.k_gas * (rho_i - c.rho0);
+    const float p_quarter = 0.25f * P_i;
+    const int total_words = (int)uni(gnw[item]);
+    const bool stored = total_words <= (int)c.max_words;
+    const uint32_t pstarts = stored ? uni(gpart[item]) : 0u;
+    uint32_t cnt = 0;
+    for (int part = (int)wave; part < (wave == 0 ? 1 : kParts); ++part) {
+        ForceSums f;
+        Cursor cu;
+        int w = 0, end = 0;
+        if (stored) {
+            w = part_word_start(pstarts, part);
+            end = part_word_end(pstarts, part, total_words);
+        } else {
+            cursor_begin(cu, ch, cs, c, 0, part);
+        }
+        for (;;) {
+            int nw, seg_part;
+            SegLane sl;
+            if (stored) {
+                if (w >= end) break;
+                nw = min(kSeg - 1, end - w);
+                load_words<kSeg>(gmask, gwj0, (size_t)item * c.max_words + w, nw, lmask, lwj0,
+                                 lane, sl);
+                w += nw;
+            } else {
+                nw = phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
+                                          seg_part);
+                if (nw == 0) break;
+            }
+            wave_sync();
+            BitWalk<kSeg> bw;
+            bw.begin(sl.nonempty, lmask, lwj0, lane);
+            force_bits_deep<kSeg, kCut, kDeepAhead>(bw, wave_max(sl.count), lmask, lwj0, lane,
+                                                    rows, pi, vi, p_quarter, c, f, cnt);
+            wave_sync();
+        }
+        const float v[6] = {f.fp.x, f.fp.y, f.fp.z, f.fv.x, f.fv.y, f.fv.z};
+#pragma unroll
+        for (int k = 0; k < 6; ++k) lsum[part][k][lane] = v[k];
     }
+    if (wave == 1) lcnt[lane] = cnt;
+    __syncthreads();
+    if (wave != 0) return;
+    if (stats) add_nbr_stats(cnt + lcnt[lane], stats, lane);
     if (!active) return;
     // ((0 + part 0) + part 1) + part 2, as the single-wavefront walk folds them
-    float t[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float t[6];
 #pragma unroll
-    for (int p = 0; p < kParts; ++p) {
-        const float4* in = ps.force + 2 * ((size_t)p * ps.cap + s);
-        const float4 a = in[0], b = in[1];
-        t[0] = t[0] + a.x;
-        t[1] = t[1] + a.y;
-        t[2] = t[2] + a.z;
-        t[3] = t[3] + b.x;
-        t[4] = t[4] + b.y;
-        t[5] = t[5] + b.z;
-    }
+    for (int k = 0; k < 6; ++k)
+        t[k] = ((0.0f + lsum[0][k][lane]) + lsum[1][k][lane]) + lsum[2][k][lane];
     ForceSums tot;
     tot.fp = make_float3(t[0], t[1], t[2]);
     tot.fv = make_float3(t[3], t[4], t[5]);
-    const float4 pi = spm[s];
-    const float4 vr = svr[s];
-    const float P_i = c.k_gas * (vr.w - c.rho0);
-    const uint32_t id = sid[s];
-    force_epilogue(tot, pi, make_float3(vr.x, vr.y, vr.z), vr.w, P_i, s,
-                   scenes[scene_of_particle(scenes, c.nscenes, id)], c, sid, dt_dev, dt_arg, pm,
-                   vel, acc_out, rho_out, prs_out);
+    force_epilogue(tot, pi, vi, rho_i, P_i, s, scenes[ch.scene], c, sid, dt_dev, dt_arg, pm, vel,
+                   acc_out, rho_out, prs_out);
 }
 
 // Particles with a non-finite coordinate (dense index G) have no neighbour, not even
@@ -1042,35 +1223,26 @@ const char* walk_shape_name(int v) {
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.  The grid is
 // padded to a multiple of 8 and sized for the most chunks a step can have (the host does not
 // know the count, which the chunk list leaves on the device); each XCD walks one contiguous
-// eighth of the chunks that exist (xcd_unit), whose candidate columns overlap.  A split shape
-// runs three wavefronts per chunk (consecutive, so mostly in one workgroup).
-template <class Shape>
-static uint32_t grid_for(uint32_t chunks, bool split = false) {
-    const uint32_t waves = split ? chunks * (uint32_t)kParts : chunks;
-    uint32_t blocks = (waves + Shape::waves - 1) / Shape::waves;
+// eighth of the chunks that exist (xcd_unit), whose candidate columns overlap.  A team (split)
+// shape runs one workgroup per chunk.
+static uint32_t grid_for(uint32_t chunks, uint32_t per_block) {
+    const uint32_t blocks = (chunks + per_block - 1) / per_block;
     return (blocks + kXcds - 1) / kXcds * kXcds;
 }
 
-// CALL sees the shape as type S and the split flag as constexpr kS.
-#define SPHK_DISPATCH_SHAPE(v, CALL)     \
-    switch (v) {                         \
-        case 0: { using S = Shape0; constexpr bool kS = false; CALL; break; } \
-        case 1: { using S = Shape1; constexpr bool kS = false; CALL; break; } \
-        case 2: { using S = Shape2; constexpr bool kS = false; CALL; break; } \
-        case 3: { using S = Shape3; constexpr bool kS = false; CALL; break; } \
-        case 5: { using S = Shape0; constexpr bool kS = true; CALL; break; } \
-        case 6: { using S = Shape1; constexpr bool kS = true; CALL; break; } \
-        case 7: { using S = Shape5; constexpr bool kS = false; CALL; break; } \
-        case 8: { using S = Shape6; constexpr bool kS = false; CALL; break; } \
-        default: { using S = Shape4; constexpr bool kS = false; CALL; break; } \
+// CALL sees the shape as type S; TEAM, for the split shapes, likewise.
+#define SPHK_DISPATCH_SHAPE(v, CALL, TEAM)  \
+    switch (v) {                            \
+        case 0: { using S = Shape0; CALL; break; } \
+        case 1: { using S = Shape1; CALL; break; } \
+        case 2: { using S = Shape2; CALL; break; } \
+        case 3: { using S = Shape3; CALL; break; } \
+        case 5: { using S = Shape0; TEAM; break; } \
+        case 6: { using S = Shape1; TEAM; break; } \
+        case 7: { using S = Shape5; CALL; break; } \
+        case 8: { using S = Shape6; CALL; break; } \
+        default: { using S = Shape4; CALL; break; } \
     }
-
-static hipError_t part_sums(const WalkBuffers& wb, uint32_t n, int shape, PartSums* ps) {
-    *ps = PartSums{wb.part_acc, wb.part_cnt, wb.part_force, wb.part_cap};
-    if (walk_shape_split(shape) && (!wb.part_acc || wb.part_cap < n))
-        return hipErrorInvalidValue;  // split shapes need per-part sums for every particle
-    return hipSuccess;
-}
 
 hipError_t launch_density_walk(const WalkBuffers& wb, const float4* spm, const uint2* sq,
                                float4* svr,
@@ -1079,25 +1251,21 @@ hipError_t launch_density_walk(const WalkBuffers& wb, const float4* spm, const u
                                const StepConsts& c, const SceneGrid* scenes, int shape,
                                hipStream_t st) {
     if (n == 0) return hipSuccess;
-    PartSums ps;
-    if (hipError_t err = part_sums(wb, n, shape, &ps)) return err;
     const uint32_t chunks = max_chunks(n, c);
-#define SPHK_DENSITY_LAUNCH(CUT)                                                            \
-    SPHK_DISPATCH_SHAPE(shape, hipLaunchKernelGGL((k_density_walk<S, kS, CUT>),               \
-                                                  dim3(grid_for<S>(chunks, kS)),             \
-                                                  dim3(S::threads), 0, st, wb.items, wb.desc, \
-                                                  wb.nitems, spm, sq, svr, rows, skey,       \
-                                                  cell_start, c, scenes, wb.mask, wb.wj0,    \
-                                                  wb.nwords, wb.pstarts, ps))
+#define SPHK_DENSITY_KERNEL(KERNEL, CUT, PER_BLOCK, THREADS)                                  \
+    hipLaunchKernelGGL((KERNEL<S, CUT>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), 0, \
+                       st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, cell_start, \
+                       c, scenes, wb.mask, wb.wj0, wb.nwords, wb.pstarts)
+#define SPHK_DENSITY_LAUNCH(CUT)                                                             \
+    SPHK_DISPATCH_SHAPE(shape, SPHK_DENSITY_KERNEL(k_density_walk, CUT, S::waves, S::threads), \
+                        SPHK_DENSITY_KERNEL(k_density_team, CUT, 1, 64 * kTeam))
     if (c.cut) {
         SPHK_DENSITY_LAUNCH(true);
     } else {
         SPHK_DENSITY_LAUNCH(false);
     }
 #undef SPHK_DENSITY_LAUNCH
-    if (walk_shape_split(shape))
-        hipLaunchKernelGGL(k_density_finish, dim3((n + 255) / 256), dim3(256), 0, st, spm, svr,
-                           rows, cell_start, c, ps);
+#undef SPHK_DENSITY_KERNEL
     return hipGetLastError();
 }
 
@@ -1110,27 +1278,22 @@ hipError_t launch_force_walk(const WalkBuffers& wb, const float4* spm, const uin
                              float4* vel, float4* acc, float* rho, float* prs, int shape,
                              unsigned long long* nbr_stats, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    PartSums ps;
-    if (hipError_t err = part_sums(wb, n, shape, &ps)) return err;
     const uint32_t chunks = max_chunks(n, c);
-#define SPHK_FORCE_LAUNCH(CUT)                                                              \
-    SPHK_DISPATCH_SHAPE(shape, hipLaunchKernelGGL((k_force_walk<S, kS, CUT>),                 \
-                                                  dim3(grid_for<S>(chunks, kS)),             \
-                                                  dim3(S::threads), 0, st, wb.items, wb.desc, \
-                                                  wb.nitems, spm, sq, svr, rows, skey, sid,  \
-                                                  cell_start, c, scenes, wb.mask, wb.wj0,    \
-                                                  wb.nwords, wb.pstarts, ps, dt_dev, dt, pm, \
-                                                  vel, acc, rho, prs, nbr_stats))
+#define SPHK_FORCE_KERNEL(KERNEL, CUT, PER_BLOCK, THREADS)                                    \
+    hipLaunchKernelGGL((KERNEL<S, CUT>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), 0, \
+                       st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, sid,       \
+                       cell_start, c, scenes, wb.mask, wb.wj0, wb.nwords, wb.pstarts, dt_dev, \
+                       dt, pm, vel, acc, rho, prs, nbr_stats)
+#define SPHK_FORCE_LAUNCH(CUT)                                                               \
+    SPHK_DISPATCH_SHAPE(shape, SPHK_FORCE_KERNEL(k_force_walk, CUT, S::waves, S::threads),    \
+                        SPHK_FORCE_KERNEL(k_force_team, CUT, 1, 64 * kForceTeam))
     if (c.cut) {
         SPHK_FORCE_LAUNCH(true);
     } else {
         SPHK_FORCE_LAUNCH(false);
     }
 #undef SPHK_FORCE_LAUNCH
-    if (walk_shape_split(shape))
-        hipLaunchKernelGGL(k_force_finish, dim3((n + 255) / 256), dim3(256), 0, st, spm, svr,
-                           sid, cell_start, c, scenes, ps, dt_dev, dt, pm, vel, acc, rho, prs,
-                           nbr_stats);
+#undef SPHK_FORCE_KERNEL
     return hipGetLastError();
 }
 
@@ -1145,10 +1308,12 @@ hipError_t launch_nbr_lists(const WalkBuffers& wb, const float4* spm, const uint
     // one wavefront per chunk in every shape (a split shape lists with its unsplit twin, a
     // ping-pong shape with the single-buffer shape of the same LDS size)
     const int base = shape == 5 ? 0 : shape == 6 ? 1 : shape == 7 ? 4 : shape == 8 ? 1 : shape;
-    SPHK_DISPATCH_SHAPE(base, hipLaunchKernelGGL(k_nbr_lists<S>, dim3(grid_for<S>(chunks)),
-                                                  dim3(S::threads), 0, st, wb.items, wb.desc, wb.nitems,
-                                                  spm, sq, skey, sid, cell_start, c, scenes,
-                                                  pass, count_by_id, offsets_by_id, idx));
+#define SPHK_LISTS_LAUNCH                                                                     \
+    hipLaunchKernelGGL(k_nbr_lists<S>, dim3(grid_for(chunks, S::waves)), dim3(S::threads), 0, \
+                       st, wb.items, wb.desc, wb.nitems, spm, sq, skey, sid, cell_start, c,   \
+                       scenes, pass, count_by_id, offsets_by_id, idx)
+    SPHK_DISPATCH_SHAPE(base, SPHK_LISTS_LAUNCH, SPHK_LISTS_LAUNCH);
+#undef SPHK_LISTS_LAUNCH
     return hipGetLastError();
 }
 

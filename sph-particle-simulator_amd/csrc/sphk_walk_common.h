@@ -141,7 +141,7 @@ __device__ __forceinline__ uint32_t uni(uint32_t v) { return __builtin_amdgcn_re
 
 constexpr uint32_t kXcds = 8;
 
-// Work unit of this wavefront (a chunk, or a chunk's part in the split walks) after the XCD
+// Work unit (chunk) of this wavefront or, with one per workgroup, of a team after the XCD
 // split: workgroups are dealt to the 8 XCDs in turn (block b runs on XCD b % 8), and XCD x
 // takes the x-th eighth of the `units` units that exist (one contiguous run, so neighbouring
 // chunks share its L2).  The grid is sized for the most units a step can have (see grid_for),
@@ -786,12 +786,15 @@ template <int kSeg>
 struct BitWalk {
     uint32_t m = 0, jb = 0, ne = 0;
     uint32_t mq = 0, jq = 0;  // the next non-empty word (or the sentinel), read ahead
+    uint32_t sent = 1u << (kSeg - 1);  // the sentinel word's bit, above every other word's
     // starts the walk of a segment whose non-empty words are `nonempty`; the first word is
     // read here, and each refill reads the one after, so a refill never waits for LDS
-    // `ne` always holds the sentinel word's bit, the highest, which is never cleared
+    // `ne` always holds the sentinel word's bit, which is never cleared
     __device__ __forceinline__ void begin(uint32_t nonempty, const uint32_t* __restrict__ lmask,
-                                          const uint32_t* __restrict__ lwj0, uint32_t lane) {
-        ne = nonempty | (1u << (kSeg - 1));
+                                          const uint32_t* __restrict__ lwj0, uint32_t lane,
+                                          uint32_t sentinel = 1u << (kSeg - 1)) {
+        sent = sentinel;
+        ne = nonempty | sent;
         m = 0u;
         fetch(lmask, lwj0, lane);
     }
@@ -800,7 +803,7 @@ struct BitWalk {
         const uint32_t w = (uint32_t)__builtin_ctz(ne);
         mq = lmask[w * 64 + lane];
         jq = lwj0[w];
-        ne = (ne & (ne - 1u)) | (1u << (kSeg - 1));
+        ne = (ne & (ne - 1u)) | sent;
     }
     // next candidate: its slot (kShift 0) or its byte offset in rows of 2^kShift bytes, so
     // a gather needs one 32-bit add-shift and a load with the row base in SGPRs
