@@ -295,11 +295,12 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
             // the next segment is made.
             const bool overlap = pp.nw_new != 0;
             if (!overlap && walk_part < 0) break;  // no segment at all
-            if ((overlap ? pp.older_steps() : pp.all_steps()) != 0) {
+            const uint32_t need = overlap ? pp.older_steps() : pp.all_steps();
+            if (need != 0) {
                 q0 = row_at(spm, pp.bw.template next<4>(lmask, lwj0, lane));
                 q1 = row_at(spm, pp.bw.template next<4>(lmask, lwj0, lane));
                 pp.walked(2);
-                const uint32_t steps = overlap ? pp.older_steps() : pp.all_steps();
+                const uint32_t steps = need > 2u ? need - 2u : 0u;
                 cur = density_run<kCut>(pp.bw, q0, q1, steps, lmask, lwj0, lane, spm, pi, c, cur);
                 pp.walked(steps);
                 cur = density_pair<kCut>(pi, q0, c, hh, cur);
@@ -739,8 +740,18 @@ void k_force_walk(
     uint32_t s;
     bool active;
     float4 pi;
-    if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
-    const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
+    const int total_words = (int)uni(gnw[item]);
+    const bool stored = total_words <= (int)c.max_words;
+    const uint32_t pstarts = uni(gpart[item]);
+    // (the whole chunk description serves the re-test alone)
+    uint2 qi = make_uint2(0u, 0u);
+    if (stored) {
+        load_targets(item, items, desc, spm, c, lane, ch, s, active, pi);
+    } else {
+        if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi))
+            return;
+        if (active) qi = sq[s];
+    }
     init_sentinel<kLds>(lmask, lwj0, lane, c);
     if (kLdsTot) {
 #pragma unroll
@@ -754,9 +765,6 @@ void k_force_walk(
     ForceSums f;
     uint32_t cnt = 0;  // neighbours of this wavefront's part(s)
     int cur_part = 0;
-    const int total_words = (int)uni(gnw[item]);
-    const bool stored = total_words <= (int)c.max_words;
-    const uint32_t pstarts = stored ? uni(gpart[item]) : 0u;
     Cursor cu;
     if (!stored) cursor_begin(cu, ch, cs, c);
     int seg_base = 0;
@@ -821,9 +829,10 @@ void k_force_walk(
             // A phase, as in the density walk: nothing stays in flight between phases.
             const bool overlap = pp.nw_new != 0;
             if (!overlap && walk_part < 0) break;  // no segment at all
-            if ((overlap ? pp.older_steps() : pp.all_steps()) != 0) {
+            const uint32_t need = overlap ? pp.older_steps() : pp.all_steps();
+            if (need != 0) {
                 request_ahead();
-                const uint32_t steps = overlap ? pp.older_steps() : pp.all_steps();
+                const uint32_t steps = need > kPPAhead ? need - kPPAhead : 0u;
                 force_run_n<kLds, kCut, kPPAhead>(pp.bw, a, b, steps, lmask, lwj0, lane, rows,
                                                   pi, vi, p_quarter, c, f, cnt);
                 pp.walked(steps);
@@ -926,17 +935,24 @@ __global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
     uint32_t s;
     bool active;
     float4 pi;
-    if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
-    const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
+    const int total_words = (int)uni(gnw[item]);
+    const bool stored = total_words <= (int)c.max_words;
+    const uint32_t pstarts = uni(gpart[item]);
+    // (the whole chunk description serves the re-test alone)
+    uint2 qi = make_uint2(0u, 0u);
+    if (stored) {
+        load_targets(item, items, desc, spm, c, lane, ch, s, active, pi);
+    } else {
+        if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi))
+            return;
+        if (active) qi = sq[s];
+    }
     init_sentinel<kSeg>(lmask, lwj0, lane, c);
     const float4 vr = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 1.f);
     const float3 vi = make_float3(vr.x, vr.y, vr.z);
     const float rho_i = vr.w;
     const float P_i = c.k_gas * (rho_i - c.rho0);
     const float p_quarter = 0.25f * P_i;
-    const int total_words = (int)uni(gnw[item]);
-    const bool stored = total_words <= (int)c.max_words;
-    const uint32_t pstarts = stored ? uni(gpart[item]) : 0u;
     uint32_t cnt = 0;
     for (int part = (int)wave; part < (wave == 0 ? 1 : kParts); ++part) {
         ForceSums f;

@@ -353,14 +353,40 @@ struct WordTable {
     int total;        // uniform: words of the whole chunk
 };
 
-// Inclusive prefix sums over lanes 0-31 and, separately, over lanes 32-63 (row shifts within
-// 16 lanes, then lane 15 of each first row added to the second).
+// The value of lane `src` under a DPP control, 0 where it has none.
+template <int kCtrl, int kRowMask = 0xf>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRowMask, 0xf, true);
+}
+// Wave max and wave sum (every lane active): row shifts within 16 lanes, then lane 15 of rows
+// 0 and 2 and lane 31 on to the next rows; lane 63 ends with the result.  Six dependent VALU
+// operations: by LDS permutes (130 cycles each) the maxima alone took 5 % of a force walk.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    v = max(v, dpp0<0x111>(v));
+    v = max(v, dpp0<0x112>(v));
+    v = max(v, dpp0<0x114>(v));
+    v = max(v, dpp0<0x118>(v));
+    v = max(v, dpp0<0x142, 0xa>(v));
+    v = max(v, dpp0<0x143, 0xc>(v));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+    v += dpp0<0x111>(v);
+    v += dpp0<0x112>(v);
+    v += dpp0<0x114>(v);
+    v += dpp0<0x118>(v);
+    v += dpp0<0x142, 0xa>(v);
+    v += dpp0<0x143, 0xc>(v);
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Inclusive prefix sums over lanes 0-31 and, separately, over lanes 32-63.
 __device__ __forceinline__ uint32_t half_wave_scan(uint32_t v) {
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, true);
+    v += dpp0<0x111>(v);
+    v += dpp0<0x112>(v);
+    v += dpp0<0x114>(v);
+    v += dpp0<0x118>(v);
+    v += dpp0<0x142, 0xa>(v);
     return v;
 }
 __device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
@@ -728,6 +754,24 @@ __device__ __forceinline__ int phase1_table(const WordTable& t, int& i,
     return nw;
 }
 
+// The chunk's particles alone, for walks over stored words: slots, scene and this lane's row.
+// Lanes past the chunk get NaN coordinates, so every test fails for them.
+__device__ __forceinline__ void load_targets(uint32_t item, const uint32_t* __restrict__ items,
+                                             const uint4* __restrict__ desc,
+                                             const float4* __restrict__ spm, const StepConsts& c,
+                                             uint32_t lane, Chunk& ch, uint32_t& s, bool& active,
+                                             float4& pi) {
+    ch.s0 = uni(items[item]);
+    const uint4 d = desc[item];
+    s = ch.s0 + lane;
+    const float4 row = spm[min(s, c.pad_slot)];
+    ch.s_end = uni(d.x);
+    ch.scene = uni(d.y);
+    active = s < ch.s_end;
+    const float qnan = __int_as_float(0x7fc00000);
+    pi = active ? row : make_float4(qnan, qnan, qnan, 0.0f);
+}
+
 // Builds the wave-uniform chunk description; returns false for an out-of-range item.
 // Lanes past the chunk get NaN coordinates, so every test fails for them.
 __device__ __forceinline__ bool load_chunk(uint32_t item, const uint32_t* __restrict__ items,
@@ -837,17 +881,14 @@ __device__ __forceinline__ void init_sentinel(uint32_t* __restrict__ lmask,
     if (lane == 0) lwj0[kSeg - 1] = c.pad_slot;
 }
 
-// Adds a wavefront's neighbour counts to the statistics slot of its workgroup.
+// Adds a wavefront's neighbour counts to the statistics slot of its workgroup.  (A count has
+// up to 27 bits: the halves of 16 bits are summed apart.)
 __device__ __forceinline__ void add_nbr_stats(uint32_t cnt, unsigned long long* stats,
                                               uint32_t lane) {
     stats += (blockIdx.x % kStatSlots) * kStatStride;
-    uint32_t mx = cnt;
-    unsigned long long sm = cnt;
-    for (int off = 32; off > 0; off >>= 1) {
-        uint32_t o = __shfl_xor(mx, off);
-        mx = o > mx ? o : mx;
-        sm += __shfl_xor(sm, off);
-    }
+    const uint32_t mx = wave_max(cnt);
+    const unsigned long long sm = (unsigned long long)wave_sum(cnt & 0xffffu) +
+                                  ((unsigned long long)wave_sum(cnt >> 16) << 16);
     if (lane == 0) {
         atomicMax(&stats[0], (unsigned long long)mx);
         atomicAdd(&stats[1], sm);
@@ -873,16 +914,6 @@ __device__ __forceinline__ void store_words(uint32_t max_words, int seg_base, in
 // from the front, the upper one from the back, each its share of the count, so every lane
 // walks continuously (no per-segment maxima) and the two never meet.
 // ---------------------------------------------------------------------------
-// Wave max of a per-lane count.
-__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const uint32_t o = __shfl_xor(x, off);
-        x = o > x ? o : x;
-    }
-    return uni(x);
-}
-
 // Ping-pong segments of a wavefront: the older segment's words at LDS words [0, kSeg - 1),
 // the newer one's at [kSeg, 2 kSeg - 1), the sentinel at word 2 kSeg - 1; the bit walk runs
 // over both (its set holds older words in bits 0.., newer ones in bits kSeg..), so a lane
