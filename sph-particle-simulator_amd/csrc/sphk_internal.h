@@ -93,13 +93,15 @@ const char* walk_shape_name(int v);
 // Parts of a chunk's candidate columns (corners, edges, centre with the outer ring).
 constexpr int kParts = 3;
 // Shapes an engine uses until the caller sets its own: below kSplitBelow particles the
-// single-wavefront walk leaves most of the GPU idle and the team seg32_waves4 is faster;
-// above, seg24_waves4 for the density walk and pp16_waves4 for the force walk (the fastest
-// pair on the 1M dam break on MI355X).
+// single-wavefront walk leaves SIMDs idle or runs one chunk more on some of them than on others,
+// and the team seg32_waves4 is faster; above, seg24_waves4 for the density walk and
+// pp16_waves4 for the force walk (the fastest pair on the 1M dam break on MI355X).  Steps with the
+// team shape against the pair: 68,000 particles 178 / 226 us, 99,000 209 / 233, 127,000
+// 254 / 278, 160,000 276 / 283, but 184,000 310 / 287 and five steps of 293,000 2.73 / 2.59 ms.
 constexpr int kShapeSmall = 6;
 constexpr int kShapeLargeDensity = 4;
 constexpr int kShapeLargeForce = 8;
-constexpr uint64_t kSplitBelow = 65536;
+constexpr uint64_t kSplitBelow = 163840;
 
 // Neighbour statistics (maximum and total of the neighbour counts) are kept in kStatSlots pairs,
 // one 128-byte line each, and folded when they are read.  Every wavefront of a force walk adds
