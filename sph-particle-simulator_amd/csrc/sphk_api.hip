@@ -543,15 +543,21 @@ int total_key_bits(uint64_t G) {
 int build_sorted(sphk_engine* e, const StepTail* tail) {
     const uint32_t n = (uint32_t)e->n;
     hipStream_t st = e->stream;
-    uint32_t* ko = nullptr;
-    uint32_t* vo = nullptr;
-    HIP_TRY(radix_sort_keys(e->pm, e->consts, e->d_scenes, e->uscal, e->keys, e->keys_alt, e->vals,
-                            e->vals_alt, e->hist, e->lookback, e->scan_scratch, n,
-                            total_key_bits(e->consts.G), &ko, &vo, st));
-    e->skey = ko;
-    e->sid = vo;
-    HIP_TRY(launch_gather_cells(e->pm, e->vel, e->sid, e->skey, n, e->consts.G, e->consts.qscale,
-                                e->sq, e->spm, e->svr, e->cell_start, st));
+    const int bits = total_key_bits(e->consts.G);
+    const bool small = small_build(n, e->consts);
+    if (small) {
+        e->skey = e->keys;
+        e->sid = e->vals;
+        HIP_TRY(launch_small_sort(e->pm, n, bits, e->consts, e->d_scenes, e->uscal, e->skey,
+                                  e->sid, e->cell_start, e->walk.items, e->walk.desc,
+                                  e->walk.nitems, st));
+    } else {
+        HIP_TRY(radix_sort_keys(e->pm, e->consts, e->d_scenes, e->uscal, e->keys, e->keys_alt,
+                                e->vals, e->vals_alt, e->hist, e->lookback, e->scan_scratch, n,
+                                bits, &e->skey, &e->sid, st));
+        HIP_TRY(launch_gather_cells(e->pm, e->vel, e->sid, e->skey, n, e->consts.G,
+                                    e->consts.qscale, e->sq, e->spm, e->svr, e->cell_start, st));
+    }
     StepTail t;
     if (tail) {
         t = *tail;
@@ -560,8 +566,14 @@ int build_sorted(sphk_engine* e, const StepTail* tail) {
         t.sid = e->sid;
         t.n = n;
     }
-    HIP_TRY(launch_chunks(e->cell_start, e->consts, e->d_scenes, e->walk.colcnt, e->scan_scratch,
-                          e->walk.items, e->walk.desc, e->walk.nitems, tail ? &t : nullptr, st));
+    if (small)
+        HIP_TRY(launch_gather_rows(e->pm, e->vel, e->sid, n, e->consts.qscale, e->sq, e->spm,
+                                   e->svr, e->cell_start, e->consts, e->d_scenes,
+                                   tail ? &t : nullptr, st));
+    else
+        HIP_TRY(launch_chunks(e->cell_start, e->consts, e->d_scenes, e->walk.colcnt,
+                              e->scan_scratch, e->walk.items, e->walk.desc, e->walk.nitems,
+                              tail ? &t : nullptr, st));
     e->sorted_valid = true;
     return SPHK_OK;
 }

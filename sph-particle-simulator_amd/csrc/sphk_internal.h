@@ -159,6 +159,12 @@ __device__ __forceinline__ uint32_t scene_of_particle(const SceneGrid* __restric
     return lo;
 }
 
+// The value of the lane a DPP control selects, 0 where it selects none.
+template <int kCtrl, int kRowMask = 0xf>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRowMask, 0xf, true);
+}
+
 // Exclusive prefix of v over the 256 threads of a workgroup (all threads call it); *total, if
 // given, receives the workgroup's sum.  lds_waves: 4 words of LDS.
 __device__ __forceinline__ uint32_t block_exclusive_scan_256(uint32_t v, uint32_t* lds_waves,
@@ -179,6 +185,27 @@ __device__ __forceinline__ uint32_t block_exclusive_scan_256(uint32_t v, uint32_
     }
     if (total) *total = tot;
     return wbase + x - v;
+}
+
+// Quantized coordinate of the candidate filter: floor(x * qscale) modulo 2^32, computed in
+// FP64 (exact for |x * qscale| < 2^52; 0 for non-finite or larger values, whose particles
+// are never candidates).
+__device__ __forceinline__ uint32_t quantize(float x, double qscale) {
+    const double v = floor((double)x * qscale);
+    if (!(fabs(v) < 4503599627370496.0)) return 0u;
+    return (uint32_t)(v - 4294967296.0 * floor(v * (1.0 / 4294967296.0)));
+}
+
+// Items and descriptions of one column's chunks, its slots [r.x, r.y), from item `o` on.
+__device__ __forceinline__ void column_items(uint2 r, uint32_t scene, const SceneGrid& g,
+                                             uint32_t col, uint32_t o,
+                                             uint32_t* __restrict__ items,
+                                             uint4* __restrict__ desc) {
+    const uint32_t rx = (col - g.col_base) / (uint32_t)g.ny, ry = (col - g.col_base) % (uint32_t)g.ny;
+    for (uint32_t s = r.x; s < r.y; s += 64u) {
+        items[o] = s;
+        desc[o++] = make_uint4(min(s + 64u, r.y), scene, rx, ry);
+    }
 }
 
 // Device-side arguments of the step's last part for the particles of the non-finite bin
@@ -220,6 +247,25 @@ hipError_t launch_gather_cells(const float4* pm, const float4* vel, const uint32
                                const uint32_t* skey, uint32_t n, uint32_t G, double qscale,
                                uint2* sq, float4* spm, float4* svr, uint32_t* cell_start,
                                hipStream_t st);
+// The build of small scenes: at most kSmallBuildN particles on at most kSmallBuildCells cells (the
+// non-finite bin and the table's end among them).  One workgroup sorts them and writes sorted
+// keys and ids, the cell table and the chunk list; a second launch gathers the rows and, with
+// `tail`, steps the non-finite particles.  Steps with it against the radix sort's launches: 720
+// particles 69 / 80 us, 2,145 80 / 93, 6,156 96 / 104, 10,000 102 / 108, 12,193 110 / 113, 13,824
+// 112 / 111.
+constexpr uint32_t kSmallBuildN = 12288;
+constexpr uint32_t kSmallBuildCells = 8192;
+inline bool small_build(uint32_t n, const StepConsts& c) {
+    return n >= 1u && n <= kSmallBuildN && c.G <= kSmallBuildCells - 2u;
+}
+hipError_t launch_small_sort(const float4* pm, uint32_t n, int total_bits, const StepConsts& c,
+                             const SceneGrid* scenes, uint32_t* err_flag, uint32_t* skey,
+                             uint32_t* sid, uint32_t* cell_start, uint32_t* items, uint4* desc,
+                             uint32_t* nitems, hipStream_t st);
+hipError_t launch_gather_rows(const float4* pm, const float4* vel, const uint32_t* sid, uint32_t n,
+                              double qscale, uint2* sq, float4* spm, float4* svr,
+                              const uint32_t* cell_start, const StepConsts& c,
+                              const SceneGrid* scenes, const StepTail* tail, hipStream_t st);
 uint32_t max_chunks(uint32_t n, const StepConsts& c);
 // chunk list of the sorted particles; with `tail`, also the non-finite particles' step
 hipError_t launch_chunks(const uint32_t* cell_start, const StepConsts& c, const SceneGrid* scenes,

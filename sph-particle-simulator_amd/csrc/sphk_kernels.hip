@@ -24,12 +24,12 @@ __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 // dense cell index per particle (caller order)
 // ---------------------------------------------------------------------------
 // Dense index of particle i at p: its cell in its scene's grid, or G (the non-finite bin) for a
-// non-finite coordinate.  A finite particle outside the grid's interior sets *err.
+// non-finite coordinate.  A finite particle outside the grid's interior sets `outside`.
 // kOne: a one-scene grid, whose geometry g0 is loaded once instead of looked up per particle.
 template <bool kOne>
 __device__ __forceinline__ uint32_t cell_key(const float4& p, uint32_t i, const StepConsts& c,
                                              const SceneGrid* __restrict__ scenes,
-                                             const SceneGrid& g0, uint32_t* __restrict__ err) {
+                                             const SceneGrid& g0, bool& outside) {
     uint32_t L = c.G;
     if (__builtin_isfinite(p.x) && __builtin_isfinite(p.y) && __builtin_isfinite(p.z)) {
         const SceneGrid& g = kOne ? g0 : scenes[scene_of_particle(scenes, c.nscenes, i)];
@@ -45,7 +45,7 @@ __device__ __forceinline__ uint32_t cell_key(const float4& p, uint32_t i, const 
             L = g.cell_base +
                 ((uint32_t)rx * (uint32_t)g.ny + (uint32_t)ry) * (uint32_t)g.nz + (uint32_t)rz;
         } else {
-            atomicOr(err, 1u);
+            outside = true;
         }
     }
     return L;
@@ -85,12 +85,13 @@ __global__ __launch_bounds__(kRadixThreads) void k_radix_upsweep(
             p[k] = idx < n ? pm[idx] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         const SceneGrid g0 = scenes[0];
+        bool outside = false;
         if (c.nscenes == 1) {
 #pragma unroll
             for (int k = 0; k < kRadixItems; ++k) {
                 const uint32_t idx = base + k * kRadixThreads + threadIdx.x;
                 if (idx < n) {
-                    key[k] = cell_key<true>(p[k], idx, c, scenes, g0, err);
+                    key[k] = cell_key<true>(p[k], idx, c, scenes, g0, outside);
                     keys_out[idx] = key[k];
                 }
             }
@@ -99,11 +100,12 @@ __global__ __launch_bounds__(kRadixThreads) void k_radix_upsweep(
             for (int k = 0; k < kRadixItems; ++k) {
                 const uint32_t idx = base + k * kRadixThreads + threadIdx.x;
                 if (idx < n) {
-                    key[k] = cell_key<false>(p[k], idx, c, scenes, g0, err);
+                    key[k] = cell_key<false>(p[k], idx, c, scenes, g0, outside);
                     keys_out[idx] = key[k];
                 }
             }
         }
+        if (outside) atomicOr(err, 1u);
     } else {
 #pragma unroll
         for (int k = 0; k < kRadixItems; ++k) {
@@ -483,17 +485,214 @@ hipError_t radix_sort_keys(const float4* pm, const StepConsts& c, const SceneGri
 }
 
 // ---------------------------------------------------------------------------
-// gather into cell-sorted order
+// Small scenes: sort, cell table and chunk list by one workgroup.  A step of a few thousand
+// particles is a row of short launches: histogram, scan, scatter, table and chunk list took
+// 5 launches and 27 us at 10,000 particles, most of it start-up, LDS counters of 2,048 digits and
+// waits for the launch before.  Here cell and id of a particle are one word (13 + 14 bits) that
+// stays in LDS from the first pass to the last; 6-bit digits make one counter a thread (16
+// wavefronts x 64 digits).  Wavefronts own consecutive runs, ranks within a wavefront come from
+// ballots: stable, the same order as the radix sort.  Loops stay rolled: the instructions come
+// from a cold cache (2,145 particles: 14 us unrolled, 10 rolled).
+// Bound by the latency of LDS and barriers in one workgroup (10,000 particles: 24 us), so by n:
+// the launches it replaces take less from kSmallBuildN on.
 // ---------------------------------------------------------------------------
-// Quantized coordinate of the candidate filter: floor(x * qscale) modulo 2^32, computed in
-// FP64 (exact for |x * qscale| < 2^52; 0 for non-finite or larger values, whose particles
-// are never candidates).
-__device__ __forceinline__ uint32_t quantize(float x, double qscale) {
-    const double v = floor((double)x * qscale);
-    if (!(fabs(v) < 4503599627370496.0)) return 0u;
-    return (uint32_t)(v - 4294967296.0 * floor(v * (1.0 / 4294967296.0)));
+constexpr uint32_t kSmallThreads = 1024;
+constexpr uint32_t kSmallWaves = kSmallThreads / 64;
+constexpr int kSmallBits = 6;
+constexpr uint32_t kSmallDigits = 1u << kSmallBits;
+constexpr int kSmallIdBits = 14;
+static_assert(kSmallWaves * kSmallDigits == kSmallThreads, "one counter per thread");
+static_assert(kSmallBuildN <= 1u << kSmallIdBits && kSmallBuildCells <= kSmallBuildN &&
+                  (uint64_t)kSmallBuildCells << kSmallIdBits <= 1ull << 32,
+              "cell and id in one word, the cell table in a key buffer");
+
+// Exclusive prefix (sum, or unsigned maximum) over the workgroup's 1,024 threads; all call it.
+// *total receives the whole.
+template <bool kMax>
+__device__ __forceinline__ uint32_t small_scan(uint32_t v, uint32_t* lw, uint32_t* total) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    auto op = [](uint32_t a, uint32_t b) { return kMax ? max(a, b) : a + b; };
+    uint32_t x = v;
+    x = op(x, dpp0<0x111>(x));
+    x = op(x, dpp0<0x112>(x));
+    x = op(x, dpp0<0x114>(x));
+    x = op(x, dpp0<0x118>(x));
+    x = op(x, dpp0<0x142, 0xa>(x));
+    x = op(x, dpp0<0x143, 0xc>(x));
+    const uint32_t left = dpp0<0x138>(x);  // the lane before's (wave shift by one)
+    __syncthreads();                       // lw may hold the values of the scan before
+    if (lane == 63u) lw[wave] = x;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kSmallWaves; ++k) {
+        const uint32_t t = lw[k];
+        before = op(before, k < wave ? t : 0u);
+        all = op(all, t);
+    }
+    if (total) *total = all;
+    return op(before, left);
 }
 
+template <bool kOne>
+__global__ __launch_bounds__(kSmallThreads) void k_small_sort(
+    const float4* __restrict__ pm, uint32_t n, int total_bits, StepConsts c,
+    const SceneGrid* __restrict__ scenes, uint32_t* __restrict__ err, uint32_t* __restrict__ skey,
+    uint32_t* __restrict__ sid, uint32_t* __restrict__ cs, uint32_t* __restrict__ items,
+    uint4* __restrict__ desc, uint32_t* __restrict__ nitems) {
+    __shared__ uint32_t buf[2][kSmallBuildN];
+    __shared__ uint32_t wc_all[2][kSmallThreads];  // this pass's and the next pass's counters
+    __shared__ uint32_t lw[kSmallWaves];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t per = (n + kSmallThreads - 1) / kSmallThreads;  // items a thread
+    const uint32_t base = wave * per * 64u + lane, end = min(n, (wave + 1u) * per * 64u);
+    const uint32_t run_inv = ~0u / (per * 64u) + 1u;  // x / (per * 64) for x < 2^14, by __umulhi
+    uint32_t* wc = wc_all[0];
+    uint32_t* wn = wc_all[1];
+    uint32_t* src = buf[0];
+    uint32_t* dst = buf[1];
+    const SceneGrid g0 = scenes[0];
+    wc[tid] = 0u;  // (this wavefront's own counters: digit `lane` of its run)
+    bool outside = false;
+    constexpr int kLoad = 4;  // rows in flight
+#pragma unroll 1
+    for (uint32_t i0 = base; i0 < end; i0 += kLoad * 64u) {
+        float4 p[kLoad];
+#pragma unroll
+        for (int k = 0; k < kLoad; ++k) p[k] = pm[min(i0 + (uint32_t)k * 64u, n - 1u)];
+#pragma unroll
+        for (int k = 0; k < kLoad; ++k) {
+            const uint32_t i = i0 + (uint32_t)k * 64u;
+            if (i < end) {
+                const uint32_t cell = cell_key<kOne>(p[k], i, c, scenes, g0, outside);
+                src[i] = cell << kSmallIdBits | i;
+                atomicAdd(&wc[wave * kSmallDigits + (cell & (kSmallDigits - 1u))], 1u);
+            }
+        }
+    }
+    if (outside) atomicOr(err, 1u);
+    for (int shift = kSmallIdBits;; shift += kSmallBits) {
+        const bool more = shift + kSmallBits < kSmallIdBits + total_bits;
+        __syncthreads();
+        wn[tid] = 0u;
+        // counters in digit-major order: thread t holds digit t / 16 of wavefront t % 16
+        uint32_t& ctr = wc[tid % kSmallWaves * kSmallDigits + tid / kSmallWaves];
+        const uint32_t first = small_scan<false>(ctr, lw, nullptr);
+        ctr = first;
+        __syncthreads();
+        uint32_t* const mine = wc + wave * kSmallDigits;  // next places of this wavefront's digits
+        // (every lane stays in the loop: the ballots need the run's 64 lanes together)
+#pragma unroll 1
+        for (uint32_t k = 0; k < per; ++k) {
+            const uint32_t i = base + k * 64u;
+            const bool valid = i < end;
+            const uint32_t v = valid ? src[i] : 0u;
+            const uint32_t d = (v >> shift) & (kSmallDigits - 1u);
+            const uint32_t next = mine[d];
+            const uint64_t all = __ballot(valid);
+            uint32_t lo = 0u, hi = 0u;  // lanes whose digit differs
+#pragma unroll
+            for (int b = 0; b < kSmallBits; ++b) {
+                const uint32_t m = (uint32_t)((int32_t)(d << (31 - b)) >> 31);
+                const uint64_t bal = __ballot(m != 0u);
+                lo |= (uint32_t)bal ^ m;
+                hi |= (uint32_t)(bal >> 32) ^ m;
+            }
+            lo = (uint32_t)all & ~lo;
+            hi = (uint32_t)(all >> 32) & ~hi;
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+            if (valid) {
+                const uint32_t to = next + below;
+                dst[to] = v;
+                if (below == 0u) mine[d] = next + (uint32_t)(__popc(lo) + __popc(hi));
+                if (more)
+                    atomicAdd(&wn[__umulhi(to, run_inv) * kSmallDigits +
+                                  ((v >> (shift + kSmallBits)) & (kSmallDigits - 1u))], 1u);
+            }
+        }
+        __syncthreads();
+        uint32_t* t = src;
+        src = dst;
+        dst = t;
+        t = wc;
+        wc = wn;
+        wn = t;
+        if (!more) break;
+    }
+    // cell table, in the free buffer: cells[c] is the end of cell c's particles (0: none), and
+    // the first slot with a key of at least c the largest end before c
+    uint32_t* const cells = dst;
+    const uint32_t ncells = c.G + 2u;
+#pragma unroll 1
+    for (uint32_t i = tid; i < ncells; i += kSmallThreads) cells[i] = 0u;
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t i = tid; i < n; i += kSmallThreads) {
+        const uint32_t v = src[i], cell = v >> kSmallIdBits;
+        skey[i] = cell;
+        sid[i] = v & ((1u << kSmallIdBits) - 1u);
+        if (i + 1u == n || src[min(i + 1u, n - 1u)] >> kSmallIdBits != cell) cells[cell] = i + 1u;
+    }
+    __syncthreads();
+    const uint32_t cper = (ncells + kSmallThreads - 1) / kSmallThreads;
+    const uint32_t c0 = min(ncells, tid * cper), c1 = min(ncells, c0 + cper);
+    uint32_t mx = 0;
+#pragma unroll 1
+    for (uint32_t i = c0; i < c1; ++i) mx = max(mx, cells[i]);
+    uint32_t run = small_scan<true>(mx, lw, nullptr);
+#pragma unroll 1
+    for (uint32_t i = c0; i < c1; ++i) {
+        const uint32_t e = cells[i];
+        cells[i] = run;
+        cs[i] = run;
+        run = max(run, e);
+    }
+    __syncthreads();
+    // chunk list: per column, ceil(particles / 64) chunks
+    const uint32_t colper = (c.ncols + kSmallThreads - 1) / kSmallThreads;
+    const uint32_t col0 = min(c.ncols, tid * colper), col1 = min(c.ncols, col0 + colper);
+    auto column = [&](uint32_t col, uint32_t& scene, SceneGrid& g) {
+        scene = kOne ? 0u : scene_of_col(scenes, c.nscenes, col);
+        g = kOne ? g0 : scenes[scene];
+        const uint32_t f = g.cell_base + (col - g.col_base) * (uint32_t)g.nz;
+        return make_uint2(cells[f], cells[f + (uint32_t)g.nz]);
+    };
+    uint32_t chunks = 0, scene;
+    SceneGrid g;
+#pragma unroll 1
+    for (uint32_t col = col0; col < col1; ++col) {
+        const uint2 r = column(col, scene, g);
+        chunks += (r.y - r.x + 63u) / 64u;
+    }
+    uint32_t total;
+    run = small_scan<false>(chunks, lw, &total);
+    if (tid == 0) nitems[0] = total;
+#pragma unroll 1
+    for (uint32_t col = col0; col < col1; ++col) {
+        const uint2 r = column(col, scene, g);
+        column_items(r, scene, g, col, run, items, desc);
+        run += (r.y - r.x + 63u) / 64u;
+    }
+}
+
+hipError_t launch_small_sort(const float4* pm, uint32_t n, int total_bits, const StepConsts& c,
+                             const SceneGrid* scenes, uint32_t* err_flag, uint32_t* skey,
+                             uint32_t* sid, uint32_t* cell_start, uint32_t* items, uint4* desc,
+                             uint32_t* nitems, hipStream_t st) {
+    if (c.nscenes == 1)
+        hipLaunchKernelGGL(k_small_sort<true>, dim3(1), dim3(kSmallThreads), 0, st, pm, n,
+                           total_bits, c, scenes, err_flag, skey, sid, cell_start, items, desc,
+                           nitems);
+    else
+        hipLaunchKernelGGL(k_small_sort<false>, dim3(1), dim3(kSmallThreads), 0, st, pm, n,
+                           total_bits, c, scenes, err_flag, skey, sid, cell_start, items, desc,
+                           nitems);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// gather into cell-sorted order
+// ---------------------------------------------------------------------------
 // One launch, two independent parts that need only the sorted keys and ids: workgroups below
 // `gather_blocks` gather particle s into sorted order, the rest fill the cell table
 // cs[c] = first sorted slot with key >= c, for c in [0, G + 1] (binary search per cell).

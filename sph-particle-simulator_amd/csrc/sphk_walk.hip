@@ -50,18 +50,6 @@ __global__ __launch_bounds__(256) void k_chunk_count(const uint32_t* __restrict_
     cnt[col] = (b - a + 63u) / 64u;
 }
 
-// Items and descriptions of one column's chunks, its slots [r.x, r.y), from item `o` on.
-__device__ __forceinline__ void column_items(uint2 r, uint32_t scene, const SceneGrid& g,
-                                             uint32_t col, uint32_t o,
-                                             uint32_t* __restrict__ items,
-                                             uint4* __restrict__ desc) {
-    const uint32_t rx = (col - g.col_base) / (uint32_t)g.ny, ry = (col - g.col_base) % (uint32_t)g.ny;
-    for (uint32_t s = r.x; s < r.y; s += 64u) {
-        items[o] = s;
-        desc[o++] = make_uint4(min(s + 64u, r.y), scene, rx, ry);
-    }
-}
-
 __global__ __launch_bounds__(256) void k_chunk_fill(const uint32_t* __restrict__ cs, StepConsts c,
                                                     const SceneGrid* __restrict__ scenes,
                                                     const uint32_t* __restrict__ offs,
@@ -1007,9 +995,28 @@ __global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
 }
 
 // Particles with a non-finite coordinate (dense index G) have no neighbour, not even
-// themselves: rho = m W(0), a = (0, g, 0); they are integrated and clamped like the rest.  The
-// bin holds the sorted slots [cs[G], n); workgroup `b` of `nb` takes every nb-th run of 256.
-// Workgroup 0 also advances the simulation time (time_dev, if given) by dt.
+// themselves: rho = m W(0), a = (0, g, 0); they are integrated and clamped like the rest.
+__device__ __forceinline__ void nonfinite_particle(const StepTail& t, const float4& pi,
+                                                   const float4& vi, uint32_t id, float dt,
+                                                   const StepConsts& c,
+                                                   const SceneGrid* __restrict__ scenes) {
+    const float rho_i = pi.w * c.w0;
+    const float P_i = c.k_gas * (rho_i - c.rho0);
+    const float3 a = final_accel(make_float3(0.f, 0.f, 0.f), make_float3(0.f, 0.f, 0.f), pi.w,
+                                 rho_i, c);
+    float3 v = make_float3(vi.x, vi.y, vi.z);
+    float4 p = pi;
+    const SceneGrid& g = scenes[scene_of_particle(scenes, c.nscenes, id)];
+    integrate_clamp(p, v, a, dt, c, g.lo, g.hi);
+    t.pm[id] = p;
+    t.vel[id] = make_float4(v.x, v.y, v.z, 0.0f);
+    t.acc[id] = make_float4(a.x, a.y, a.z, 0.0f);
+    t.rho[id] = rho_i;
+    t.prs[id] = P_i;
+}
+
+// The non-finite bin's step: it holds the sorted slots [cs[G], n); workgroup `b` of `nb` takes
+// every nb-th run of 256.  Workgroup 0 also advances the simulation time (time_dev, if given) by dt.
 __device__ __forceinline__ void nonfinite_particles(const StepTail& t,
                                                     const uint32_t* __restrict__ cs,
                                                     const StepConsts& c,
@@ -1017,24 +1024,8 @@ __device__ __forceinline__ void nonfinite_particles(const StepTail& t,
                                                     uint32_t b, uint32_t nb) {
     const float dt = t.dt_dev ? *t.dt_dev : t.dt;
     if (t.time_dev && b == 0 && threadIdx.x == 0) *t.time_dev = *t.time_dev + dt;
-    for (uint32_t s = cs[c.G] + b * blockDim.x + threadIdx.x; s < t.n; s += nb * blockDim.x) {
-        const float4 pi = t.spm[s];
-        const float4 vi = t.svr[s];
-        const float rho_i = pi.w * c.w0;
-        const float P_i = c.k_gas * (rho_i - c.rho0);
-        const float3 a = final_accel(make_float3(0.f, 0.f, 0.f), make_float3(0.f, 0.f, 0.f),
-                                     pi.w, rho_i, c);
-        float3 v = make_float3(vi.x, vi.y, vi.z);
-        float4 p = pi;
-        const uint32_t id = t.sid[s];
-        const SceneGrid& g = scenes[scene_of_particle(scenes, c.nscenes, id)];
-        integrate_clamp(p, v, a, dt, c, g.lo, g.hi);
-        t.pm[id] = p;
-        t.vel[id] = make_float4(v.x, v.y, v.z, 0.0f);
-        t.acc[id] = make_float4(a.x, a.y, a.z, 0.0f);
-        t.rho[id] = rho_i;
-        t.prs[id] = P_i;
-    }
+    for (uint32_t s = cs[c.G] + b * blockDim.x + threadIdx.x; s < t.n; s += nb * blockDim.x)
+        nonfinite_particle(t, t.spm[s], t.svr[s], t.sid[s], dt, c, scenes);
 }
 
 __global__ __launch_bounds__(256) void k_nonfinite_step(StepTail t, const uint32_t* __restrict__ cs,
@@ -1122,6 +1113,48 @@ __global__ __launch_bounds__(256) void k_chunk_list(const uint32_t* __restrict__
     const uint32_t scene = one ? 0u : scene_of_col(scenes, c.nscenes, col);
     const SceneGrid g = one ? g0 : scenes[scene];
     column_items(column_slots<true>(cs, scenes, c, g, col), scene, g, col, off[col], items, desc);
+}
+
+// Small scenes: rows in sorted order (see k_gather_cells); with kTail, the thread that gathers
+// a particle of the non-finite bin also steps it (nobody else reads its home rows).
+template <bool kTail>
+__global__ __launch_bounds__(256) void k_gather_rows(const float4* pm, const float4* vel,
+                                                     const uint32_t* __restrict__ sid, uint32_t n,
+                                                     double qscale, uint2* __restrict__ sq,
+                                                     float4* __restrict__ spm,
+                                                     float4* __restrict__ svr,
+                                                     const uint32_t* __restrict__ cs, StepConsts c,
+                                                     const SceneGrid* __restrict__ scenes,
+                                                     StepTail t) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t id = s < n ? sid[s] : 0u;
+    float4 p = pm[id], v = vel[id];
+    if constexpr (kTail) {
+        if (s == 0u && t.time_dev) *t.time_dev = *t.time_dev + (t.dt_dev ? *t.dt_dev : t.dt);
+    }
+    if (s >= n) return;
+    v.w = 0.0f;
+    spm[s] = p;
+    svr[s] = v;
+    const uint32_t qx = quantize(p.x, qscale), qy = quantize(p.y, qscale);
+    sq[s] = make_uint2((qx & 0xffffu) | (qy << 16), quantize(p.z, qscale));
+    if constexpr (kTail) {
+        if (s >= cs[c.G]) nonfinite_particle(t, p, v, id, t.dt_dev ? *t.dt_dev : t.dt, c, scenes);
+    }
+}
+
+hipError_t launch_gather_rows(const float4* pm, const float4* vel, const uint32_t* sid, uint32_t n,
+                              double qscale, uint2* sq, float4* spm, float4* svr,
+                              const uint32_t* cell_start, const StepConsts& c,
+                              const SceneGrid* scenes, const StepTail* tail, hipStream_t st) {
+    const dim3 grid((n + 255) / 256);
+    if (tail)
+        hipLaunchKernelGGL(k_gather_rows<true>, grid, dim3(256), 0, st, pm, vel, sid, n, qscale,
+                           sq, spm, svr, cell_start, c, scenes, *tail);
+    else
+        hipLaunchKernelGGL(k_gather_rows<false>, grid, dim3(256), 0, st, pm, vel, sid, n, qscale,
+                           sq, spm, svr, cell_start, c, scenes, StepTail{});
+    return hipGetLastError();
 }
 
 hipError_t launch_chunks(const uint32_t* cell_start, const StepConsts& c, const SceneGrid* scenes,

@@ -353,11 +353,6 @@ struct WordTable {
     int total;        // uniform: words of the whole chunk
 };
 
-// The value of lane `src` under a DPP control, 0 where it has none.
-template <int kCtrl, int kRowMask = 0xf>
-__device__ __forceinline__ uint32_t dpp0(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRowMask, 0xf, true);
-}
 // Wave max and wave sum (every lane active): row shifts within 16 lanes, then lane 15 of rows
 // 0 and 2 and lane 31 on to the next rows; lane 63 ends with the result.  Six dependent VALU
 // operations: by LDS permutes (130 cycles each) the maxima alone took 5 % of a force walk.

@@ -68,3 +68,34 @@ def test_uploads_and_downloads_return_the_rows(sphk, n):
     np.testing.assert_array_equal(e.masses()[n:],
                                   np.full(m, sphk.default_params().particle_mass, np.float32))
     assert e.densities().shape == (n + 300,)
+
+
+@pytest.mark.parametrize("scenes", [1, 2])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1025, 4097, 12287, 12288, 12289])
+def test_small_build_equals_the_launches_it_replaces(sphk, n, scenes):
+    # Up to 12,288 particles on up to 8,190 cells are sorted, tabled and listed by one workgroup.
+    # The same particles in wider bounds have more cells and take the radix sort: from the second
+    # step on (the grid then covers the bounds) the two engines build differently, and
+    # walk the same pairs in the same order.  A pile-up of one cell, empty columns, particles
+    # with a NaN coordinate (their own bin, stepped by the gather) and two scenes.
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(0.12, 0.28, (n, 3)).astype(np.float32)
+    pos[: n // 3] = rng.uniform(0.20, 0.24, (n // 3, 3))
+    pos[n // 2 + 1 : n // 2 + 4, 1] = np.nan
+    vel = rng.normal(0, 0.1, (n, 3)).astype(np.float32)
+    out = []
+    for hi in (0.4, 2.0):
+        p = sphk.default_params(xmin=0, xmax=hi, ymin=0, ymax=hi, zmin=0, zmax=hi, formulation=1)
+        e = sphk.Engine(n, p)
+        e.upload(pos, vel)
+        if scenes == 2:
+            e.set_scenes(np.array([0, n // 2, n], np.uint64))
+        for _ in range(3):
+            e.step(1e-6)
+        offs, idx = e.neighbors()
+        cells = e.grid()[2]
+        assert (cells <= 8190) == (hi == 0.4), cells
+        out.append((e.positions(), e.velocities(), e.densities()[:n], e.accelerations(), offs,
+                    idx))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
