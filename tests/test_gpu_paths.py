@@ -99,3 +99,26 @@ def test_small_build_equals_the_launches_it_replaces(sphk, n, scenes):
                     idx))
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape", ["seg32_waves4_split", "seg24_waves4", "pp16_waves4"])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 33, 1000, 1025])
+def test_every_particle_its_own_chunk(sphk, n, shape):
+    # The walks' launches provide for at most n chunks: here every particle is alone in its
+    # (x, y) column, so there are exactly n.  Each has only itself as a neighbour: density
+    # m W(0), which the force rows and the integration then use.
+    side = 40
+    k = np.random.default_rng(n).permutation(side * side)[:n]
+    pos = np.stack([0.1 * (k // side) + 0.02, 0.1 * (k % side) + 0.02, 0.001 * (k % 7)], 1)
+    p = sphk.default_params(xmin=-1, xmax=5, ymin=-1, ymax=5, zmin=-1, zmax=1)
+    e = sphk.Engine(n, p)
+    e.upload(pos.astype(np.float32))
+    v = sphk.walk_shape_names().index(shape)
+    e.set_walk_shapes(v, v)
+    e.step(1e-4)
+    assert len(e.walk_words()[0]) == n
+    h, m = float(np.float32(p.smoothing_length)), float(np.float32(p.particle_mass))
+    w0 = m * (2.0 / 3.0) / (np.pi * h**3)
+    # one FP32 product each for sigma, W(0) and m W(0), and the spline's own two roundings
+    np.testing.assert_allclose(e.densities()[:n], w0, rtol=8 * 2.0**-24)
+    np.testing.assert_allclose(e.accelerations()[:, 1], -9.81, rtol=4 * 2.0**-24)
