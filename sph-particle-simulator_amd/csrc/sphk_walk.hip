@@ -10,9 +10,10 @@
 // Phase 1 (test): the chunk's candidate words (32 consecutive slots of one column) are
 //   visited in the cursor's order (parts, passes, columns: see kPasses), and each lane gets
 //   one bit per candidate from the conservative integer filter: on the matrix cores
-//   (mfma_filter_word, 32 candidates x 64 targets per word), or one candidate at a time for
-//   the whole wave (push_quant, candidate data through the scalar cache) in the force walk's
-//   re-test and the neighbour-list export.  `wj0[w]` is the sorted slot of the first candidate of
+//   (filter_word, 32 candidates x 64 targets per word), or one candidate at a time for
+//   the whole wave (push_quant) in the words that span too many z cells for them and, with the
+//   candidate data through the scalar cache, in the force walk's re-test and the
+//   neighbour-list export; the bits are the same.  `wj0[w]` is the sorted slot of the first candidate of
 //   word w.  Segments hold up to kSeg - 1 words and never span two parts.
 // Phase 2 (evaluate): every lane walks only its own set bits and evaluates the kernel for
 //   those pairs (pairs the filter let through beyond the radius weigh exactly zero).
@@ -249,8 +250,8 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
             if (pp.nw_new == 0 && !pend && more) {
                 SegLane sl;
                 int seg_part;
-                const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, qi, active, lm_new, lj_new,
-                                                        gm, gj, lane, sl, seg_part, mf)
+                const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, lm_new, lj_new, gm, gj,
+                                                        lane, sl, seg_part, mf)
                                    : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active,
                                                                 lm_new, lj_new, lane, sl,
                                                                 seg_part, &mf);
@@ -312,8 +313,7 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
             SegLane sl;
             int seg_part;
             const int nw =
-                tab ? phase1_table<kSeg>(wt, ti, sq, c, qi, active, lmask, lwj0, gm, gj, lane, sl,
-                                         seg_part, mf)
+                tab ? phase1_table<kSeg>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl, seg_part, mf)
                     : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
                                                  sl, seg_part, &mf);
             if (nw == 0) break;
@@ -380,8 +380,8 @@ __device__ __forceinline__ float density_part_alone(
     for (;;) {
         SegLane sl;
         int seg_part;
-        const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, qi, active, lmask, lwj0, gm, gj,
-                                                lane, sl, seg_part, mf)
+        const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl,
+                                                seg_part, mf)
                            : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
                                                         lane, sl, seg_part, &mf);
         if (nw == 0) break;
@@ -442,45 +442,15 @@ __global__ __launch_bounds__(64 * kTeam) void k_density_team(
             const int l = w < wt.ps1 ? w : w < wt.ps2 ? w - wt.ps1 : w - wt.ps2;
             return (w < wt.ps1 ? 0 : w < wt.ps2 ? r1 : r2) + l + l / kGroup;
         };
-        auto form = [&](int w, auto&& verdicts) {
-            uint32_t j0, cnt;
-            word_table_entry(wt, w, j0, cnt);
-            const uint32_t word = verdicts(j0, cnt);
-            const int r = row_of(w);
-            lmask[r * 64 + lane] = word;
-            if (lane == 0) lwj0[r] = j0;
-            if (w < (int)c.max_words)
-                __builtin_nontemporal_store(word, &gm[(size_t)w * 64 + lane]);
-        };
-        if (mf.on) {
-            uint2 q[kAheadWords] = {};
-            auto request = [&](int w, uint2& r) {
-                if (w >= wt.total) return;
-                uint32_t j0, cnt;
-                word_table_entry(wt, w, j0, cnt);
-                r = mfma_filter_row(mf, sq, j0, cnt);
-            };
-#pragma unroll
-            for (int k = 0; k < kAheadWords; ++k) request((int)wave + k * kTeam, q[k]);
-            for (int w0 = (int)wave; w0 < wt.total; w0 += kAheadWords * kTeam) {
-#pragma unroll
-                for (int k = 0; k < kAheadWords; ++k) {
-                    const int w = w0 + k * kTeam;
-                    if (w < wt.total) {
-                        form(w, [&](uint32_t, uint32_t cnt) {
-                            const uint32_t word = mfma_filter_word(mf, q[k], cnt, lane);
-                            request(w + kAheadWords * kTeam, q[k]);
-                            return word;
-                        });
-                    }
-                }
-            }
-        } else {
-            for (int w = (int)wave; w < wt.total; w += kTeam)
-                form(w, [&](uint32_t j0, uint32_t cnt) {
-                    return valu_filter_word(sq, uni(j0), uni(cnt), qi, active, c.qneg);
-                });
-        }
+        table_words<kTeam, true>(wt, mf, sq, (int)wave, wt.total, c.qneg, lane,
+                                 [&](uint32_t word, int w, uint32_t j0) {
+                                     const int r = row_of(w);
+                                     lmask[r * 64 + lane] = word;
+                                     if (lane == 0) lwj0[r] = j0;
+                                     if (w < (int)c.max_words)
+                                         __builtin_nontemporal_store(
+                                             word, &gm[(size_t)w * 64 + lane]);
+                                 });
         if (wave == kTeam - 1) {
             constexpr uint32_t kSlot = (1u << 27) - 1u;
             const int stored = min(wt.total, (int)c.max_words);

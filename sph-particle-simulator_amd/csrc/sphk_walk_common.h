@@ -487,30 +487,40 @@ __device__ __forceinline__ uint32_t push_quant(uint32_t word, uint2 a, uint2 b, 
 // one v_mfma_f32_32x32x16_f16 evaluates it for 32 candidates (rows) x 32 targets (columns):
 // K slots 0-2 hold b and -2a, slots 3-4 b.b as lo + 2048 hi against (1, 2048), slots 5-6
 // (1, 2048) against a.a - T - 1 as lo + 2048 hi, the rest zero.  Every operand is an integer of
-// magnitude <= 2048 (exact in f16) and every partial sum an integer below 2^24 (exact in the
-// FP32 accumulator) when all coordinates lie within +-1024 of the origin: the first target's
-// x, y (candidates are at most 2 cells + 1 unit away: |.| <= 769) and, in z, the middle of the
+// magnitude <= 2048, or even and <= 4096 (exact in f16), and every partial sum an integer below
+// 2^24 (exact in the FP32 accumulator).  The origin is the first target's x, y (candidates are
+// at most 2 cells + 1 unit away: |.| <= 769; targets |.| <= 257) and, in z, the middle of the
 // candidate cells (|.| <= 128 (zhi - zlo + 1) + 257: at most 5 candidate z cells).
 // Chunks of more z cells (sparse columns: the faces and the free surface of every scene) take
-// the z origin of each word in the middle of its first and last candidate and clamp both
-// sides' z to +-1023 of it.  Clamping brings no two points apart, so it can turn a far
-// candidate into a passing one, never a neighbour into a failing one.  Testing such chunks on
-// the VALU instead took 3 times the words' time, and with one wavefront per chunk they ended
-// the launch: a density walk of 184,000 particles 149 -> 106 us, of 1M 430 -> 389 us with this,
-// the word table by lanes and the words stored as they are formed.
-// Only chunks of 2^21 z cells and more, whose z differences could wrap around in 32 bits, use
-// the VALU test.  The verdicts equal the VALU test's but for far candidates, and those
-// add exactly zero.
+// the z origin of each word in the middle of its first and last candidate, and test the word
+// here if all its candidates lie within kWideReach of it (b.b <= 2048 2048 + 2047).  Targets are
+// clamped to +-kWideClamp: a clamped one is at least 258 units from every candidate before and
+// after, and 258^2 >= T + 1 (sqrt(T) < 257.8: 256 units a cell, see make_consts), so it fails
+// either way.  The sums stay below 2 1735 1993 + 2 2 769 257 + b.b + 1993^2 + 2 257^2 < 2^24.
+// A word that spans more (fewer than two or three particles a cell) is tested on the VALU.
+// The verdicts thus equal the VALU test's in every word: which pairs are walked, and a pair's
+// place in its target's order, do not depend on which unit tested them.  Only chunks of 180 z
+// cells and more (its 32-bit squares wrap around there) take the VALU for every word.
+// Every word of a wide chunk on the VALU took 3 times the words' time, and with one wavefront
+// per chunk such chunks ended the launch: a density walk of 184,000 particles 149 -> 106 us, of 1M
+// 430 -> 389 us with this, the word table by lanes and the words stored as they are formed.
 // ---------------------------------------------------------------------------
 typedef _Float16 sphk_half8 __attribute__((ext_vector_type(8)));
 typedef float sphk_f32x16 __attribute__((ext_vector_type(16)));
 
+constexpr int32_t kWideReach = 1735;   // largest |z| of a wide chunk's candidates tested here
+constexpr int32_t kWideClamp = 1993;   // its targets' z are clamped to +- this
+constexpr int32_t kWideApart = kWideClamp - kWideReach;
+static_assert((kWideReach * kWideReach + 2 * 769 * 769) >> 11 <= 2048 &&
+                  (kWideClamp * kWideClamp + 2 * 257 * 257) >> 11 <= 2048 && kWideClamp <= 2048,
+              "operands exact in f16");
+
 struct MfmaFilter {
-    bool on;             // uniform: tested on the matrix cores
     bool wide;           // uniform: more than 5 candidate z cells, a z origin per word
+    bool never;          // uniform: every word on the VALU
     uint32_t ox, oz;     // origin: packed x | y << 16 (16-bit wrap-around), z
-    sphk_short2 axy;     // this lane's target: x, y from the origin, its z, and
-    uint32_t qz;         //   x^2 + y^2 + qneg
+    sphk_short2 axy;     // this lane's target: x, y from the origin, its coordinates, and
+    uint2 qi;            //   x^2 + y^2 + qneg
     int32_t axy2;
     bool active;         // this lane has a target
     sphk_half8 b1, b2;   // B operands: targets 0-31 and 32-63 (lanes 0-31 hold them)
@@ -519,7 +529,7 @@ struct MfmaFilter {
 
 // The B operands for z origin mf.oz.
 __device__ __forceinline__ void mfma_filter_targets(MfmaFilter& mf, uint32_t lane) {
-    const int32_t az = min(max((int32_t)(mf.qz - mf.oz), -1023), 1023);
+    const int32_t az = min(max((int32_t)(mf.qi.y - mf.oz), -kWideClamp), kWideClamp);
     const int32_t aa = mf.axy2 + az * az;
     sphk_half8 p;
     p[0] = (_Float16)(-2 * (int32_t)mf.axy.x);
@@ -553,14 +563,14 @@ __device__ __forceinline__ void mfma_filter_begin(MfmaFilter& mf, const Chunk& c
                                                   const uint2* __restrict__ sq, uint2 qi,
                                                   bool active, uint32_t lane, int32_t qneg) {
     const int zspan = ch.zhi - ch.zlo;
-    mf.on = zspan < (1 << 21);
     mf.wide = zspan > 4;
+    mf.never = zspan >= 180 || qneg < -kWideApart * kWideApart;
     // (the first target is lane 0's)
     mf.ox = uni(qi.x);
     mf.oz = uni(qi.y) + (uint32_t)(128 * (ch.zlo + ch.zhi + 1 - 2 * ch.zfirst));
     mf.axy = __builtin_bit_cast(sphk_short2, qi.x) - __builtin_bit_cast(sphk_short2, mf.ox);
     mf.axy2 = __builtin_amdgcn_sdot2(mf.axy, mf.axy, qneg, false);
-    mf.qz = qi.y;
+    mf.qi = qi;
     mf.active = active;
     const uint32_t m = lane & 31u;
     mf.crow = 16u * ((m >> 2) & 1u) + 4u * (m >> 3) + (m & 3u);
@@ -574,17 +584,53 @@ __device__ __forceinline__ uint2 mfma_filter_row(const MfmaFilter& mf,
     return sq[j0 + min(mf.crow, cnt - 1u)];
 }
 
+// Verdict word of this lane's target over the `cnt` candidates from slot j0 on, on the VALU.
+__device__ __forceinline__ uint32_t valu_filter_word(const uint2* __restrict__ sq, uint32_t j0,
+                                                     uint32_t cnt, uint2 qi, bool active,
+                                                     int32_t qneg) {
+    const uint2* __restrict__ pb = sq + j0;  // uniform base: scalar loads
+    uint32_t word = 0;
+    if (cnt == 32u) {
+#pragma unroll
+        for (int k = 0; k < 32; ++k) word = push_quant(word, qi, pb[k], qneg);
+    } else {
+        for (uint32_t k = 0; k < cnt; ++k) word = push_quant(word, qi, pb[k], qneg);
+        word <<= (32u - cnt);
+    }
+    return active ? word : 0u;
+}
+
+// Verdict word of this lane's target over the word's `cnt` candidates on the VALU, from the rows
+// the lanes hold (the candidates 4 q .. 4 q + 3 are lanes 8 (q & 3) + 4 (q >> 2) and on).
+__device__ __forceinline__ uint32_t rows_filter_word(const MfmaFilter& mf, uint2 qb, uint32_t cnt,
+                                                     int32_t qneg) {
+    const uint32_t quads = (cnt + 3u) / 4u;
+    uint32_t word = 0;
+#pragma unroll 2
+    for (uint32_t q = 0; q < quads; ++q) {
+        const int l = (int)(8u * (q & 3u) + 4u * (q >> 2));
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            word = push_quant(word, mf.qi,
+                              make_uint2(lane_value(qb.x, l + k), lane_value(qb.y, l + k)), qneg);
+    }
+    word <<= 32u - 4u * quads;
+    return mf.active ? word & (~0u << (32u - cnt)) : 0u;
+}
+
 // Verdict word of this lane's target over the word's `cnt` candidates, candidate k at bit
-// 31 - k, like the VALU test (no bit for lanes without a target).  qb: this lane's row.
-__device__ __forceinline__ uint32_t mfma_filter_word(MfmaFilter& mf, uint2 qb, uint32_t cnt,
-                                                     uint32_t lane) {
+// 31 - k (no bit for lanes without a target).  qb: this lane's row of the word; wide: mf.wide.
+__device__ __forceinline__ uint32_t filter_word(MfmaFilter& mf, uint2 qb, uint32_t cnt,
+                                                int32_t qneg, uint32_t lane, bool wide) {
     int32_t bz;
-    if (mf.wide) {
+    if (wide) {
         // rows 0 and 31 (the last candidate) are lane 0's and lane 31's
         const uint32_t z0 = uni(qb.y), z1 = lane_value(qb.y, 31);
         mf.oz = z0 + (uint32_t)((int32_t)(z1 - z0) >> 1);
+        bz = (int32_t)(qb.y - mf.oz);
+        if (mf.never || __ballot(bz < -kWideReach || bz > kWideReach) != 0ull)
+            return rows_filter_word(mf, qb, cnt, qneg);
         mfma_filter_targets(mf, lane);
-        bz = min(max((int32_t)(qb.y - mf.oz), -1023), 1023);
     } else {
         bz = (int16_t)(qb.y - mf.oz);
     }
@@ -622,22 +668,6 @@ __device__ __forceinline__ uint32_t mfma_filter_word(MfmaFilter& mf, uint2 qb, u
     return word & (~0u << (32u - cnt));
 }
 
-// The same word on the VALU.
-__device__ __forceinline__ uint32_t valu_filter_word(const uint2* __restrict__ sq, uint32_t j0,
-                                                     uint32_t cnt, uint2 qi, bool active,
-                                                     int32_t qneg) {
-    const uint2* __restrict__ pb = sq + j0;  // uniform base: scalar loads
-    uint32_t word = 0;
-    if (cnt == 32u) {
-#pragma unroll
-        for (int k = 0; k < 32; ++k) word = push_quant(word, qi, pb[k], qneg);
-    } else {
-        for (uint32_t k = 0; k < cnt; ++k) word = push_quant(word, qi, pb[k], qneg);
-        word <<= (32u - cnt);
-    }
-    return active ? word : 0u;
-}
-
 // A formed word `w` of a segment: into LDS and the lane's summary.
 __device__ __forceinline__ void put_word(uint32_t word, int w, uint32_t* __restrict__ lmask,
                                          uint32_t lane, SegLane& sl) {
@@ -669,10 +699,12 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
         const uint32_t j0 = uni(cu.j);
         const uint32_t cnt = uni(min(32u, cu.end - j0));
         uint32_t word;
-        if (kMfma && mf->on)
-            word = mfma_filter_word(*mf, mfma_filter_row(*mf, sq, j0, cnt), cnt, lane);
-        else
+        if (kMfma) {
+            const uint2 qb = mfma_filter_row(*mf, sq, j0, cnt);
+            word = filter_word(*mf, qb, cnt, c.qneg, lane, mf->wide);
+        } else {
             word = valu_filter_word(sq, j0, cnt, qi, active, c.qneg);
+        }
         put_word(word, w, lmask, lane, sl);
         if (lane == 0) lwj0[w] = j0;
         cu.j = j0 + cu.step;
@@ -681,16 +713,63 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
     return w;
 }
 
+// The words of table entries first, first + kStride, ... below `end`, in turn to
+// put(word, entry, first slot).  The candidate rows of kAheadWords words are in flight.
+// kApart: wide chunks take a rolled loop of their own, so the unrolled one holds no test of
+// theirs (the team walks: a step of 2,145 particles 82 -> 80 us, of 10,000 103.5 -> 101.5); the
+// second copy of the product costs registers, which the walks of one wavefront per chunk don't
+// have (16 instead of 2 spilled, a step of 184,000 particles 285 -> 299 us).
+constexpr int kAheadWords = 4;
+template <int kStride, bool kApart, class Put>
+__device__ __forceinline__ void table_words(const WordTable& t, MfmaFilter& mf,
+                                            const uint2* __restrict__ sq, int first, int end,
+                                            int32_t qneg, uint32_t lane, Put&& put) {
+    uint2 q[kAheadWords] = {};
+    auto request = [&](int e, uint2& r) {
+        if (e >= end) return;
+        uint32_t j0, cnt;
+        word_table_entry(t, e, j0, cnt);
+        r = mfma_filter_row(mf, sq, j0, cnt);
+    };
+#pragma unroll
+    for (int k = 0; k < kAheadWords; ++k) request(first + k * kStride, q[k]);
+    if (kApart && mf.wide) {
+#pragma unroll 1
+        for (int e = first; e < end; e += kStride) {
+            uint32_t j0, cnt;
+            word_table_entry(t, e, j0, cnt);
+            const uint32_t word = filter_word(mf, q[0], cnt, qneg, lane, true);
+#pragma unroll
+            for (int k = 0; k + 1 < kAheadWords; ++k) q[k] = q[k + 1];
+            request(e + kAheadWords * kStride, q[kAheadWords - 1]);
+            put(word, e, j0);
+        }
+        return;
+    }
+    for (int e0 = first; e0 < end; e0 += kAheadWords * kStride) {
+#pragma unroll
+        for (int k = 0; k < kAheadWords; ++k) {
+            const int e = e0 + k * kStride;
+            if (e < end) {
+                uint32_t j0, cnt;
+                word_table_entry(t, e, j0, cnt);
+                const uint32_t word = filter_word(mf, q[k], cnt, qneg, lane, !kApart && mf.wide);
+                request(e + kAheadWords * kStride, q[k]);
+                put(word, e, j0);
+            }
+        }
+    }
+}
+
 // Phase 1 over the word table: the next segment of up to kSeg - 1 words from local entry `i`
 // (advanced), never past a part start.  Same words and order as phase1_segment.  The words go
 // to LDS and, from the registers that formed them, to the chunk's stored words (gm: its word
 // 0, `max_words` of them; nontemporal: the force walk reads them once, long after, and the rows
-// the walks gather should keep L2).  The candidate rows of kAheadWords words are in flight.
-constexpr int kAheadWords = 4;
+// the walks gather should keep L2).
 template <int kSeg>
 __device__ __forceinline__ int phase1_table(const WordTable& t, int& i,
                                             const uint2* __restrict__ sq, const StepConsts& c,
-                                            uint2 qi, bool active, uint32_t* __restrict__ lmask,
+                                            uint32_t* __restrict__ lmask,
                                             uint32_t* __restrict__ lwj0,
                                             uint32_t* __restrict__ gm,
                                             uint32_t* __restrict__ gj, uint32_t lane,
@@ -705,42 +784,15 @@ __device__ __forceinline__ int phase1_table(const WordTable& t, int& i,
     if (nw <= 0) return 0;
     const int stored = (int)c.max_words - g0;  // words of the segment the engine stores
     uint32_t jv = 0;                           // lane w: first slot of word w
-    auto store = [&](uint32_t word, int w) {
-        put_word(word, w, lmask, lane, sl);
-        if (w < stored) __builtin_nontemporal_store(word, &gm[(size_t)(g0 + w) * 64 + lane]);
-    };
-    if (mf.on) {
-        uint2 q[kAheadWords] = {};
-        auto request = [&](int w, uint2& r) {
-            uint32_t j0, cnt;
-            if (w >= nw) return;
-            word_table_entry(t, i + w, j0, cnt);
-            r = mfma_filter_row(mf, sq, j0, cnt);
-        };
-#pragma unroll
-        for (int k = 0; k < kAheadWords; ++k) request(k, q[k]);
-        for (int w0 = 0; w0 < nw; w0 += kAheadWords) {
-#pragma unroll
-            for (int k = 0; k < kAheadWords; ++k) {
-                const int w = w0 + k;
-                if (w < nw) {
-                    uint32_t j0, cnt;
-                    word_table_entry(t, i + w, j0, cnt);
-                    jv = lane == (uint32_t)w ? j0 : jv;
-                    const uint32_t word = mfma_filter_word(mf, q[k], cnt, lane);
-                    request(w + kAheadWords, q[k]);
-                    store(word, w);
-                }
-            }
-        }
-    } else {
-        for (int w = 0; w < nw; ++w) {
-            uint32_t j0, cnt;
-            word_table_entry(t, i + w, j0, cnt);
-            jv = lane == (uint32_t)w ? j0 : jv;
-            store(valu_filter_word(sq, uni(j0), uni(cnt), qi, active, c.qneg), w);
-        }
-    }
+    table_words<1, false>(t, mf, sq, i, i + nw, c.qneg, lane,
+                          [&](uint32_t word, int e, uint32_t j0) {
+                              const int w = e - i;
+                              jv = lane == (uint32_t)w ? j0 : jv;
+                              put_word(word, w, lmask, lane, sl);
+                              if (w < stored)
+                                  __builtin_nontemporal_store(
+                                      word, &gm[(size_t)(g0 + w) * 64 + lane]);
+                          });
     if ((int)lane < nw) {
         lwj0[lane] = jv;
         if ((int)lane < stored) gj[g0 + (int)lane] = jv;
