@@ -461,17 +461,21 @@ struct SegLane {
 };
 
 // Appends the quantized filter's verdict on one candidate to a 32-bit word: with
-// dX, dY (16-bit wrap-around) and dZ (24-bit) the differences of the quantized coordinates,
+// dX, dY (16-bit wrap-around) and dZ the differences of the quantized coordinates,
 // t = dX^2 + dY^2 + dZ^2 + qneg is negative exactly when the squared distance is at most T,
 // and word = 2 * word + sign(t).  Five VALU: packed 16-bit subtract, subtract, 24-bit
-// multiply-add, dot2, align-bit.  Wrap-around can only turn a far candidate into a passing
-// one, never a neighbour into a failing one.
+// multiply-add, dot2, align-bit.  kFar: dZ is clamped first (one more), for candidates 180 cells
+// and more away, whose square would wrap around in 32 bits and let them pass.
 typedef short sphk_short2 __attribute__((ext_vector_type(2)));
+constexpr int kFarCells = 180;  // (180 cells + 2 units)^2 < 2^31
+template <bool kFar>
 __device__ __forceinline__ uint32_t push_quant(uint32_t word, uint2 a, uint2 b, int32_t qneg) {
     const sphk_short2 dxy =
         __builtin_bit_cast(sphk_short2, a.x) - __builtin_bit_cast(sphk_short2, b.x);
-    const uint32_t dz = (uint32_t)(((int32_t)((a.y - b.y) << 8)) >> 8);
-    const int32_t t = __builtin_amdgcn_sdot2(dxy, dxy, (int32_t)(dz * dz + (uint32_t)qneg), false);
+    int32_t dz = (int32_t)(a.y - b.y);
+    if (kFar) dz = min(max(dz, -32767), 32767);
+    const int32_t t =
+        __builtin_amdgcn_sdot2(dxy, dxy, (int32_t)((uint32_t)__mul24(dz, dz) + (uint32_t)qneg), false);
     return __builtin_amdgcn_alignbit(word, (uint32_t)t, 31);
 }
 
@@ -499,8 +503,8 @@ __device__ __forceinline__ uint32_t push_quant(uint32_t word, uint2 a, uint2 b, 
 // either way.  The sums stay below 2 1735 1993 + 2 2 769 257 + b.b + 1993^2 + 2 257^2 < 2^24.
 // A word that spans more (fewer than two or three particles a cell) is tested on the VALU.
 // The verdicts thus equal the VALU test's in every word: which pairs are walked, and a pair's
-// place in its target's order, do not depend on which unit tested them.  Only chunks of 180 z
-// cells and more (its 32-bit squares wrap around there) take the VALU for every word.
+// place in its target's order, do not depend on which unit tested them.  Only chunks of 2^21 z
+// cells and more, whose z differences could wrap around, take the VALU for every word.
 // Every word of a wide chunk on the VALU took 3 times the words' time, and with one wavefront
 // per chunk such chunks ended the launch: a density walk of 184,000 particles 149 -> 106 us, of 1M
 // 430 -> 389 us with this, the word table by lanes and the words stored as they are formed.
@@ -518,6 +522,7 @@ static_assert((kWideReach * kWideReach + 2 * 769 * 769) >> 11 <= 2048 &&
 struct MfmaFilter {
     bool wide;           // uniform: more than 5 candidate z cells, a z origin per word
     bool never;          // uniform: every word on the VALU
+    bool far;            // uniform: kFarCells candidate z cells or more (see push_quant)
     uint32_t ox, oz;     // origin: packed x | y << 16 (16-bit wrap-around), z
     sphk_short2 axy;     // this lane's target: x, y from the origin, its coordinates, and
     uint2 qi;            //   x^2 + y^2 + qneg
@@ -564,7 +569,8 @@ __device__ __forceinline__ void mfma_filter_begin(MfmaFilter& mf, const Chunk& c
                                                   bool active, uint32_t lane, int32_t qneg) {
     const int zspan = ch.zhi - ch.zlo;
     mf.wide = zspan > 4;
-    mf.never = zspan >= 180 || qneg < -kWideApart * kWideApart;
+    mf.far = zspan >= kFarCells;
+    mf.never = zspan >= (1 << 21) || qneg < -kWideApart * kWideApart;
     // (the first target is lane 0's)
     mf.ox = uni(qi.x);
     mf.oz = uni(qi.y) + (uint32_t)(128 * (ch.zlo + ch.zhi + 1 - 2 * ch.zfirst));
@@ -592,9 +598,9 @@ __device__ __forceinline__ uint32_t valu_filter_word(const uint2* __restrict__ s
     uint32_t word = 0;
     if (cnt == 32u) {
 #pragma unroll
-        for (int k = 0; k < 32; ++k) word = push_quant(word, qi, pb[k], qneg);
+        for (int k = 0; k < 32; ++k) word = push_quant<true>(word, qi, pb[k], qneg);
     } else {
-        for (uint32_t k = 0; k < cnt; ++k) word = push_quant(word, qi, pb[k], qneg);
+        for (uint32_t k = 0; k < cnt; ++k) word = push_quant<true>(word, qi, pb[k], qneg);
         word <<= (32u - cnt);
     }
     return active ? word : 0u;
@@ -602,6 +608,7 @@ __device__ __forceinline__ uint32_t valu_filter_word(const uint2* __restrict__ s
 
 // Verdict word of this lane's target over the word's `cnt` candidates on the VALU, from the rows
 // the lanes hold (the candidates 4 q .. 4 q + 3 are lanes 8 (q & 3) + 4 (q >> 2) and on).
+template <bool kFar>
 __device__ __forceinline__ uint32_t rows_filter_word(const MfmaFilter& mf, uint2 qb, uint32_t cnt,
                                                      int32_t qneg) {
     const uint32_t quads = (cnt + 3u) / 4u;
@@ -611,8 +618,8 @@ __device__ __forceinline__ uint32_t rows_filter_word(const MfmaFilter& mf, uint2
         const int l = (int)(8u * (q & 3u) + 4u * (q >> 2));
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-            word = push_quant(word, mf.qi,
-                              make_uint2(lane_value(qb.x, l + k), lane_value(qb.y, l + k)), qneg);
+            word = push_quant<kFar>(
+                word, mf.qi, make_uint2(lane_value(qb.x, l + k), lane_value(qb.y, l + k)), qneg);
     }
     word <<= 32u - 4u * quads;
     return mf.active ? word & (~0u << (32u - cnt)) : 0u;
@@ -629,7 +636,8 @@ __device__ __forceinline__ uint32_t filter_word(MfmaFilter& mf, uint2 qb, uint32
         mf.oz = z0 + (uint32_t)((int32_t)(z1 - z0) >> 1);
         bz = (int32_t)(qb.y - mf.oz);
         if (mf.never || __ballot(bz < -kWideReach || bz > kWideReach) != 0ull)
-            return rows_filter_word(mf, qb, cnt, qneg);
+            return mf.far ? rows_filter_word<true>(mf, qb, cnt, qneg)
+                          : rows_filter_word<false>(mf, qb, cnt, qneg);
         mfma_filter_targets(mf, lane);
     } else {
         bz = (int16_t)(qb.y - mf.oz);

@@ -34,17 +34,10 @@ def _integer_test(pos):
     return x, int(np.floor(reach * reach))
 
 
-@pytest.mark.parametrize("shape", ["seg24_waves4", "seg16_waves4_split", "seg32_waves4_split",
-                                   "pp12_waves4"])
-@pytest.mark.parametrize("per_cell", [0.3, 1.0, 3.0, 6.0, 12.0])
-def test_words_of_sparse_columns_equal_the_integer_test(sphk, per_cell, shape):
-    # The matrix cores take a word whose candidates lie within six z cells or so, the VALU any
-    # other: bit by bit both are the integer test, so no pair beyond it is walked (its row, if
-    # not finite, would reach the sums) and the order of a target's pairs does not depend on
-    # which unit tested them.
-    pos = _column_scene(per_cell, int(10 * per_cell))
+def _check_words(sphk, pos, params, shape):
+    """Every stored bit against the integer test; the stored pairs and those within the radius."""
     n = len(pos)
-    e = sphk.Engine(n, _params(sphk))
+    e = sphk.Engine(n, params)
     e.upload(pos)
     names = sphk.walk_shape_names()
     e.set_walk_shapes(names.index(shape), names.index("seg32_waves4"))
@@ -81,7 +74,34 @@ def test_words_of_sparse_columns_equal_the_integer_test(sphk, per_cell, shape):
         pairs += int(got.sum())
         near += int((d2[got] <= 256 * 256).sum())
     assert wide > 0
+    return pairs, near
+
+
+@pytest.mark.parametrize("shape", ["seg24_waves4", "seg16_waves4_split", "seg32_waves4_split",
+                                   "pp12_waves4"])
+@pytest.mark.parametrize("per_cell", [0.3, 1.0, 3.0, 6.0, 12.0])
+def test_words_of_sparse_columns_equal_the_integer_test(sphk, per_cell, shape):
+    # The matrix cores take a word whose candidates lie within some z cells, the VALU any
+    # other: bit by bit both are the integer test, so no pair beyond it is walked (its row, if
+    # not finite, would reach the sums) and the order of a target's pairs does not depend on
+    # which unit tested them.
+    pairs, near = _check_words(sphk, _column_scene(per_cell, int(10 * per_cell)), _params(sphk),
+                               shape)
     assert pairs <= 1.06 * near, (pairs, near)
+
+
+@pytest.mark.parametrize("shape", ["seg24_waves4", "seg32_waves4_split"])
+@pytest.mark.parametrize("cells", [300, 65536])
+def test_words_of_tall_columns_equal_the_integer_test(sphk, cells, shape):
+    # Candidates so far apart that the square of their distance passes 2^31 units, or the
+    # distance itself 2^24: neither may wrap around into the radius.
+    rng = np.random.default_rng(cells)
+    top = cells * 0.04
+    ends = [rng.uniform([0.01, 0.01, z], [0.17, 0.17, z + 0.08], size=(400, 3)) for z in (0.0, top)]
+    between = rng.uniform([0.01, 0.01, 0.0], [0.17, 0.17, top], size=(1200, 3))
+    pos = np.concatenate(ends + [between]).astype(F32)
+    p = sphk.default_params(xmin=0, xmax=1, ymin=0, ymax=1, zmin=-1, zmax=top + 1)
+    _check_words(sphk, pos, p, shape)
 
 
 @pytest.mark.parametrize("shape", ["seg24_waves4", "seg32_waves4_split", "pp16_waves4"])
