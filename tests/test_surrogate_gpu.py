@@ -307,3 +307,53 @@ def test_gradient_of_ragged_batches(sphk, oracle, scenes, batch_chunks):
     again = e.surrogate_loss_grad(target, batch_seed=7, batch_chunks=batch_chunks)
     assert again[0] == loss
     np.testing.assert_array_equal(again[1], grad)
+
+
+def _bf16(x):
+    u = np.ascontiguousarray(x, dtype=F32).view(np.uint32).astype(np.uint64)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000).astype(np.uint32).view(F32)
+
+
+def _kernel_feature(r, inv_h):
+    """W(r) / W(0), q < 1, in the oracle's order of operations."""
+    q = r * inv_h
+    q2 = q * q
+    return F32(1.5) * ((F32(2) / F32(3) - q2) + F32(0.5) * q2 * q)
+
+
+def _kernel_feature_by_cubes(r, inv_h):
+    """The same by clamped cubes, which rounds differently."""
+    r64 = r.astype(np.float64)
+    u = (1.0 - np.float64(F32(0.5) * inv_h) * r64).astype(F32)
+    s = (1.0 - np.float64(inv_h) * r64).astype(F32)
+    return F32(2) * ((s * s).astype(np.float64) * (F32(-0.5) * s) + (u * u * u).astype(F32)).astype(F32)
+
+
+def test_backward_takes_the_features_of_the_forward(sphk):
+    # Two particles: both edges have the same kernel feature f, so column 7 of dW1 is f times
+    # db1, and the quotient shows the bf16 value that the backward pass used.  It is the value
+    # the forward pass (and the oracle) rounds to, at distances where another order of
+    # operations rounds to its neighbour (2^-8 away; the quotient is FP32 arithmetic).
+    p = sphk.default_params(xmin=0, xmax=1, ymin=0, ymax=1, zmin=0, zmax=1, formulation=1)
+    inv_h = F32(1) / F32(p.smoothing_length)
+    r = np.unique(np.linspace(0.0005, 0.003, 2500001).astype(F32))
+    ours, other = _bf16(_kernel_feature(r, inv_h)), _bf16(_kernel_feature_by_cubes(r, inv_h))
+    split = ours != other
+    split[1:-1] &= split[:-2] & split[2:]  # and one ulp of r to either side (sqrt)
+    where = np.nonzero(split[:-1])[0]
+    _, first = np.unique(ours[where], return_index=True)
+    where = where[first]
+    assert len(where) >= 4
+    e = sphk.Engine(2, p)
+    e.upload(np.zeros((2, 3), F32))
+    e.surrogate_init(seed=9)
+    _active_params(e, seed=2)
+    for k in where:
+        pos = np.array([[0, 0.5, 0.5], [r[k], 0.5, 0.5]], F32)
+        e.upload(pos, np.array([[0.3, -0.2, 0.1], [-0.1, 0.4, 0.2]], F32))
+        _, grad, mask = e.surrogate_loss_grad(np.array([[5, -7, 3], [2, 9, -4]], F32), 1, 4)
+        assert mask.all()
+        dw, db = grad[:1152].reshape(128, 9)[:, 7].astype(np.float64), grad[1152:1280].astype(np.float64)
+        on = np.abs(db) > 1e-3 * np.abs(db).max()
+        assert on.sum() > 20
+        np.testing.assert_allclose(dw[on] / db[on], float(ours[k]), rtol=2.0**-16)
