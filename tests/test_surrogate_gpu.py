@@ -357,3 +357,55 @@ def test_backward_takes_the_features_of_the_forward(sphk):
         on = np.abs(db) > 1e-3 * np.abs(db).max()
         assert on.sum() > 20
         np.testing.assert_allclose(dw[on] / db[on], float(ours[k]), rtol=2.0**-16)
+
+
+@pytest.mark.parametrize("kind", ["block", "cluster"])
+def test_macro_step_matches_oracle(sphk, oracle, scenes, kind):
+    # The macro-step's walk is its own instance of the forward pass (windows, operand order, kernel
+    # feature, sums): its accelerations against the oracle's network with the tolerances of
+    # test_forward_matches_oracle, the state against the macro-step formula in FP64.  Ragged
+    # chunks; in the cluster, targets with more non-empty words than one window surely holds
+    # (56 of them, and 16 more).
+    s = _moving_block(scenes, seed=8)
+    pos, vel, mass = s.pos, s.vel, np.full(s.n, 1e-3, F32)
+    if kind == "cluster":
+        rng = np.random.default_rng(1)
+        extra = rng.uniform([0.50, 0.10, 0.10], [0.55, 0.15, 0.15], (3000, 3)).astype(F32)
+        pos = np.concatenate([pos, extra])
+        vel = np.concatenate([vel, rng.normal(0, 0.3, extra.shape).astype(F32)])
+        mass = np.concatenate([mass, np.full(3000, 2e-5, F32)])
+    n = len(pos)
+    e = sphk.Engine(n, s.params(sphk, 1))
+    e.upload(pos, vel, mass)
+    e.surrogate_init(seed=6)
+    params = _active_params(e, seed=5)
+    items, nwords, _, mask = e.walk_words()
+    assert any((b - a) % 64 for a, b in zip(items, items[1:]))
+    if kind == "cluster":
+        full = [int((mask[c, : nwords[c]] != 0).sum(0).max()) for c in range(len(items))]
+        assert max(full) > 72
+    rho = e.surrogate_densities()
+    offs, idx = e.neighbors()
+    cfg = _cfg(oracle, e)
+    ref = oracle.sur_forward(cfg, params, pos, vel, rho, offs, idx) * cfg.acc_scale
+    dt = 2e-4
+    e.surrogate_macro_step(dt)
+    acc = e.accelerations()
+    rms = np.sqrt(np.mean(ref**2))
+    err = np.abs(acc - ref)
+    assert np.linalg.norm(acc - ref) / np.linalg.norm(ref) < 2e-3
+    assert np.quantile(err, 0.99) < 1e-3 * rms
+    assert err.max() < 2e-2 * rms
+    p = e.params()
+    T = float(F32(dt)) * e.surrogate_config().substeps
+    dk = float(F32(p.damping)) ** e.surrogate_config().substeps
+    v1 = dk * vel.astype(np.float64) + acc.astype(np.float64) * T
+    x1 = pos + 0.5 * T * (vel.astype(np.float64) + v1)
+    lo = np.array([p.xmin, p.ymin, p.zmin])
+    hi = np.array([p.xmax, p.ymax, p.zmax])
+    v1 = np.where((x1 < lo) | (x1 > hi), v1 * float(F32(-0.8)), v1)
+    # five roundings behind a velocity, three more behind a position
+    scale = np.abs(vel).max() + T * np.abs(acc).max()
+    np.testing.assert_allclose(e.velocities(), v1, rtol=0, atol=8 * 2.0**-24 * scale)
+    np.testing.assert_allclose(e.positions(), np.clip(x1, lo, hi), rtol=0, atol=8 * 2.0**-24)
+    np.testing.assert_array_equal(e.densities()[:n], rho)
