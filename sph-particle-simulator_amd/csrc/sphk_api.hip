@@ -475,8 +475,7 @@ int ensure_grid(sphk_engine* e) {
     e->consts.ncols = (uint32_t)ncols;
     e->consts.nscenes = (uint32_t)S;
     e->consts.pad_slot = (uint32_t)e->cap;
-    // chunk work lists and neighbour words: at most ceil(C/64) + one partial chunk per column
-    const uint64_t chunks = (e->cap + 63) / 64 + ncols;
+    const uint64_t chunks = max_chunks((uint32_t)e->cap, e->consts);
     WalkBuffers& wb = e->walk;
     if (chunks > wb.chunk_cap) {
         // every member is cleared as it is freed, so a failed allocation below leaves no

@@ -67,7 +67,10 @@ __global__ __launch_bounds__(256) void k_chunk_fill(const uint32_t* __restrict__
                  items, desc);
 }
 
-uint32_t max_chunks(uint32_t n, const StepConsts& c) { return (n + 63u) / 64u + c.ncols; }
+// Every column may end with a part-filled chunk, and every chunk holds a particle.  (Without the
+// second bound the launches of a sparse scene follow its columns: 97,000 particles on 755 x 755 of
+// them step 476 -> 302 us, 10,600 369 -> 192.)
+uint32_t max_chunks(uint32_t n, const StepConsts& c) { return std::min((n + 63u) / 64u + c.ncols, n); }
 
 // ---------------------------------------------------------------------------
 // Launch shapes of the walks: words per LDS segment x wavefronts per workgroup.  Every
@@ -1249,12 +1252,6 @@ static uint32_t grid_for(uint32_t chunks, uint32_t per_block) {
     return (blocks + kXcds - 1) / kXcds * kXcds;
 }
 
-// Chunks a launch provides for: no more than there are particles, whatever the grid's columns.
-// (97,000 particles on 755 x 755 columns: step 476 -> 302 us, 10,600: 369 -> 192.)
-static uint32_t launch_chunks_bound(uint32_t n, const StepConsts& c) {
-    return std::min(max_chunks(n, c), n);
-}
-
 // CALL sees the shape as type S; TEAM, for the split shapes, likewise.
 #define SPHK_DISPATCH_SHAPE(v, CALL, TEAM)  \
     switch (v) {                            \
@@ -1276,7 +1273,7 @@ hipError_t launch_density_walk(const WalkBuffers& wb, const float4* spm, const u
                                const StepConsts& c, const SceneGrid* scenes, int shape,
                                hipStream_t st) {
     if (n == 0) return hipSuccess;
-    const uint32_t chunks = launch_chunks_bound(n, c);
+    const uint32_t chunks = max_chunks(n, c);
 #define SPHK_DENSITY_KERNEL(KERNEL, CUT, PER_BLOCK, THREADS)                                  \
     hipLaunchKernelGGL((KERNEL<S, CUT>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), 0, \
                        st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, cell_start, \
@@ -1303,7 +1300,7 @@ hipError_t launch_force_walk(const WalkBuffers& wb, const float4* spm, const uin
                              float4* vel, float4* acc, float* rho, float* prs, int shape,
                              unsigned long long* nbr_stats, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    const uint32_t chunks = launch_chunks_bound(n, c);
+    const uint32_t chunks = max_chunks(n, c);
 #define SPHK_FORCE_KERNEL(KERNEL, CUT, PER_BLOCK, THREADS)                                    \
     hipLaunchKernelGGL((KERNEL<S, CUT>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), 0, \
                        st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, sid,       \
@@ -1329,7 +1326,7 @@ hipError_t launch_nbr_lists(const WalkBuffers& wb, const float4* spm, const uint
                             uint32_t* count_by_id, const int64_t* offsets_by_id, int64_t* idx,
                             int shape, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    const uint32_t chunks = launch_chunks_bound(n, c);
+    const uint32_t chunks = max_chunks(n, c);
     // one wavefront per chunk in every shape (a split shape lists with its unsplit twin, a
     // ping-pong shape with the single-buffer shape of the same LDS size)
     const int base = shape == 5 ? 0 : shape == 6 ? 1 : shape == 7 ? 4 : shape == 8 ? 1 : shape;

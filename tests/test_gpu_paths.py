@@ -122,3 +122,52 @@ def test_every_particle_its_own_chunk(sphk, n, shape):
     # one FP32 product each for sigma, W(0) and m W(0), and the spline's own two roundings
     np.testing.assert_allclose(e.densities()[:n], w0, rtol=8 * 2.0**-24)
     np.testing.assert_allclose(e.accelerations()[:, 1], -9.81, rtol=4 * 2.0**-24)
+
+
+def test_wide_grid_stores_words_for_its_particles_only(sphk):
+    # A chunk holds at least one particle, so 2,000 of them have at most 2,000 chunks, however many
+    # columns their grid has (a million here): the word buffers stay at 2,000 x 64 KiB and all
+    # 256 words of a chunk are stored.
+    import ctypes
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert e.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    n = 2000
+    rng = np.random.default_rng(3)
+    pos = rng.uniform([0, 0, 0], [40, 40, 0.4], (n, 3)).astype(np.float32)
+    p = sphk.default_params(xmin=0, xmax=40, ymin=0, ymax=40, zmin=0, zmax=1)
+    e = sphk.Engine(n, p)
+    e.upload(pos)
+    before = free_bytes()
+    items, _, wj0, _ = e.walk_words()
+    dims = e.grid()[1]
+    assert int(dims[0]) * int(dims[1]) > 900000 and len(items) <= n
+    assert wj0.shape[1] == 256
+    # (the sort, scan and cell table of ten million cells among it)
+    assert before - free_bytes() < 1 << 30
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 1000])
+def test_surrogate_of_particles_alone_in_their_columns(sphk, n):
+    # The surrogate's launches provide for as many chunks as there are particles: here there are
+    # exactly that many, each particle without a neighbour, and so with the same prediction.
+    side = 40
+    k = np.random.default_rng(n).permutation(side * side)[:n]
+    pos = np.stack([0.1 * (k // side) + 0.02, 0.1 * (k % side) + 0.02, 0.001 * (k % 7)], 1)
+    p = sphk.default_params(xmin=-1, xmax=5, ymin=-1, ymax=5, zmin=-1, zmax=1, formulation=1)
+    e = sphk.Engine(n, p)
+    e.upload(pos.astype(np.float32))
+    e.surrogate_init(seed=1)
+    w = e.surrogate_params()
+    w[-3:] = [1.0, -2.0, 3.0]  # the output bias
+    e.surrogate_set_params(w)
+    assert len(e.walk_words()[0]) == n
+    out = e.surrogate_predict()
+    assert np.abs(out).min() > 0.0
+    np.testing.assert_array_equal(out, np.broadcast_to(out[0], out.shape))
+    e.surrogate_macro_step(1e-4)
+    np.testing.assert_array_equal(e.accelerations(), np.broadcast_to(e.accelerations()[0], out.shape))
+    np.testing.assert_allclose(e.accelerations(), out, rtol=1e-5)
