@@ -171,3 +171,44 @@ def test_surrogate_of_particles_alone_in_their_columns(sphk, n):
     e.surrogate_macro_step(1e-4)
     np.testing.assert_array_equal(e.accelerations(), np.broadcast_to(e.accelerations()[0], out.shape))
     np.testing.assert_allclose(e.accelerations(), out, rtol=1e-5)
+
+
+@pytest.mark.parametrize("radius", [0.04, 0.03, 0.0123, 0.9])
+def test_pairs_two_cells_apart_are_listed(sphk, oracle, radius):
+    # Pairs whose rounding puts them two cells apart and yet within the radius, a few ulps from a
+    # cell edge, along each axis and in both directions: the walks look two cells out only
+    # for chunks with a particle that the quick test lets through.
+    f = np.float32
+    R = f(radius)
+    inv, r2 = f(1) / R, R * R
+    rng = np.random.default_rng(5)
+    x = np.concatenate([-R * 10.0 ** rng.uniform(-30, -6, 60),
+                        [np.nextafter(k * R, f(-np.inf)) for k in range(-40, 40)]]).astype(f)
+    c = np.floor(x * inv)
+    b = x + R
+    for _ in range(6):
+        b = np.nextafter(b, f(-np.inf))
+    pairs = []
+    for _ in range(13):
+        d = b - x
+        pairs += [(x[i], b[i]) for i in np.nonzero((np.floor(b * inv) == c + 2) & (d * d <= r2))[0]]
+        b = np.nextafter(b, f(np.inf))
+    assert pairs
+    pairs = pairs[:: max(1, len(pairs) // 40)]
+    pos = []
+    for k, (lo, hi) in enumerate(pairs):
+        p = np.full((2, 3), 2.5 * R * (k // 3 + 1), f)  # pairs apart from each other
+        p[:, k % 3] = (lo, hi) if k % 2 else (hi, lo)
+        p[:, (k + 1) % 3] *= -1
+        pos.append(p)
+    pos = np.concatenate(pos)
+    w = float(200 * R)
+    e = sphk.Engine(len(pos), sphk.default_params(xmin=-w, xmax=w, ymin=-w, ymax=w, zmin=-w, zmax=w,
+                                                  neighbor_search_radius=float(R),
+                                                  smoothing_length=float(R) / 2))
+    e.upload(pos)
+    offs, idx = e.neighbors()
+    boffs, bidx = oracle.brute_neighbors(pos, r2)
+    for i in range(len(pos)):
+        got = sorted(idx[offs[i]:offs[i + 1]].tolist())
+        assert got == bidx[boffs[i]:boffs[i + 1]].tolist() and i ^ 1 in got
