@@ -765,7 +765,7 @@ void k_force_walk(
                     }
                     if (seg_base >= words_end) more = false;
                 } else {
-                    nw = phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lm_new, lj_new, lane,
+                    nw = retest_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lm_new, lj_new, lane,
                                               sl, seg_part);
                     if (cu.done) more = false;
                 }
@@ -824,7 +824,7 @@ void k_force_walk(
                 load_words<kSeg>(gmask, gwj0, (size_t)item * c.max_words + seg_base, nw, lmask,
                                  lwj0, lane, sl);
             } else {
-                nw = phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
+                nw = retest_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
                                           seg_part);
                 if (nw == 0) break;
             }
@@ -935,7 +935,7 @@ __global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
                                  lane, sl);
                 w += nw;
             } else {
-                nw = phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
+                nw = retest_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
                                           seg_part);
                 if (nw == 0) break;
             }

@@ -503,16 +503,17 @@ __device__ __forceinline__ uint2 mfma_filter_row(const MfmaFilter& mf,
 }
 
 // Verdict word of this lane's target over the `cnt` candidates from slot j0 on, on the VALU.
+template <bool kFar>
 __device__ __forceinline__ uint32_t valu_filter_word(const uint2* __restrict__ sq, uint32_t j0,
                                                      uint32_t cnt, uint2 qi, bool active,
                                                      int32_t qneg) {
     const uint2* __restrict__ pb = sq + j0;  // uniform base: scalar loads
     uint32_t word = 0;
-    if (cnt == 32u) {
+    if (!kFar && cnt == 32u) {
 #pragma unroll
-        for (int k = 0; k < 32; ++k) word = push_quant<true>(word, qi, pb[k], qneg);
+        for (int k = 0; k < 32; ++k) word = push_quant<kFar>(word, qi, pb[k], qneg);
     } else {
-        for (uint32_t k = 0; k < cnt; ++k) word = push_quant<true>(word, qi, pb[k], qneg);
+        for (uint32_t k = 0; k < cnt; ++k) word = push_quant<kFar>(word, qi, pb[k], qneg);
         word <<= (32u - cnt);
     }
     return active ? word : 0u;
@@ -596,7 +597,7 @@ __device__ __forceinline__ void put_word(uint32_t word, int w, uint32_t* __restr
     sl.count += (uint32_t)__builtin_popcount(word);
 }
 
-template <int kSeg, bool kMfma = false>
+template <int kSeg, bool kMfma = false, bool kFar = false>
 __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
                                               const uint2* __restrict__ sq,
                                               const uint32_t* __restrict__ cs,
@@ -623,7 +624,7 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
             const uint2 qb = mfma_filter_row(*mf, sq, j0, cnt);
             word = filter_word(*mf, qb, cnt, c.qneg, lane, mf->wide);
         } else {
-            word = valu_filter_word(sq, j0, cnt, qi, active, c.qneg);
+            word = valu_filter_word<kFar>(sq, j0, cnt, qi, active, c.qneg);
         }
         put_word(word, w, lmask, lane, sl);
         if (lane == 0) lwj0[w] = j0;
@@ -631,6 +632,22 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
         ++w;
     }
     return w;
+}
+
+// The force walk's re-test.  A loop of its own for tall chunks: the flag in the words' loop cost it
+// the scalar registers that hold its pointers (300,000 particles at 400 a cell, 2.80 -> 2.95 ms).
+template <int kSeg>
+__device__ __forceinline__ int retest_segment(Cursor& cu, const Chunk& ch,
+                                              const uint2* __restrict__ sq,
+                                              const uint32_t* __restrict__ cs,
+                                              const StepConsts& c, uint2 qi, bool active,
+                                              uint32_t* __restrict__ lmask,
+                                              uint32_t* __restrict__ lwj0, uint32_t lane,
+                                              SegLane& sl, int& part) {
+    return ch.zhi - ch.zlo >= kFarCells
+               ? phase1_segment<kSeg, false, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
+                                                   sl, part)
+               : phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl, part);
 }
 
 // The words of table entries first, first + kStride, ... below `end`, in turn to
