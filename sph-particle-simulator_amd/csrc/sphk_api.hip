@@ -652,6 +652,95 @@ int download_packed(sphk_engine* e, const void* src, size_t count, float* out) {
     return rc;
 }
 
+// Box of the finite positions of an upload.
+struct Extent {
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    bool any = false;
+    void add(const float* l, const float* h) {
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = std::min(lo[d], l[d]);
+            hi[d] = std::max(hi[d], h[d]);
+        }
+        any = true;
+    }
+};
+
+int refused_upload(size_t id, const float* p) {
+    return set_error(SPHK_E_DOMAIN, "particle %zu at (%g, %g, %g) needs a cell index beyond +-2^30",
+                     id, (double)p[0], (double)p[1], (double)p[2]);
+}
+
+// Uploads of up to this many rows are checked and packed on the host: two copies and one wait, where
+// the device's check adds a copy back and two launches.  One row 20 us / 36 by the device, 1,000
+// rows 27 / 40, 10,000 92 / 64 (the host's loop takes ~7 ns a row).
+constexpr size_t kUploadHostRows = 2048;
+
+int upload_by_host(sphk_engine* e, size_t offset, size_t n, const float* pos, const float* vel,
+                   const float* mass, Extent* ext) {
+    std::vector<float4> hp(n), hv(n);
+    const float inv = 1.0f / e->params.neighbor_search_radius;
+    for (size_t i = 0; i < n; ++i) {
+        const float* p = pos + 3 * i;
+        hp[i] = make_float4(p[0], p[1], p[2], mass ? mass[i] : e->params.particle_mass);
+        hv[i] = vel ? make_float4(vel[3 * i], vel[3 * i + 1], vel[3 * i + 2], 0.0f)
+                    : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (!std::isfinite(p[0]) || !std::isfinite(p[1]) || !std::isfinite(p[2])) continue;
+        int64_t c;
+        if (floor_cell(p[0], inv, &c) || floor_cell(p[1], inv, &c) || floor_cell(p[2], inv, &c))
+            return refused_upload(offset + i, p);
+        ext->add(p, p);
+    }
+    HIP_TRY(hipMemcpyAsync(e->pm + offset, hp.data(), n * sizeof(float4), hipMemcpyHostToDevice,
+                           e->stream));
+    HIP_TRY(hipMemcpyAsync(e->vel + offset, hv.data(), n * sizeof(float4), hipMemcpyHostToDevice,
+                           e->stream));
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    return SPHK_OK;
+}
+
+// The rows go up as they are, into the sorted arrays (work memory of a build, one row more than
+// the capacity, the last untouched), and are checked and spread to the home arrays there:
+// 177,000 particles ~150 us; the same loops and 16-byte rows on the host took most of a
+// millisecond.
+int upload_by_device(sphk_engine* e, size_t offset, size_t n, const float* pos, const float* vel,
+                     const float* mass, Extent* ext) {
+    const float inv = 1.0f / e->params.neighbor_search_radius;
+    float* const dpos = reinterpret_cast<float*>(e->spm);
+    float* const dvel = reinterpret_cast<float*>(e->svr);
+    float* const dmass = reinterpret_cast<float*>(e->frows);
+    const uint32_t blocks = (uint32_t)std::min<size_t>((n + 255) / 256, 256);
+    uint64_t unused = 0;  // no captured step reads this buffer
+    if (int rc = grow(&e->bbox_out, e->bbox_out_cap, 8 * (uint64_t)blocks, unused)) return rc;
+    e->sorted_valid = false;
+    HIP_TRY(hipMemcpyAsync(dpos, pos, 3 * n * sizeof(float), hipMemcpyHostToDevice, e->stream));
+    hipLaunchKernelGGL(k_upload_check, dim3(blocks), dim3(256), 0, e->stream, dpos, (uint32_t)n, inv,
+                       e->bbox_out);
+    HIP_TRY(hipGetLastError());
+    if (vel)
+        HIP_TRY(hipMemcpyAsync(dvel, vel, 3 * n * sizeof(float), hipMemcpyHostToDevice, e->stream));
+    if (mass)
+        HIP_TRY(hipMemcpyAsync(dmass, mass, n * sizeof(float), hipMemcpyHostToDevice, e->stream));
+    std::vector<uint32_t> box(8 * blocks);
+    HIP_TRY(hipMemcpyAsync(box.data(), e->bbox_out, box.size() * 4, hipMemcpyDeviceToHost,
+                           e->stream));
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    uint32_t bad = ~0u;
+    for (uint32_t b = 0; b < blocks; ++b) {
+        const uint32_t* o = box.data() + 8 * b;
+        bad = std::min(bad, o[7]);
+        if (!o[6]) continue;
+        const float l[3] = {unord(o[0]), unord(o[1]), unord(o[2])};
+        const float h[3] = {unord(o[3]), unord(o[4]), unord(o[5])};
+        ext->add(l, h);
+    }
+    if (bad != ~0u) return refused_upload(offset + bad, pos + 3 * (size_t)bad);
+    hipLaunchKernelGGL(k_upload_rows, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, e->stream,
+                       dpos, vel ? dvel : nullptr, mass ? dmass : nullptr, e->params.particle_mass,
+                       (uint32_t)n, e->pm + offset, e->vel + offset);
+    HIP_TRY(hipGetLastError());
+    return SPHK_OK;
+}
+
 // A download into too small a buffer: a raised grid flag is the graver error.
 int refused_download(sphk_engine* e, size_t need) {
     if (int rc = check_grid_flag(e)) return rc;
@@ -998,59 +1087,12 @@ int sphk_upload(sphk_engine* e, size_t offset, size_t n, const float* pos, const
     if (offset > e->n) return set_error(SPHK_E_INVALID, "offset %zu beyond count %zu", offset, e->n);
     if (n && !pos) return set_error(SPHK_E_INVALID, "null positions");
     if (int rc = set_device(e)) return rc;
-    // The rows go up as they are, into the sorted arrays (work memory of a build, one row
-    // more than the capacity, the last untouched), and are checked and spread to the home
-    // arrays there: 177,000 particles ~150 us; the same loops and 16-byte rows on the host took
-    // most of a millisecond.
     const size_t fit = std::min(n, e->cap - offset);
-    float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-    bool any = false;
+    Extent ext;
     if (fit) {
-        const float inv = 1.0f / e->params.neighbor_search_radius;
-        float* const dpos = reinterpret_cast<float*>(e->spm);
-        float* const dvel = reinterpret_cast<float*>(e->svr);
-        float* const dmass = reinterpret_cast<float*>(e->frows);
-        const uint32_t blocks = (uint32_t)std::min<size_t>((fit + 255) / 256, 256);
-        uint64_t unused = 0;  // no captured step reads this buffer
-        if (int rc = grow(&e->bbox_out, e->bbox_out_cap, 8 * (uint64_t)blocks, unused)) return rc;
-        e->sorted_valid = false;
-        HIP_TRY(hipMemcpyAsync(dpos, pos, 3 * fit * sizeof(float), hipMemcpyHostToDevice,
-                               e->stream));
-        hipLaunchKernelGGL(k_upload_check, dim3(blocks), dim3(256), 0, e->stream, dpos,
-                           (uint32_t)fit, inv, e->bbox_out);
-        HIP_TRY(hipGetLastError());
-        if (vel)
-            HIP_TRY(hipMemcpyAsync(dvel, vel, 3 * fit * sizeof(float), hipMemcpyHostToDevice,
-                                   e->stream));
-        if (mass)
-            HIP_TRY(hipMemcpyAsync(dmass, mass, fit * sizeof(float), hipMemcpyHostToDevice,
-                                   e->stream));
-        std::vector<uint32_t> box(8 * blocks);
-        HIP_TRY(hipMemcpyAsync(box.data(), e->bbox_out, box.size() * 4, hipMemcpyDeviceToHost,
-                               e->stream));
-        HIP_TRY(hipStreamSynchronize(e->stream));
-        uint32_t bad = ~0u;
-        for (uint32_t b = 0; b < blocks; ++b) {
-            const uint32_t* o = box.data() + 8 * b;
-            bad = std::min(bad, o[7]);
-            if (!o[6]) continue;
-            for (int d = 0; d < 3; ++d) {
-                const float l = unord(o[d]), h = unord(o[3 + d]);
-                lo[d] = any ? std::min(lo[d], l) : l;
-                hi[d] = any ? std::max(hi[d], h) : h;
-            }
-            any = true;
-        }
-        if (bad != ~0u)
-            return set_error(SPHK_E_DOMAIN,
-                             "particle %zu at (%g, %g, %g) needs a cell index beyond +-2^30",
-                             offset + bad, (double)pos[3 * (size_t)bad],
-                             (double)pos[3 * (size_t)bad + 1], (double)pos[3 * (size_t)bad + 2]);
-        hipLaunchKernelGGL(k_upload_rows, dim3((uint32_t)((fit + 255) / 256)), dim3(256), 0,
-                           e->stream, dpos, vel ? dvel : nullptr, mass ? dmass : nullptr,
-                           e->params.particle_mass, (uint32_t)fit, e->pm + offset,
-                           e->vel + offset);
-        HIP_TRY(hipGetLastError());
+        const int rc = fit <= kUploadHostRows ? upload_by_host(e, offset, fit, pos, vel, mass, &ext)
+                                              : upload_by_device(e, offset, fit, pos, vel, mass, &ext);
+        if (rc) return rc;
     }
     e->n = offset + fit;
     if (!e->scenes_explicit) {
@@ -1058,7 +1100,7 @@ int sphk_upload(sphk_engine* e, size_t offset, size_t n, const float* pos, const
         e->scenes.resize(1);
         SceneHost& sc = e->scenes[0];
         if (offset == 0) sc.ext_any = false;
-        if (any) ext_add_box(sc, lo, hi);
+        if (ext.any) ext_add_box(sc, ext.lo, ext.hi);
         if (offset == 0) e->ext_unknown = false;
     } else {
         // explicit scenes: measure every scene's extent on the device before the next build

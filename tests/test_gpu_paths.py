@@ -212,3 +212,32 @@ def test_pairs_two_cells_apart_are_listed(sphk, oracle, radius):
     for i in range(len(pos)):
         got = sorted(idx[offs[i]:offs[i + 1]].tolist())
         assert got == bidx[boffs[i]:boffs[i + 1]].tolist() and i ^ 1 in got
+
+
+@pytest.mark.parametrize("rows", [9, 2054, 2055, 2056, 5000])
+def test_refused_uploads_on_both_routes(sphk, rows):
+    # Up to 2,048 rows are checked on the host, more on the device: either way the first row
+    # beyond the cell range is named and the state stays as it was, and what is accepted sets the
+    # same extent (the next step finds every particle inside its grid).
+    rng = np.random.default_rng(rows)
+    pos = rng.uniform(-1, 1, (100, 3)).astype(np.float32)
+    more = rng.uniform(2, 3, (rows, 3)).astype(np.float32)
+    p = sphk.default_params(xmin=-4, xmax=4, ymin=-4, ymax=4, zmin=-4, zmax=4, formulation=1)
+    e = sphk.Engine(100 + rows - 7, p)  # the last seven rows do not fit
+    e.upload(pos)
+    before = e.neighbors()
+    far = more.copy()
+    far[rows - 9] = far[rows - 8, 2] = 1e9
+    with pytest.raises(sphk.SphkError, match=f"particle {100 + rows - 9} "):
+        e.upload(far, offset=100)
+    assert e.size() == 100
+    for a, b in zip(before, e.neighbors()):
+        np.testing.assert_array_equal(a, b)
+    more[5, 1] = np.nan
+    more[rows - 3] = 1e9  # beyond the capacity: dropped, not checked
+    with pytest.raises(sphk.SphkError, match="capacity"):
+        e.upload(more, offset=100)
+    assert e.size() == 100 + rows - 7
+    np.testing.assert_array_equal(e.positions(), np.concatenate([pos, more[:-7]]))
+    e.step(1e-5)
+    e.positions()  # (would report a particle outside its grid)
