@@ -767,9 +767,11 @@ __global__ __launch_bounds__(256) void k_sur_wgrad(SurGradRows g, const __bf16* 
 //  - The features are written to LDS as ten rows of 64 edges, in the order the B operand takes
 //    them (the accumulator's row order), so an operand is one 16-byte read instead of eight
 //    2-byte ones and their packing.
-// The features are the forward pass's to the bit: formed in another order one of them now and
-// then rounds to the next bf16 value, in the ReLU masks and in dW1 (W(r) by clamped cubes is
-// 5 us of a call of 880 faster).
+// The features and the layer-1 product are the forward pass's to the bit.  W(r) by clamped cubes
+// (5 us of a call of 880 faster) now and then rounds to the next bf16 value, in the ReLU masks and
+// in dW1; operands with the halves of K the same way round in both blocks (no time) give the sums
+// that lie within a rounding of zero another sign, some of 2e9 a call: one such mask moved a
+// small scene's gradient by 5e-6 of its norm.
 // 1,024 chunks: 600 -> 231 us.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kEdgeRow = 72;  // LDS row stride (bf16) of one feature over 64 edges
@@ -800,10 +802,14 @@ k_sur_edges_bwd(
                     pi))
         return;
     const float4 vi = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    bf16x8 B[4];
-    load_layer1(pk, lane, B);
+    bf16x8 B[2][4];
+    load_layer1(pk, lane, B[0]);
+    load_layer1<true>(pk, lane, B[1]);
 #pragma unroll
-    for (int hb = 0; hb < 4; ++hb) B[hb] = negated(B[hb]);
+    for (int hb = 0; hb < 4; ++hb) {
+        B[0][hb] = negated(B[0][hb]);
+        B[1][hb] = negated(B[1][hb]);
+    }
     // dS of this lane's hidden units for the 16 accumulator rows, as bf16 pairs (rows v, v + 1)
     uint32_t ds[4][8];
 #pragma unroll
@@ -837,7 +843,7 @@ k_sur_edges_bwd(
                    le[9 * kEdgeRow + epos] = (uint16_t)ext;
                    wave_sync();
                    bf16x8 a[2];
-                   layer1_a<false>(fe, ext, a[0], a[1]);
+                   layer1_a<true>(fe, ext, a[0], a[1]);
 #pragma unroll
                    for (int blk = 0; blk < 2; ++blk) {
                        const bf16x8 e0 = load8(erow + 32 * blk);
@@ -845,7 +851,7 @@ k_sur_edges_bwd(
 #pragma unroll
                        for (int hb = 0; hb < 4; ++hb) {
                            // -u of 16 edges
-                           const f32x16 d = mfma16(a[blk], B[hb], zero16());
+                           const f32x16 d = mfma16(a[blk], B[blk][hb], zero16());
                            uint32_t g[8];
 #pragma unroll
                            for (int k = 0; k < 8; ++k)
