@@ -214,9 +214,10 @@ int sphk_debug_walk_words(sphk_engine* e, uint32_t* items, uint32_t* nwords, uin
 int sphk_debug_grid(sphk_engine* e, int32_t* origin3, int32_t* dims3, uint64_t* ncells);
 
 /* Launch shapes of the two neighbour walks (LDS words per segment x wavefronts per
- * workgroup; "_split" shapes give each chunk a workgroup of its own, whose wavefronts
- * share its candidate words and walk one part of its candidate columns each; "pp" shapes hold two segments,
- * so a lane through one goes on into the next), indexed 0..sphk_walk_shape_count()-1.
+ * workgroup; "_split" shapes give each chunk a workgroup of its own, whose wavefronts share
+ * its candidate words and the parts of its candidate columns -- three walk them in the density
+ * walk, two in the force walk; "pp" shapes hold two segments, so a lane through one goes on
+ * into the next), indexed 0..sphk_walk_shape_count()-1.
  * Results do not depend on the shape (each particle's sums run in the same order in every
  * shape); only speed does.  Until set, an engine uses seg32_waves4_split below 163,840
  * particles and seg24_waves4 (density) with pp16_waves4 (force) above (chosen again whenever

@@ -614,7 +614,8 @@ __global__ __launch_bounds__(64 * kNodeWaves) void k_sur_node_bwd(
 // wide, coalesced loads and its column t belongs to tile t: a byte permute per operand dword
 // does the transpose, no LDS.  The 16 columns of Q beyond 128 (the bias columns and the last
 // node inputs) are a fifth tile.  The next K step's rows are requested before this one's
-// products.  Bound by the read of the rows (4.6 KB and 5 KB a K step of 16): 65,536 rows,
+// products.  Bound by the read of the rows (a K step of 16: 4 KB of P, 0.1 KB in the output
+// layer, and 4.6 KB of Q): 65,536 rows,
 // three products 218 -> 25 us, against one 32 x 32 tile per wavefront with 2-byte loads.
 // kMT 2: P has 128 columns; two wavefronts split them, two pairs split the rows.
 // kMT 1: P is the output gradient (3 of 4 columns); the four wavefronts split the rows.

@@ -74,7 +74,8 @@ uint32_t max_chunks(uint32_t n, const StepConsts& c) { return std::min((n + 63u)
 
 // ---------------------------------------------------------------------------
 // Launch shapes of the walks: words per LDS segment x wavefronts per workgroup.  Every
-// wavefront works on its own chunk; the waves of a workgroup never synchronise.
+// wavefront works on its own chunk and the waves of a workgroup never synchronise, but for the
+// team walks (the "_split" shapes, below), which give a chunk a workgroup.
 // ---------------------------------------------------------------------------
 
 // ---------------------------------------------------------------------------
@@ -218,7 +219,7 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
     if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
     const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
     MfmaFilter mf;
-    mfma_filter_begin(mf, ch, sq, qi, active, lane, c.qneg);
+    mfma_filter_begin(mf, ch, qi, active, lane, c.qneg);
     WordTable wt;
     static_assert(kLds * 64 >= kTableWords, "the word table is built in the mask buffer");
     const bool tab = word_table_build(wt, ch, cs, -1, lane, lmask);
@@ -350,8 +351,8 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
 // words of the chunk (about 1,000 cycles each), then each part's pairs are walked by one
 // wavefront (a part's sum runs in candidate order) and the first one finishes the
 // particles from LDS.  Against three independent wavefronts per chunk and a finishing launch
-// per walk: a step of 2,145 particles 108 -> 96 us, of 10,000 126 -> 110 us, ten steps of 34,000
-// 1.36 -> 1.24 ms.  Eight wavefronts a team are slower from 10,000 particles on (two
+// per walk: a step of 2,145 particles 108 -> 96 us, of 10,000 126 -> 110 us, ten steps of 33,000
+// 1.36 -> 1.27 ms.  Eight wavefronts a team are slower from 10,000 particles on (two
 // workgroups a CU).
 // ---------------------------------------------------------------------------
 constexpr int kTeam = 4;
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(64 * kTeam) void k_density_team(
     if (!load_chunk(item, items, desc, nitems, skey, spm, c, scenes, lane, ch, s, active, pi)) return;
     const uint2 qi = active ? sq[s] : make_uint2(0u, 0u);
     MfmaFilter mf;
-    mfma_filter_begin(mf, ch, sq, qi, active, lane, c.qneg);
+    mfma_filter_begin(mf, ch, qi, active, lane, c.qneg);
     WordTable wt;
     const bool tab = word_table_build(wt, ch, cs, -1, lane, scratch[wave]);
     uint32_t* const gm = gmask + (size_t)item * c.max_words * 64;
@@ -608,7 +609,7 @@ __device__ __forceinline__ void force_run_n(BitWalk<kW>& bw, float4 (&a)[kAhead 
 
 // Folds the sums of finished parts into the running total, which starts at +0:
 // ((0 + part 0) + part 1) + part 2.  Closing `n` parts at once adds `f` for the first and
-// +0 for each further (empty) one, as the three-wavefront finish does.  The single-wavefront
+// +0 for each further (empty) one, as the team walk does.  The single-wavefront
 // walk keeps the total in LDS (`t`, six rows of 64 lanes): six more live registers would cost
 // it a wavefront per SIMD.
 __device__ __forceinline__ void fold_parts(float* __restrict__ t, uint32_t lane, ForceSums& f,
@@ -864,8 +865,8 @@ void k_force_walk(
 // Force pass over one chunk by a team of two wavefronts (see k_density_team): the first walks
 // part 0, the second parts 1 and 2 (the ring two columns out is nearly always empty); the first
 // folds the parts' sums from LDS and finishes the particles.  Two teams in one workgroup of four
-// wavefronts were slower (ten steps of 34,000 particles 1.24 -> 1.33 ms: coarser workgroups
-// spread the chunks less evenly over the CUs).
+// wavefronts were slower (33,000 particles: 41 -> 46 us a walk: coarser workgroups spread the
+// chunks less evenly over the CUs), a wavefront per part no faster.
 constexpr int kForceTeam = 2;
 
 template <class Shape, bool kCut>

@@ -91,7 +91,7 @@ __constant__ uint8_t kColumnOrder[2][25] = {
 // Parts of a walk (balanced order): the corner columns with the centre (positions 0-4), the
 // edge columns (5-8), the outer ring (9-24).  Sums over a chunk's neighbours are formed per
 // part, each in candidate order, and combined as (0 + part 0) + part 1) + part 2, so a walk
-// split over three wavefronts (one part each) gives the same bits as one wavefront walking
+// whose parts are shared out among wavefronts gives the same bits as one wavefront walking
 // all three.  Part starts are segment breaks.
 __device__ __forceinline__ int part_begin(int p) { return p == 0 ? 0 : p == 1 ? 5 : 9; }
 __device__ __forceinline__ int part_end(int p) { return p == 0 ? 5 : p == 1 ? 9 : 25; }
@@ -476,8 +476,7 @@ __device__ __forceinline__ void mfma_filter_targets(MfmaFilter& mf, uint32_t lan
     mf.b2 = __builtin_bit_cast(sphk_half8, make_uint4(h[0], h[1], h[2], h[3]));
 }
 
-__device__ __forceinline__ void mfma_filter_begin(MfmaFilter& mf, const Chunk& ch,
-                                                  const uint2* __restrict__ sq, uint2 qi,
+__device__ __forceinline__ void mfma_filter_begin(MfmaFilter& mf, const Chunk& ch, uint2 qi,
                                                   bool active, uint32_t lane, int32_t qneg) {
     const int zspan = ch.zhi - ch.zlo;
     mf.wide = zspan > 4;
