@@ -474,6 +474,7 @@ int ensure_grid(sphk_engine* e) {
     e->consts.G = (uint32_t)G;
     e->consts.ncols = (uint32_t)ncols;
     e->consts.nscenes = (uint32_t)S;
+    for (const SceneGrid& t : e->table) e->consts.far |= t.nz > kFarCells;
     e->consts.pad_slot = (uint32_t)e->cap;
     const uint64_t chunks = max_chunks((uint32_t)e->cap, e->consts);
     WalkBuffers& wb = e->walk;

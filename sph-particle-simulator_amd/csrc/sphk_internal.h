@@ -35,6 +35,8 @@ struct StepConsts {
     int32_t cut;      // 1 when the search radius is below the kernel support 2h: the walks
                       // then drop pairs beyond the radius explicitly (else their weight is
                       // zero or below 2^-75 of a neighbour's)
+    int32_t far;      // 1 when a scene grid has more than kFarCells z cells: the candidate test
+                      // then guards the square of the z difference against wrap-around
     uint32_t G;       // cells of all scene grids; particles with dense index G have a
                       // non-finite coordinate
     uint32_t ncols;   // (x, y) columns of all scene grids
@@ -46,6 +48,10 @@ struct StepConsts {
                         // with more are tested again by the force walk
     double qscale;      // quantized coordinate = floor(x * qscale): 256 units per cell
 };
+
+// z cells within which the squared distance of two particles of a scene, 256 units a cell, stays
+// below 2^31.
+constexpr int kFarCells = 180;
 
 // Neighbour row of the force walk, one per sorted slot: a = (x, y, z, m/rho),
 // b = (vx, vy, vz, m P / (4 rho^2)); both halves share one 32-byte block.

@@ -13,8 +13,8 @@
 //   (filter_word, 32 candidates x 64 targets per word), or one candidate at a time for
 //   the whole wave (push_quant) in the words that span too many z cells for them and, with the
 //   candidate data through the scalar cache, in the force walk's re-test and the
-//   neighbour-list export; the bits are the same.  `wj0[w]` is the sorted slot of the first candidate of
-//   word w.  Segments hold up to kSeg - 1 words and never span two parts.
+//   neighbour-list export; the bits are the same.  `wj0[w]` is the sorted slot of the first
+//   candidate of word w.  Segments hold up to kSeg - 1 words and never span two parts.
 // Phase 2 (evaluate): every lane walks only its own set bits and evaluates the kernel for
 //   those pairs (pairs the filter let through beyond the radius weigh exactly zero).
 // The density pass stores the words of each chunk in HBM (masks, wj0, word count, part
@@ -70,7 +70,9 @@ __global__ __launch_bounds__(256) void k_chunk_fill(const uint32_t* __restrict__
 // Every column may end with a part-filled chunk, and every chunk holds a particle.  (Without the
 // second bound the launches of a sparse scene follow its columns: 97,000 particles on 755 x 755 of
 // them step 476 -> 302 us, 10,600 369 -> 192.)
-uint32_t max_chunks(uint32_t n, const StepConsts& c) { return std::min((n + 63u) / 64u + c.ncols, n); }
+uint32_t max_chunks(uint32_t n, const StepConsts& c) {
+    return std::min((n + 63u) / 64u + c.ncols, n);
+}
 
 // ---------------------------------------------------------------------------
 // Launch shapes of the walks: words per LDS segment x wavefronts per workgroup.  Every
@@ -193,7 +195,7 @@ __device__ __forceinline__ float density_run(BitWalk<kW>& bw, float4& q0, float4
 // allows (six with 24-word segments): the walk is VALU-bound (a few spills outside the walk
 // loops).  The ping-pong shapes aim at what their LDS
 // allows (6 with two 12-word buffers, 4 with two 16-word ones).
-template <class Shape, bool kCut>
+template <class Shape, bool kCut, bool kFar>
 __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(Shape::density_waves, 8))) void k_density_walk(
     const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
     const uint32_t* __restrict__ nitems,
@@ -254,11 +256,11 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
             if (pp.nw_new == 0 && !pend && more) {
                 SegLane sl;
                 int seg_part;
-                const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, lm_new, lj_new, gm, gj,
-                                                        lane, sl, seg_part, mf)
-                                   : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active,
-                                                                lm_new, lj_new, lane, sl,
-                                                                seg_part, &mf);
+                const int nw =
+                    tab ? phase1_table<kSeg, kFar>(wt, ti, sq, c, lm_new, lj_new, gm, gj, lane, sl,
+                                                   seg_part, mf)
+                        : phase1_segment<kSeg, true, kFar>(cu, ch, sq, cs, c, qi, active, lm_new,
+                                                           lj_new, lane, sl, seg_part, &mf);
                 if (nw == 0) {
                     more = false;
                 } else {
@@ -317,9 +319,10 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
             SegLane sl;
             int seg_part;
             const int nw =
-                tab ? phase1_table<kSeg>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl, seg_part, mf)
-                    : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
-                                                 sl, seg_part, &mf);
+                tab ? phase1_table<kSeg, kFar>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl,
+                                               seg_part, mf)
+                    : phase1_segment<kSeg, true, kFar>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
+                                                       lane, sl, seg_part, &mf);
             if (nw == 0) break;
             for (; cur_part < seg_part; ++cur_part) {
                 total = cur_part == 0 ? cur : total + cur;
@@ -352,7 +355,10 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
 // wavefront (a part's sum runs in candidate order) and the first one finishes the
 // particles from LDS.  Against three independent wavefronts per chunk and a finishing launch
 // per walk: a step of 2,145 particles 108 -> 96 us, of 10,000 126 -> 110 us, ten steps of 33,000
-// 1.36 -> 1.27 ms.  Eight wavefronts a team are slower from 10,000 particles on (two
+// 1.36 -> 1.27 ms.  Pile-ups, whose chunks have too many words for the table, gain less (400 a
+// cell: 3,000 particles 249 -> 220 us, 50,000 850 -> 824, 100,000 1483 -> 1210) and lose around
+// 20,000 to 30,000, where the independent wavefronts filled every CU once (590 -> 604, 708 -> 752;
+// at 1,500 a cell 1424 -> 1627).  Eight wavefronts a team are slower from 10,000 particles on (two
 // workgroups a CU).
 // ---------------------------------------------------------------------------
 constexpr int kTeam = 4;
@@ -365,7 +371,7 @@ __device__ __forceinline__ int team_rows(int words, int group) {
 
 // The part's sum over the words of its cursor or its own table: chunks of more than kTableWords
 // words, one wavefront per part.
-template <class Shape, bool kCut>
+template <class Shape, bool kCut, bool kFar>
 __device__ __forceinline__ float density_part_alone(
     const Chunk& ch, MfmaFilter& mf, int part, const float4* __restrict__ spm,
     const uint2* __restrict__ sq, const uint32_t* __restrict__ cs, const StepConsts& c, uint2 qi,
@@ -384,10 +390,10 @@ __device__ __forceinline__ float density_part_alone(
     for (;;) {
         SegLane sl;
         int seg_part;
-        const int nw = tab ? phase1_table<kSeg>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl,
+        const int nw = tab ? phase1_table<kSeg, kFar>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl,
                                                 seg_part, mf)
-                           : phase1_segment<kSeg, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
-                                                        lane, sl, seg_part, &mf);
+                           : phase1_segment<kSeg, true, kFar>(cu, ch, sq, cs, c, qi, active, lmask,
+                                                              lwj0, lane, sl, seg_part, &mf);
         if (nw == 0) break;
         wave_sync();
         if (!tab) store_words(c.max_words, seg_base, nw, lmask, lwj0, gm, gj, lane);
@@ -402,7 +408,7 @@ __device__ __forceinline__ float density_part_alone(
     return cur;
 }
 
-template <class Shape, bool kCut>
+template <class Shape, bool kCut, bool kFar>
 __global__ __launch_bounds__(64 * kTeam) void k_density_team(
     const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
     const uint32_t* __restrict__ nitems, const float4* __restrict__ spm,
@@ -446,7 +452,7 @@ __global__ __launch_bounds__(64 * kTeam) void k_density_team(
             const int l = w < wt.ps1 ? w : w < wt.ps2 ? w - wt.ps1 : w - wt.ps2;
             return (w < wt.ps1 ? 0 : w < wt.ps2 ? r1 : r2) + l + l / kGroup;
         };
-        table_words<kTeam, true>(wt, mf, sq, (int)wave, wt.total, c.qneg, lane,
+        table_words<kTeam, true, kFar>(wt, mf, sq, (int)wave, wt.total, c.qneg, lane,
                                  [&](uint32_t word, int w, uint32_t j0) {
                                      const int r = row_of(w);
                                      lmask[r * 64 + lane] = word;
@@ -486,9 +492,9 @@ __global__ __launch_bounds__(64 * kTeam) void k_density_team(
             }
         }
     } else if (wave < kParts) {
-        cur = density_part_alone<Shape, kCut>(ch, mf, (int)wave, spm, sq, cs, c, qi, active, pi,
-                                              gm, gj, lmask + wave * kSeg * 64,
-                                              lwj0 + wave * kSeg, scratch[wave], lane);
+        cur = density_part_alone<Shape, kCut, kFar>(ch, mf, (int)wave, spm, sq, cs, c, qi, active,
+                                                    pi, gm, gj, lmask + wave * kSeg * 64,
+                                                    lwj0 + wave * kSeg, scratch[wave], lane);
     }
     if (wave < kParts) lsum[wave][lane] = cur;
     __syncthreads();
@@ -668,7 +674,7 @@ __device__ __forceinline__ void load_words(const uint32_t* __restrict__ gmask,
 // Force pass over one chunk by one wavefront.  Shapes of 24 words and more keep
 // the parts' running total in registers: their LDS, not their registers, limits occupancy,
 // and the 1.5 KB per wavefront it frees lets the 28-word shape run 5 wavefronts per SIMD.
-template <class Shape, bool kCut>
+template <class Shape, bool kCut, bool kFar>
 __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(Shape::force_waves)))
 void k_force_walk(
     const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
@@ -766,8 +772,8 @@ void k_force_walk(
                     }
                     if (seg_base >= words_end) more = false;
                 } else {
-                    nw = retest_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lm_new, lj_new, lane,
-                                              sl, seg_part);
+                    nw = phase1_segment<kSeg, false, kFar>(cu, ch, sq, cs, c, qi, active, lm_new,
+                                                           lj_new, lane, sl, seg_part);
                     if (cu.done) more = false;
                 }
                 if (nw == 0) {
@@ -825,8 +831,8 @@ void k_force_walk(
                 load_words<kSeg>(gmask, gwj0, (size_t)item * c.max_words + seg_base, nw, lmask,
                                  lwj0, lane, sl);
             } else {
-                nw = retest_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
-                                          seg_part);
+                nw = phase1_segment<kSeg, false, kFar>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
+                                                       lane, sl, seg_part);
                 if (nw == 0) break;
             }
             if (kRegTot)
@@ -869,7 +875,7 @@ void k_force_walk(
 // chunks less evenly over the CUs), a wavefront per part no faster.
 constexpr int kForceTeam = 2;
 
-template <class Shape, bool kCut>
+template <class Shape, bool kCut, bool kFar>
 __global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
     const uint32_t* __restrict__ items, const uint4* __restrict__ desc,
     const uint32_t* __restrict__ nitems, const float4* __restrict__ spm,
@@ -936,8 +942,8 @@ __global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
                                  lane, sl);
                 w += nw;
             } else {
-                nw = retest_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
-                                          seg_part);
+                nw = phase1_segment<kSeg, false, kFar>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
+                                                       lane, sl, seg_part);
                 if (nw == 0) break;
             }
             wave_sync();
@@ -1198,7 +1204,8 @@ __global__ __launch_bounds__(Shape::threads) void k_nbr_lists(
         SegLane sl;
         int part;  // always 0 in the reference order
         const int nw =
-            phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl, part);
+            phase1_segment<kSeg, false, false>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl,
+                                               part);
         if (nw == 0) break;
         wave_sync();
         BitWalk<kSeg> bw;
@@ -1275,17 +1282,26 @@ hipError_t launch_density_walk(const WalkBuffers& wb, const float4* spm, const u
                                hipStream_t st) {
     if (n == 0) return hipSuccess;
     const uint32_t chunks = max_chunks(n, c);
-#define SPHK_DENSITY_KERNEL(KERNEL, CUT, PER_BLOCK, THREADS)                                  \
-    hipLaunchKernelGGL((KERNEL<S, CUT>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), 0, \
-                       st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, cell_start, \
+#define SPHK_DENSITY_KERNEL(KERNEL, CUT, FAR, PER_BLOCK, THREADS)                              \
+    hipLaunchKernelGGL((KERNEL<S, CUT, FAR>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), \
+                       0, st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, cell_start, \
                        c, scenes, wb.mask, wb.wj0, wb.nwords, wb.pstarts)
-#define SPHK_DENSITY_LAUNCH(CUT)                                                             \
-    SPHK_DISPATCH_SHAPE(shape, SPHK_DENSITY_KERNEL(k_density_walk, CUT, S::waves, S::threads), \
-                        SPHK_DENSITY_KERNEL(k_density_team, CUT, 1, 64 * kTeam))
+#define SPHK_DENSITY_LAUNCH(CUT, FAR)                                                         \
+    SPHK_DISPATCH_SHAPE(                                                                      \
+        shape, SPHK_DENSITY_KERNEL(k_density_walk, CUT, FAR, S::waves, S::threads),           \
+        SPHK_DENSITY_KERNEL(k_density_team, CUT, FAR, 1, 64 * kTeam))
     if (c.cut) {
-        SPHK_DENSITY_LAUNCH(true);
+        if (c.far) {
+            SPHK_DENSITY_LAUNCH(true, true);
+        } else {
+            SPHK_DENSITY_LAUNCH(true, false);
+        }
     } else {
-        SPHK_DENSITY_LAUNCH(false);
+        if (c.far) {
+            SPHK_DENSITY_LAUNCH(false, true);
+        } else {
+            SPHK_DENSITY_LAUNCH(false, false);
+        }
     }
 #undef SPHK_DENSITY_LAUNCH
 #undef SPHK_DENSITY_KERNEL
@@ -1302,18 +1318,27 @@ hipError_t launch_force_walk(const WalkBuffers& wb, const float4* spm, const uin
                              unsigned long long* nbr_stats, hipStream_t st) {
     if (n == 0) return hipSuccess;
     const uint32_t chunks = max_chunks(n, c);
-#define SPHK_FORCE_KERNEL(KERNEL, CUT, PER_BLOCK, THREADS)                                    \
-    hipLaunchKernelGGL((KERNEL<S, CUT>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), 0, \
-                       st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, sid,       \
-                       cell_start, c, scenes, wb.mask, wb.wj0, wb.nwords, wb.pstarts, dt_dev, \
+#define SPHK_FORCE_KERNEL(KERNEL, CUT, FAR, PER_BLOCK, THREADS)                               \
+    hipLaunchKernelGGL((KERNEL<S, CUT, FAR>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), \
+                       0, st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, sid,     \
+                       cell_start, c, scenes, wb.mask, wb.wj0, wb.nwords, wb.pstarts, dt_dev,  \
                        dt, pm, vel, acc, rho, prs, nbr_stats)
-#define SPHK_FORCE_LAUNCH(CUT)                                                               \
-    SPHK_DISPATCH_SHAPE(shape, SPHK_FORCE_KERNEL(k_force_walk, CUT, S::waves, S::threads),    \
-                        SPHK_FORCE_KERNEL(k_force_team, CUT, 1, 64 * kForceTeam))
+#define SPHK_FORCE_LAUNCH(CUT, FAR)                                                           \
+    SPHK_DISPATCH_SHAPE(shape,                                                                \
+                        SPHK_FORCE_KERNEL(k_force_walk, CUT, FAR, S::waves, S::threads),      \
+                        SPHK_FORCE_KERNEL(k_force_team, CUT, FAR, 1, 64 * kForceTeam))
     if (c.cut) {
-        SPHK_FORCE_LAUNCH(true);
+        if (c.far) {
+            SPHK_FORCE_LAUNCH(true, true);
+        } else {
+            SPHK_FORCE_LAUNCH(true, false);
+        }
     } else {
-        SPHK_FORCE_LAUNCH(false);
+        if (c.far) {
+            SPHK_FORCE_LAUNCH(false, true);
+        } else {
+            SPHK_FORCE_LAUNCH(false, false);
+        }
     }
 #undef SPHK_FORCE_LAUNCH
 #undef SPHK_FORCE_KERNEL

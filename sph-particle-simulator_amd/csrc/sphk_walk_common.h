@@ -376,18 +376,19 @@ struct SegLane {
 // dX, dY (16-bit wrap-around) and dZ the differences of the quantized coordinates,
 // t = dX^2 + dY^2 + dZ^2 + qneg is negative exactly when the squared distance is at most T,
 // and word = 2 * word + sign(t).  Five VALU: packed 16-bit subtract, subtract, 24-bit
-// multiply-add, dot2, align-bit.  kFar: dZ is clamped first (one more), for candidates 180 cells
-// and more away, whose square would wrap around in 32 bits and let them pass.
+// multiply-add, dot2, align-bit.  kFar (StepConsts::far): dZ is clamped first,
+// as the square of 181 cells would wrap around in 32 bits and let a far candidate pass.  Such
+// grids get kernels of their own: as a flag the clamp cost the walks registers on every grid
+// (300,000 particles at 400 a cell 2.80 -> 2.95 ms a step, five steps of 293,000 2.56 -> 2.58).
 typedef short sphk_short2 __attribute__((ext_vector_type(2)));
-constexpr int kFarCells = 180;  // (180 cells + 2 units)^2 < 2^31
 template <bool kFar>
 __device__ __forceinline__ uint32_t push_quant(uint32_t word, uint2 a, uint2 b, int32_t qneg) {
     const sphk_short2 dxy =
         __builtin_bit_cast(sphk_short2, a.x) - __builtin_bit_cast(sphk_short2, b.x);
     int32_t dz = (int32_t)(a.y - b.y);
     if (kFar) dz = min(max(dz, -32767), 32767);
-    const int32_t t =
-        __builtin_amdgcn_sdot2(dxy, dxy, (int32_t)((uint32_t)__mul24(dz, dz) + (uint32_t)qneg), false);
+    const int32_t zz = (int32_t)((uint32_t)__mul24(dz, dz) + (uint32_t)qneg);
+    const int32_t t = __builtin_amdgcn_sdot2(dxy, dxy, zz, false);
     return __builtin_amdgcn_alignbit(word, (uint32_t)t, 31);
 }
 
@@ -434,7 +435,6 @@ static_assert((kWideReach * kWideReach + 2 * 769 * 769) >> 11 <= 2048 &&
 struct MfmaFilter {
     bool wide;           // uniform: more than 5 candidate z cells, a z origin per word
     bool never;          // uniform: every word on the VALU
-    bool far;            // uniform: kFarCells candidate z cells or more (see push_quant)
     uint32_t ox, oz;     // origin: packed x | y << 16 (16-bit wrap-around), z
     sphk_short2 axy;     // this lane's target: x, y from the origin, its coordinates, and
     uint2 qi;            //   x^2 + y^2 + qneg
@@ -480,7 +480,6 @@ __device__ __forceinline__ void mfma_filter_begin(MfmaFilter& mf, const Chunk& c
                                                   bool active, uint32_t lane, int32_t qneg) {
     const int zspan = ch.zhi - ch.zlo;
     mf.wide = zspan > 4;
-    mf.far = zspan >= kFarCells;
     mf.never = zspan >= (1 << 21) || qneg < -kWideApart * kWideApart;
     // (the first target is lane 0's)
     mf.ox = uni(qi.x);
@@ -539,6 +538,7 @@ __device__ __forceinline__ uint32_t rows_filter_word(const MfmaFilter& mf, uint2
 
 // Verdict word of this lane's target over the word's `cnt` candidates, candidate k at bit
 // 31 - k (no bit for lanes without a target).  qb: this lane's row of the word; wide: mf.wide.
+template <bool kFar>
 __device__ __forceinline__ uint32_t filter_word(MfmaFilter& mf, uint2 qb, uint32_t cnt,
                                                 int32_t qneg, uint32_t lane, bool wide) {
     int32_t bz;
@@ -548,8 +548,7 @@ __device__ __forceinline__ uint32_t filter_word(MfmaFilter& mf, uint2 qb, uint32
         mf.oz = z0 + (uint32_t)((int32_t)(z1 - z0) >> 1);
         bz = (int32_t)(qb.y - mf.oz);
         if (mf.never || __ballot(bz < -kWideReach || bz > kWideReach) != 0ull)
-            return mf.far ? rows_filter_word<true>(mf, qb, cnt, qneg)
-                          : rows_filter_word<false>(mf, qb, cnt, qneg);
+            return rows_filter_word<kFar>(mf, qb, cnt, qneg);
         mfma_filter_targets(mf, lane);
     } else {
         bz = (int16_t)(qb.y - mf.oz);
@@ -596,7 +595,7 @@ __device__ __forceinline__ void put_word(uint32_t word, int w, uint32_t* __restr
     sl.count += (uint32_t)__builtin_popcount(word);
 }
 
-template <int kSeg, bool kMfma = false, bool kFar = false>
+template <int kSeg, bool kMfma, bool kFar>
 __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
                                               const uint2* __restrict__ sq,
                                               const uint32_t* __restrict__ cs,
@@ -621,7 +620,7 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
         uint32_t word;
         if (kMfma) {
             const uint2 qb = mfma_filter_row(*mf, sq, j0, cnt);
-            word = filter_word(*mf, qb, cnt, c.qneg, lane, mf->wide);
+            word = filter_word<kFar>(*mf, qb, cnt, c.qneg, lane, mf->wide);
         } else {
             word = valu_filter_word<kFar>(sq, j0, cnt, qi, active, c.qneg);
         }
@@ -633,22 +632,6 @@ __device__ __forceinline__ int phase1_segment(Cursor& cu, const Chunk& ch,
     return w;
 }
 
-// The force walk's re-test.  A loop of its own for tall chunks: the flag in the words' loop cost it
-// the scalar registers that hold its pointers (300,000 particles at 400 a cell, 2.80 -> 2.95 ms).
-template <int kSeg>
-__device__ __forceinline__ int retest_segment(Cursor& cu, const Chunk& ch,
-                                              const uint2* __restrict__ sq,
-                                              const uint32_t* __restrict__ cs,
-                                              const StepConsts& c, uint2 qi, bool active,
-                                              uint32_t* __restrict__ lmask,
-                                              uint32_t* __restrict__ lwj0, uint32_t lane,
-                                              SegLane& sl, int& part) {
-    return ch.zhi - ch.zlo >= kFarCells
-               ? phase1_segment<kSeg, false, true>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
-                                                   sl, part)
-               : phase1_segment<kSeg>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane, sl, part);
-}
-
 // The words of table entries first, first + kStride, ... below `end`, in turn to
 // put(word, entry, first slot).  The candidate rows of kAheadWords words are in flight.
 // kApart: wide chunks take a rolled loop of their own, so the unrolled one holds no test of
@@ -656,7 +639,7 @@ __device__ __forceinline__ int retest_segment(Cursor& cu, const Chunk& ch,
 // second copy of the product costs registers, which the walks of one wavefront per chunk don't
 // have (16 instead of 2 spilled, a step of 184,000 particles 285 -> 299 us).
 constexpr int kAheadWords = 4;
-template <int kStride, bool kApart, class Put>
+template <int kStride, bool kApart, bool kFar, class Put>
 __device__ __forceinline__ void table_words(const WordTable& t, MfmaFilter& mf,
                                             const uint2* __restrict__ sq, int first, int end,
                                             int32_t qneg, uint32_t lane, Put&& put) {
@@ -674,7 +657,7 @@ __device__ __forceinline__ void table_words(const WordTable& t, MfmaFilter& mf,
         for (int e = first; e < end; e += kStride) {
             uint32_t j0, cnt;
             word_table_entry(t, e, j0, cnt);
-            const uint32_t word = filter_word(mf, q[0], cnt, qneg, lane, true);
+            const uint32_t word = filter_word<kFar>(mf, q[0], cnt, qneg, lane, true);
 #pragma unroll
             for (int k = 0; k + 1 < kAheadWords; ++k) q[k] = q[k + 1];
             request(e + kAheadWords * kStride, q[kAheadWords - 1]);
@@ -689,7 +672,8 @@ __device__ __forceinline__ void table_words(const WordTable& t, MfmaFilter& mf,
             if (e < end) {
                 uint32_t j0, cnt;
                 word_table_entry(t, e, j0, cnt);
-                const uint32_t word = filter_word(mf, q[k], cnt, qneg, lane, !kApart && mf.wide);
+                const uint32_t word =
+                    filter_word<kFar>(mf, q[k], cnt, qneg, lane, !kApart && mf.wide);
                 request(e + kAheadWords * kStride, q[k]);
                 put(word, e, j0);
             }
@@ -702,7 +686,7 @@ __device__ __forceinline__ void table_words(const WordTable& t, MfmaFilter& mf,
 // to LDS and, from the registers that formed them, to the chunk's stored words (gm: its word
 // 0, `max_words` of them; nontemporal: the force walk reads them once, long after, and the rows
 // the walks gather should keep L2).
-template <int kSeg>
+template <int kSeg, bool kFar>
 __device__ __forceinline__ int phase1_table(const WordTable& t, int& i,
                                             const uint2* __restrict__ sq, const StepConsts& c,
                                             uint32_t* __restrict__ lmask,
@@ -720,15 +704,15 @@ __device__ __forceinline__ int phase1_table(const WordTable& t, int& i,
     if (nw <= 0) return 0;
     const int stored = (int)c.max_words - g0;  // words of the segment the engine stores
     uint32_t jv = 0;                           // lane w: first slot of word w
-    table_words<1, false>(t, mf, sq, i, i + nw, c.qneg, lane,
-                          [&](uint32_t word, int e, uint32_t j0) {
-                              const int w = e - i;
-                              jv = lane == (uint32_t)w ? j0 : jv;
-                              put_word(word, w, lmask, lane, sl);
-                              if (w < stored)
-                                  __builtin_nontemporal_store(
-                                      word, &gm[(size_t)(g0 + w) * 64 + lane]);
-                          });
+    table_words<1, false, kFar>(t, mf, sq, i, i + nw, c.qneg, lane,
+                                [&](uint32_t word, int e, uint32_t j0) {
+                                    const int w = e - i;
+                                    jv = lane == (uint32_t)w ? j0 : jv;
+                                    put_word(word, w, lmask, lane, sl);
+                                    if (w < stored)
+                                        __builtin_nontemporal_store(
+                                            word, &gm[(size_t)(g0 + w) * 64 + lane]);
+                                });
     if ((int)lane < nw) {
         lwj0[lane] = jv;
         if ((int)lane < stored) gj[g0 + (int)lane] = jv;

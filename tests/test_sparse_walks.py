@@ -136,3 +136,33 @@ def test_far_particles_reach_no_one(sphk, shape):
     for a, b in zip(*out):
         assert np.isfinite(a[rest]).all()
         np.testing.assert_array_equal(a[rest], b[rest])
+
+
+@pytest.mark.parametrize("radius_cut", [False, True])
+@pytest.mark.parametrize("shape", ["seg32_waves4_split", "seg24_waves4", "pp16_waves4"])
+def test_tall_grids_step_like_low_ones(sphk, shape, radius_cut):
+    # Grids of more than 180 z cells take walk kernels of their own.  The same particles, a pile
+    # with more words than are stored (tested again by the force walk) among them, in low and in
+    # tall bounds: from the second step on, when the grid covers the bounds, one engine takes the
+    # one, the other the other, and every bit agrees.
+    rng = np.random.default_rng(9)
+    pos = np.concatenate([rng.uniform(0.1, 0.5, (3000, 3)),
+                          rng.uniform([0.22, 0.22, 0.22], [0.26, 0.26, 0.30], (9000, 3))]).astype(F32)
+    vel = rng.normal(0, 0.1, pos.shape).astype(F32)
+    k = sphk.walk_shape_names().index(shape)
+    out = []
+    for top in (0.6, 12.0):
+        p = sphk.default_params(xmin=0, xmax=0.6, ymin=0, ymax=0.6, zmin=0, zmax=top, formulation=1,
+                                particle_mass=1e-5, smoothing_length=0.025 if radius_cut else 0.02)
+        e = sphk.Engine(len(pos), p)
+        e.upload(pos, vel)
+        e.set_walk_shapes(k, k)
+        for graph in (False, False, True, True):
+            e.set_graph(graph)
+            e.step(1e-6)
+        assert (int(e.grid()[1][2]) > 180) == (top > 1)
+        assert e.walk_words()[1].max() > 256
+        out.append((e.positions(), e.velocities(), e.densities()[:len(pos)], e.accelerations()))
+    for a, b in zip(*out):
+        assert np.isfinite(a).all()
+        np.testing.assert_array_equal(a, b)
