@@ -773,7 +773,7 @@ __global__ __launch_bounds__(256) void k_sur_wgrad(SurGradRows g, const __bf16* 
 // in dW1; operands with the halves of K the same way round in both blocks (no time) give the sums
 // that lie within a rounding of zero another sign, some of 2e9 a call: one such mask moved a
 // small scene's gradient by 5e-6 of its norm.
-// 1,024 chunks: 600 -> 231 us.
+// 1,024 chunks: 600 -> 241 us.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kEdgeRow = 72;  // LDS row stride (bf16) of one feature over 64 edges
 
