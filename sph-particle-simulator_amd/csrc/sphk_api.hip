@@ -513,7 +513,8 @@ int ensure_grid(sphk_engine* e) {
     if (int rc = grow(&wb.colcnt, ccap, ncols + 1, e->buffer_gen)) return rc;
     wb.col_cap = ccap;
     if (!wb.nitems) {
-        HIP_TRY(dalloc(&wb.nitems, 1));
+        HIP_TRY(dalloc(&wb.nitems, 3));
+        HIP_TRY(hipMemsetAsync(wb.nitems, 0, 3 * sizeof(uint32_t), e->stream));
         ++e->buffer_gen;
     }
     const size_t hist_words = ((size_t)1 << kRadixMaxBits) * ((e->cap + kRadixTile - 1) / kRadixTile);

@@ -124,7 +124,9 @@ struct WalkBuffers {
                                   // the walks start from it instead of looking the scene and the
                                   // column of the first particle up (a chain of dependent loads
                                   // and four divisions per wavefront)
-    uint32_t* nitems = nullptr;   // [1] number of chunks
+    uint32_t* nitems = nullptr;   // [3] number of chunks; of these, counted by the team density
+                                  // walk, those held by one column (lone_chunk); whether the team
+                                  // walks give every wavefront a chunk
     uint32_t* colcnt = nullptr;   // [ncols + 1] per-column chunk counts -> offsets
     uint32_t* mask = nullptr;     // [chunks][max_words][64] neighbour bits
     uint32_t* wj0 = nullptr;      // [chunks][max_words] first slot of each word

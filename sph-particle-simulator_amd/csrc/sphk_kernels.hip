@@ -666,7 +666,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_sort(
     }
     uint32_t total;
     run = small_scan<false>(chunks, lw, &total);
-    if (tid == 0) nitems[0] = total;
+    if (tid < 3u) nitems[tid] = tid == 0u ? total : 0u;
 #pragma unroll 1
     for (uint32_t col = col0; col < col1; ++col) {
         const uint2 r = column(col, scene, g);

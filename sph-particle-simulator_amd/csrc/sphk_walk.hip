@@ -51,6 +51,16 @@ __global__ __launch_bounds__(256) void k_chunk_count(const uint32_t* __restrict_
     cnt[col] = (b - a + 63u) / 64u;
 }
 
+constexpr uint32_t kLoneChunks = 1100;  // see lone_chunk
+
+// The number of chunks and, from the density walk before this list (lone_chunk), whether the
+// team walks of this step give every wavefront a chunk of its own.
+__device__ __forceinline__ void publish_chunks(uint32_t* __restrict__ nitems, uint32_t total) {
+    nitems[2] = 2u * nitems[1] > nitems[0] && total >= kLoneChunks ? 1u : 0u;
+    nitems[1] = 0u;
+    nitems[0] = total;
+}
+
 __global__ __launch_bounds__(256) void k_chunk_fill(const uint32_t* __restrict__ cs, StepConsts c,
                                                     const SceneGrid* __restrict__ scenes,
                                                     const uint32_t* __restrict__ offs,
@@ -58,7 +68,7 @@ __global__ __launch_bounds__(256) void k_chunk_fill(const uint32_t* __restrict__
                                                     uint4* __restrict__ desc,
                                                     uint32_t* __restrict__ nitems) {
     const uint32_t col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col == 0) nitems[0] = offs[c.ncols];
+    if (col == 0) publish_chunks(nitems, offs[c.ncols]);
     if (col >= c.ncols) return;
     const uint32_t scene = scene_of_col(scenes, c.nscenes, col);
     const SceneGrid g = scenes[scene];
@@ -191,6 +201,51 @@ __device__ __forceinline__ float density_run(BitWalk<kW>& bw, float4& q0, float4
     return acc;
 }
 
+// The sum over a chunk's words by one wavefront, a segment of kSeg - 1 of them at a time; the
+// parts' sums are folded as (p0 + p1) + p2.
+template <class Shape, bool kCut, bool kFar>
+__device__ __forceinline__ float density_segments(
+    const Chunk& ch, const WordTable& wt, bool tab, MfmaFilter& mf, const float4* __restrict__ spm,
+    const uint2* __restrict__ sq, const uint32_t* __restrict__ cs, const StepConsts& c, uint2 qi,
+    bool active, const float4& pi, uint32_t* __restrict__ gm, uint32_t* __restrict__ gj,
+    uint32_t* __restrict__ lmask, uint32_t* __restrict__ lwj0, uint32_t lane) {
+    constexpr int kSeg = Shape::seg;
+    Cursor cu;
+    if (!tab) cursor_begin(cu, ch, cs, c);
+    float total = 0.0f, cur = 0.0f;
+    int cur_part = 0;
+    int seg_base = wt.first;
+    int ti = 0;  // next table entry
+    for (;;) {
+        SegLane sl;
+        int seg_part;
+        const int nw =
+            tab ? phase1_table<kSeg, kFar>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl, seg_part,
+                                           mf)
+                : phase1_segment<kSeg, true, kFar>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
+                                                   sl, seg_part, &mf);
+        if (nw == 0) break;
+        for (; cur_part < seg_part; ++cur_part) {
+            total = cur_part == 0 ? cur : total + cur;
+            cur = 0.0f;
+        }
+        wave_sync();
+        if (!tab) store_words(c.max_words, seg_base, nw, lmask, lwj0, gm, gj, lane);
+        BitWalk<kSeg> bw;
+        bw.begin(sl.nonempty, lmask, lwj0, lane);
+        const uint32_t steps = wave_max(sl.count);
+        cur = density_bits<kCut>(bw, steps, lmask, lwj0, lane, spm, pi, c, cur);
+        seg_base += nw;
+        wave_sync();
+        if (tab ? ti >= wt.n : cu.done) break;
+    }
+    for (; cur_part < kParts; ++cur_part) {
+        total = cur_part == 0 ? cur : total + cur;
+        cur = 0.0f;
+    }
+    return total;
+}
+
 // Density pass over one chunk by one wavefront.  As many wavefronts per SIMD as the LDS
 // allows (six with 24-word segments): the walk is VALU-bound (a few spills outside the walk
 // loops).  The ping-pong shapes aim at what their LDS
@@ -232,14 +287,15 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
         gpart[item] = pack_parts(wt.ps1, wt.ps2);
         gnw[item] = (uint32_t)wt.total;
     }
-    Cursor cu;
-    if (!tab) cursor_begin(cu, ch, cs, c);
-    // per-part running sum `cur`, parts folded into `total` as (p0 + p1) + p2
-    float total = 0.0f, cur = 0.0f;
-    int cur_part = 0;
-    int seg_base = wt.first;
-    int ti = 0;  // next table entry
+    float total = 0.0f;
     if constexpr (Shape::pp) {
+        Cursor cu;
+        if (!tab) cursor_begin(cu, ch, cs, c);
+        // per-part running sum `cur`, parts folded into `total` as (p0 + p1) + p2
+        float cur = 0.0f;
+        int cur_part = 0;
+        int seg_base = wt.first;
+        int ti = 0;  // next table entry
         // Segments are made in the newer buffer.  A segment of the part being walked joins
         // the walk at once; one of the next part waits there until every lane is through the
         // current part (the parts' sums are folded between them, in the same order as in
@@ -314,34 +370,13 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
             pend = false;
             pp.add_held(pend_nw, lmask, lwj0, lane, c.pad_slot);
         }
-    } else {
-        for (;;) {
-            SegLane sl;
-            int seg_part;
-            const int nw =
-                tab ? phase1_table<kSeg, kFar>(wt, ti, sq, c, lmask, lwj0, gm, gj, lane, sl,
-                                               seg_part, mf)
-                    : phase1_segment<kSeg, true, kFar>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
-                                                       lane, sl, seg_part, &mf);
-            if (nw == 0) break;
-            for (; cur_part < seg_part; ++cur_part) {
-                total = cur_part == 0 ? cur : total + cur;
-                cur = 0.0f;
-            }
-            wave_sync();
-            if (!tab) store_words(c.max_words, seg_base, nw, lmask, lwj0, gm, gj, lane);
-            BitWalk<kSeg> bw;
-            bw.begin(sl.nonempty, lmask, lwj0, lane);
-            const uint32_t steps = wave_max(sl.count);
-            cur = density_bits<kCut>(bw, steps, lmask, lwj0, lane, spm, pi, c, cur);
-            seg_base += nw;
-            wave_sync();
-            if (tab ? ti >= wt.n : cu.done) break;
+        for (; cur_part < kParts; ++cur_part) {
+            total = cur_part == 0 ? cur : total + cur;
+            cur = 0.0f;
         }
-    }
-    for (; cur_part < kParts; ++cur_part) {
-        total = cur_part == 0 ? cur : total + cur;
-        cur = 0.0f;
+    } else {
+        total = density_segments<Shape, kCut, kFar>(ch, wt, tab, mf, spm, sq, cs, c, qi, active,
+                                                    pi, gm, gj, lmask, lwj0, lane);
     }
     if (active) density_epilogue(total, pi, s, c, svr, rows);
 }
@@ -362,6 +397,17 @@ __global__ __launch_bounds__(Shape::threads) __attribute__((amdgpu_waves_per_eu(
 // workgroups a CU).
 // ---------------------------------------------------------------------------
 constexpr int kTeam = 4;
+
+// In a pile-up (the reference formulas throw a block into its box's corners) a chunk has hundreds
+// of words and one column holds nearly all of them: a team then has work for one wavefront and
+// holds the LDS of four.  Where most chunks of the walk before were such, and enough to fill the
+// GPU, every wavefront of the teams walks a chunk of its own.  Corner pile-ups, a step: 80,000
+// particles 5.49 -> 5.38 ms, 100,000 7.37 -> 7.03, 120,000 9.69 -> 8.26, 160,000 16.06 -> 12.98;
+// 66,000 are level, and piles over several columns are faster by teams (100,000 particles at 1,500
+// a cell 4.7 ms against 6.9).
+__device__ __forceinline__ bool lone_chunk(const WordTable& wt) {
+    return wt.total > kMaxWords && 8 * max(wt.ps1, wt.ps2 - wt.ps1) > 7 * wt.total;
+}
 
 // LDS rows of the team's words: a part's words in groups of kSeg - 1, each group followed by
 // the sentinel word of its walk.
@@ -415,18 +461,20 @@ __global__ __launch_bounds__(64 * kTeam) void k_density_team(
     const uint2* __restrict__ sq, float4* __restrict__ svr, ForceRow* __restrict__ rows,
     const uint32_t* __restrict__ skey, const uint32_t* __restrict__ cs, StepConsts c,
     const SceneGrid* __restrict__ scenes, uint32_t* __restrict__ gmask,
-    uint32_t* __restrict__ gwj0, uint32_t* __restrict__ gnw, uint32_t* __restrict__ gpart) {
+    uint32_t* __restrict__ gwj0, uint32_t* __restrict__ gnw, uint32_t* __restrict__ gpart,
+    uint32_t* __restrict__ lone_chunks) {
     constexpr int kSeg = Shape::seg;
     constexpr int kGroup = kSeg - 1;
     constexpr int kRows = kTableWords + kTableWords / kGroup + kParts;
-    static_assert(kTeam >= kParts && kRows >= kParts * kSeg, "one walker and its words per part");
+    static_assert(kTeam >= kParts && kRows >= kTeam * kSeg, "a walk's words per wavefront");
     __shared__ uint32_t lmask[kRows * 64];
     __shared__ uint32_t lwj0[kRows];
     __shared__ uint32_t scratch[kTeam][kTableWords];
     __shared__ float lsum[kParts][64];
     const uint32_t wave = uni(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t item = xcd_unit(uni(nitems[0]), 1u, 0u);
+    const bool lone = uni(nitems[2]) != 0u;
+    const uint32_t item = xcd_unit(uni(nitems[0]), lone ? kTeam : 1u, lone ? wave : 0u);
     if (item == ~0u) return;
     Chunk ch;
     uint32_t s;
@@ -440,9 +488,19 @@ __global__ __launch_bounds__(64 * kTeam) void k_density_team(
     const bool tab = word_table_build(wt, ch, cs, -1, lane, scratch[wave]);
     uint32_t* const gm = gmask + (size_t)item * c.max_words * 64;
     uint32_t* const gj = gwj0 + (size_t)item * c.max_words;
-    if (wave == 0 && lane == 0) {
+    if ((lone || wave == 0) && lane == 0) {
         gpart[item] = pack_parts(wt.ps1, wt.ps2);
         gnw[item] = (uint32_t)wt.total;
+        if (lone_chunk(wt)) atomicAdd(lone_chunks, 1u);
+    }
+    if (lone) {
+        uint32_t* const lm = lmask + wave * kSeg * 64;
+        uint32_t* const lj = lwj0 + wave * kSeg;
+        init_sentinel<kSeg>(lm, lj, lane, c);
+        const float total = density_segments<Shape, kCut, kFar>(
+            ch, wt, tab, mf, spm, sq, cs, c, qi, active, pi, gm, gj, lm, lj, lane);
+        if (active) density_epilogue(total, pi, s, c, svr, rows);
+        return;
     }
     float cur = 0.0f;
     if (tab) {
@@ -644,6 +702,24 @@ __device__ __forceinline__ void fold_parts_reg(float (&t)[6], ForceSums& f, int 
     f = ForceSums();
 }
 
+// The running total as it is kept in LDS or in registers.
+__device__ __forceinline__ void clear_parts(float* __restrict__ t, uint32_t lane) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) t[k * 64 + lane] = 0.0f;
+}
+__device__ __forceinline__ ForceSums total_sums(const float* __restrict__ t, uint32_t lane) {
+    ForceSums f;
+    f.fp = make_float3(t[0 * 64 + lane], t[1 * 64 + lane], t[2 * 64 + lane]);
+    f.fv = make_float3(t[3 * 64 + lane], t[4 * 64 + lane], t[5 * 64 + lane]);
+    return f;
+}
+__device__ __forceinline__ ForceSums total_sums(const float (&t)[6]) {
+    ForceSums f;
+    f.fp = make_float3(t[0], t[1], t[2]);
+    f.fv = make_float3(t[3], t[4], t[5]);
+    return f;
+}
+
 // Loads a segment of `nw` stored words (from stored word `base` on) into LDS, with the lane's
 // summary.  All loads are issued before the first is used (a loop over nw would wait for each
 // load of its remainder in turn); slots past nw re-read word nw - 1 and are dropped.  The words
@@ -669,6 +745,60 @@ __device__ __forceinline__ void load_words(const uint32_t* __restrict__ gmask,
         }
     }
     if ((int)lane < nw) lwj0[lane] = gwj0[base + lane];
+}
+
+// The sums over a chunk's words by one wavefront, a segment at a time: stored words, or the words
+// formed again.  The parts' running total is in registers (kRegTot) or in `ltot`, six rows of 64
+// lanes in LDS.
+template <class Shape, bool kCut, bool kFar, bool kRegTot>
+__device__ __forceinline__ ForceSums force_segments(
+    const Chunk& ch, bool stored, int total_words, uint32_t pstarts, size_t first_word,
+    const uint2* __restrict__ sq, const ForceRow* __restrict__ rows,
+    const uint32_t* __restrict__ cs, const StepConsts& c, uint2 qi, bool active, const float4& pi,
+    const float3& vi, float p_quarter, const uint32_t* __restrict__ gmask,
+    const uint32_t* __restrict__ gwj0, uint32_t* __restrict__ lmask, uint32_t* __restrict__ lwj0,
+    float* __restrict__ ltot, uint32_t lane, uint32_t& cnt) {
+    constexpr int kSeg = Shape::seg;
+    float rtot[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (!kRegTot) clear_parts(ltot, lane);
+    ForceSums f;
+    int cur_part = 0;
+    Cursor cu;
+    if (!stored) cursor_begin(cu, ch, cs, c);
+    int seg_base = 0;
+    for (;;) {
+        int nw, seg_part;
+        SegLane sl;
+        if (stored) {
+            if (seg_base >= total_words) break;
+            seg_part = part_of_word(seg_base, pstarts);
+            const int pend = part_word_end(pstarts, seg_part, total_words);
+            nw = min(kSeg - 1, pend - seg_base);
+            load_words<kSeg>(gmask, gwj0, first_word + seg_base, nw, lmask, lwj0, lane, sl);
+        } else {
+            nw = phase1_segment<kSeg, false, kFar>(cu, ch, sq, cs, c, qi, active, lmask, lwj0, lane,
+                                                   sl, seg_part);
+            if (nw == 0) break;
+        }
+        if (kRegTot)
+            fold_parts_reg(rtot, f, seg_part - cur_part);
+        else
+            fold_parts(ltot, lane, f, seg_part - cur_part);
+        cur_part = seg_part;
+        wave_sync();
+        BitWalk<kSeg> bw;
+        bw.begin(sl.nonempty, lmask, lwj0, lane);
+        force_bits<kSeg, kCut>(bw, wave_max(sl.count), lmask, lwj0, lane, rows, pi, vi, p_quarter,
+                               c, f, cnt);
+        seg_base += nw;
+        wave_sync();
+        if (!stored && cu.done) break;
+    }
+    if (kRegTot)
+        fold_parts_reg(rtot, f, kParts - cur_part);
+    else
+        fold_parts(ltot, lane, f, kParts - cur_part);
+    return kRegTot ? total_sums(rtot) : total_sums(ltot, lane);
 }
 
 // Force pass over one chunk by one wavefront.  Shapes of 24 words and more keep
@@ -698,7 +828,6 @@ void k_force_walk(
     constexpr bool kRegTot = !Shape::pp && kSeg >= 24;
     constexpr bool kLdsTot = !kRegTot;
     __shared__ float ltot_all[kLdsTot ? Shape::waves : 1][kLdsTot ? 6 * 64 : 1];
-    float rtot[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     uint32_t* lmask = lmask_all[wave];
     uint32_t* lwj0 = lwj0_all[wave];
     float* ltot = ltot_all[kLdsTot ? wave : 0];
@@ -721,23 +850,21 @@ void k_force_walk(
         if (active) qi = sq[s];
     }
     init_sentinel<kLds>(lmask, lwj0, lane, c);
-    if (kLdsTot) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k) ltot[k * 64 + lane] = 0.0f;
-    }
     const float4 vr = active ? svr[s] : make_float4(0.f, 0.f, 0.f, 1.f);
     const float3 vi = make_float3(vr.x, vr.y, vr.z);
     const float rho_i = vr.w;
     const float P_i = c.k_gas * (rho_i - c.rho0);
     const float p_quarter = 0.25f * P_i;
-    ForceSums f;
-    uint32_t cnt = 0;  // neighbours of this wavefront's part(s)
-    int cur_part = 0;
-    Cursor cu;
-    if (!stored) cursor_begin(cu, ch, cs, c);
-    int seg_base = 0;
-    const int words_end = total_words;
+    ForceSums tot;
+    uint32_t cnt = 0;  // neighbours
     if constexpr (Shape::pp) {
+        clear_parts(ltot, lane);
+        ForceSums f;
+        int cur_part = 0;
+        Cursor cu;
+        if (!stored) cursor_begin(cu, ch, cs, c);
+        int seg_base = 0;
+        const int words_end = total_words;
         // As in the density walk: segments are loaded into the newer buffer; one of the part
         // being walked joins the walk at once, one of the next part waits until every lane
         // is through the current part.
@@ -819,51 +946,15 @@ void k_force_walk(
             pend = false;
             pp.add_held(pend_nw, lmask, lwj0, lane, c.pad_slot);
         }
+        fold_parts(ltot, lane, f, kParts - cur_part);
+        tot = total_sums(ltot, lane);
     } else {
-        for (;;) {
-            int nw, seg_part;
-            SegLane sl;
-            if (stored) {
-                if (seg_base >= words_end) break;
-                seg_part = part_of_word(seg_base, pstarts);
-                const int pend = part_word_end(pstarts, seg_part, total_words);
-                nw = min(kSeg - 1, pend - seg_base);
-                load_words<kSeg>(gmask, gwj0, (size_t)item * c.max_words + seg_base, nw, lmask,
-                                 lwj0, lane, sl);
-            } else {
-                nw = phase1_segment<kSeg, false, kFar>(cu, ch, sq, cs, c, qi, active, lmask, lwj0,
-                                                       lane, sl, seg_part);
-                if (nw == 0) break;
-            }
-            if (kRegTot)
-                fold_parts_reg(rtot, f, seg_part - cur_part);
-            else
-                fold_parts(ltot, lane, f, seg_part - cur_part);
-            cur_part = seg_part;
-            wave_sync();
-            BitWalk<kSeg> bw;
-            bw.begin(sl.nonempty, lmask, lwj0, lane);
-            force_bits<kSeg, kCut>(bw, wave_max(sl.count), lmask, lwj0, lane, rows, pi, vi,
-                                   p_quarter, c, f, cnt);
-            seg_base += nw;
-            wave_sync();
-            if (!stored && cu.done) break;
-        }
+        tot = force_segments<Shape, kCut, kFar, kRegTot>(
+            ch, stored, total_words, pstarts, (size_t)item * c.max_words, sq, rows, cs, c, qi,
+            active, pi, vi, p_quarter, gmask, gwj0, lmask, lwj0, ltot, lane, cnt);
     }
     if (stats) add_nbr_stats(cnt, stats, lane);
-    if (kRegTot)
-        fold_parts_reg(rtot, f, kParts - cur_part);
-    else
-        fold_parts(ltot, lane, f, kParts - cur_part);
     if (!active) return;
-    ForceSums tot;
-    if (kRegTot) {
-        tot.fp = make_float3(rtot[0], rtot[1], rtot[2]);
-        tot.fv = make_float3(rtot[3], rtot[4], rtot[5]);
-    } else {
-        tot.fp = make_float3(ltot[0 * 64 + lane], ltot[1 * 64 + lane], ltot[2 * 64 + lane]);
-        tot.fv = make_float3(ltot[3 * 64 + lane], ltot[4 * 64 + lane], ltot[5 * 64 + lane]);
-    }
     force_epilogue(tot, pi, vi, rho_i, P_i, s, scenes[ch.scene], c, sid, dt_dev, dt_arg, pm, vel,
                    acc_out, rho_out, prs_out);
 }
@@ -897,7 +988,8 @@ __global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t* lmask = lmask_all[wave];
     uint32_t* lwj0 = lwj0_all[wave];
-    const uint32_t item = xcd_unit(uni(nitems[0]), 1u, 0u);
+    const bool lone = uni(nitems[2]) != 0u;
+    const uint32_t item = xcd_unit(uni(nitems[0]), lone ? kForceTeam : 1u, lone ? wave : 0u);
     if (item == ~0u) return;
     Chunk ch;
     uint32_t s;
@@ -922,6 +1014,16 @@ __global__ __launch_bounds__(64 * kForceTeam) void k_force_team(
     const float P_i = c.k_gas * (rho_i - c.rho0);
     const float p_quarter = 0.25f * P_i;
     uint32_t cnt = 0;
+    if (lone) {
+        const ForceSums tot = force_segments<Shape, kCut, kFar, true>(
+            ch, stored, total_words, pstarts, (size_t)item * c.max_words, sq, rows, cs, c, qi,
+            active, pi, vi, p_quarter, gmask, gwj0, lmask, lwj0, nullptr, lane, cnt);
+        if (stats) add_nbr_stats(cnt, stats, lane);
+        if (active)
+            force_epilogue(tot, pi, vi, rho_i, P_i, s, scenes[ch.scene], c, sid, dt_dev, dt_arg, pm,
+                           vel, acc_out, rho_out, prs_out);
+        return;
+    }
     for (int part = (int)wave; part < (wave == 0 ? 1 : kParts); ++part) {
         ForceSums f;
         Cursor cu;
@@ -1087,7 +1189,7 @@ __global__ __launch_bounds__(256) void k_chunk_list(const uint32_t* __restrict__
         run += cnt[j];
     }
     __syncthreads();
-    if (blockIdx.x == 0 && threadIdx.x == 0) nitems[0] = total;
+    if (blockIdx.x == 0 && threadIdx.x == 0) publish_chunks(nitems, total);
     const uint32_t col = blockIdx.x * 256u + threadIdx.x;
     if (col >= ncols) return;
     const uint32_t scene = one ? 0u : scene_of_col(scenes, c.nscenes, col);
@@ -1282,14 +1384,14 @@ hipError_t launch_density_walk(const WalkBuffers& wb, const float4* spm, const u
                                hipStream_t st) {
     if (n == 0) return hipSuccess;
     const uint32_t chunks = max_chunks(n, c);
-#define SPHK_DENSITY_KERNEL(KERNEL, CUT, FAR, PER_BLOCK, THREADS)                              \
+#define SPHK_DENSITY_KERNEL(KERNEL, CUT, FAR, PER_BLOCK, THREADS, ...)                         \
     hipLaunchKernelGGL((KERNEL<S, CUT, FAR>), dim3(grid_for(chunks, PER_BLOCK)), dim3(THREADS), \
                        0, st, wb.items, wb.desc, wb.nitems, spm, sq, svr, rows, skey, cell_start, \
-                       c, scenes, wb.mask, wb.wj0, wb.nwords, wb.pstarts)
+                       c, scenes, wb.mask, wb.wj0, wb.nwords, wb.pstarts, ##__VA_ARGS__)
 #define SPHK_DENSITY_LAUNCH(CUT, FAR)                                                         \
     SPHK_DISPATCH_SHAPE(                                                                      \
         shape, SPHK_DENSITY_KERNEL(k_density_walk, CUT, FAR, S::waves, S::threads),           \
-        SPHK_DENSITY_KERNEL(k_density_team, CUT, FAR, 1, 64 * kTeam))
+        SPHK_DENSITY_KERNEL(k_density_team, CUT, FAR, 1, 64 * kTeam, wb.nitems + 1))
     if (c.cut) {
         if (c.far) {
             SPHK_DENSITY_LAUNCH(true, true);

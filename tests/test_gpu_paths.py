@@ -241,3 +241,42 @@ def test_refused_uploads_on_both_routes(sphk, rows):
     np.testing.assert_array_equal(e.positions(), np.concatenate([pos, more[:-7]]))
     e.step(1e-5)
     e.positions()  # (would report a particle outside its grid)
+
+
+@pytest.mark.parametrize("cut,graph", [(False, False), (False, True), (True, False)])
+def test_corner_pile_ups_step_alike_in_every_shape(sphk, cut, graph):
+    # The reference formulas pile a block up in its box's corners within a few steps: most chunks
+    # then have more words than are stored, nearly all of one column, and in the team shapes every
+    # wavefront goes over to a chunk of its own (1,100 chunks and more), and back to teams when
+    # the block is uploaded again.  Bits and neighbour statistics are those of the other shapes.
+    names = sphk.walk_shape_names()
+    n = 80000
+    s = n ** (1 / 3) * 0.01
+    pos = np.random.default_rng(1).uniform(0, s, (n, 3)).astype(np.float32)
+    p = sphk.default_params(xmin=0, xmax=2.5 * s, ymin=0, ymax=1.5 * s, zmin=0, zmax=1.2 * s,
+                            smoothing_length=0.025 if cut else 0.02)
+    out = []
+    for d, f in ((None, None), ("seg16_waves4_split",) * 2, ("seg24_waves4", "pp16_waves4")):
+        e = sphk.Engine(n, p)
+        e.upload(pos)
+        e.set_graph(graph)
+        if d:
+            e.set_walk_shapes(names.index(d), names.index(f))
+        got = []
+        for steps in (5, 1, 1):
+            for _ in range(steps):
+                e.step(1e-3)
+            st = e.stats()
+            got += [e.positions(), e.velocities(), e.densities()[:n], e.accelerations(),
+                    np.array([st.max_neighbors, st.total_neighbors])]
+        if d is None:
+            items, nwords, _, _ = e.walk_words()
+            assert len(items) >= 1100 and np.mean(nwords > 256) > 0.5
+        for _ in range(2):
+            e.upload(pos)
+            e.step(1e-3)
+            got += [e.positions(), e.velocities()]
+        out.append(got)
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            np.testing.assert_array_equal(a, b)
